@@ -480,16 +480,24 @@ __device__ __forceinline__ void begin_step_in(const DevScene& S, int region, Ele
 
 /* The lanes of a wave take their turn by region (one pass per region present,
  * normally one): within a pass the region index is wave-uniform, so the
- * scene records it selects are read with scalar loads. */
+ * scene records it selects are read with scalar loads.  The loop runs over a
+ * wave-uniform mask of the lanes still to do: a loop left lane by lane would
+ * let the compiler run the body after it, where the region is a per-lane
+ * value again and every scene read a vector load. */
+template <class F>
+__device__ __forceinline__ void by_region(const Elec& e, F body) {
+  unsigned long long todo = wave_ballot(true);
+  while (todo) {
+    const int r0 = __builtin_amdgcn_readlane(e.region, __ffsll((long long)todo) - 1);
+    const unsigned long long turn = wave_ballot(e.region == r0) & todo;
+    if (lane_in(turn)) body(r0);
+    todo &= ~turn;
+  }
+}
+
 __device__ __forceinline__ void begin_step(const DevScene& S, Elec& e, StepStart& st) {
   PT_UNIFORM(PH_RATES_UNI, e.region);
-  for (;;) {
-    const int r0 = __builtin_amdgcn_readfirstlane(e.region);
-    if (lane_in(wave_ballot(e.region == r0))) {
-      begin_step_in(S, r0, e, st);
-      break;
-    }
-  }
+  by_region(e, [&](int r0) { begin_step_in(S, r0, e, st); });
 }
 
 /* The check that opens MonteCarloSS::takeStep (MonteCarloSS.cu:107-115):
@@ -657,14 +665,8 @@ template <bool TAB>
 __device__ __forceinline__ int finish_step(const DevScene& S, const JobRec* jobs, Elec& e, Spawn& sp, int maxSteps,
                                            const StepStart& st) {
   PT_UNIFORM(PH_GEOM_UNI, e.region);
-  int res;
-  for (;;) {
-    const int r0 = __builtin_amdgcn_readfirstlane(e.region);
-    if (lane_in(wave_ballot(e.region == r0))) {
-      res = finish_step_in<TAB>(S, jobs, r0, e, sp, maxSteps, st);
-      break;
-    }
-  }
+  int res = STEP_CONTINUE;
+  by_region(e, [&](int r0) { res = finish_step_in<TAB>(S, jobs, r0, e, sp, maxSteps, st); });
   return res;
 }
 
