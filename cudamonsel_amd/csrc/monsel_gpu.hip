@@ -166,11 +166,16 @@ struct GenDev {
   int geo_batch;             /* lanes of a wave that wait for findEndOfStep before the wave runs it */
   int handoff;               /* new secondaries go to idle lanes of their wave first */
   int tail_lanes;            /* tail compaction threshold (0 = off) */
+  int lane_cap;              /* items a wave works on at once at most (64 = every lane) */
+  int claim_min;             /* items a wave that still steps takes at a time at least */
+  int claim_chunk;           /* items a wave claims at a time at least */
 };
 
 /* launches with fewer items than this run their tail out (compaction would
  * only pass a few electrons from launch to launch) */
 constexpr uint32_t kTailMinItems = 65536;
+/* launches with fewer items than this spread them over all waves (spread_launch) */
+constexpr uint32_t kSpreadItems = 65536;
 /* items a wave claims at a time (kept in reserve for its idle lanes);
  * 4 to 24 measure alike on the line scan, 128 and more starve other waves;
  * with the claim threshold below, 32 and 64 are 4 % and 8 % slower */
@@ -753,7 +758,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MONSEL
 k_transport(DevScene S, GenDev G) {
   Elec e;
   StepStart st;
-  bool alive = false, done = false, pending = false;
+  bool alive = false, pending = false;
+  bool done = false;                   /* wave-uniform: the launch's items are all claimed */
   uint32_t r_base = 0, r_left = 0;     /* wave-uniform reserve of claimed item indices */
   int maxSteps = 0;
   uint32_t steps0 = 0;                 /* step count when the lane took the electron */
@@ -768,14 +774,17 @@ k_transport(DevScene S, GenDev G) {
     /* claim work for idle lanes (once kClaimMin of them wait, or no lane
      * steps): from the wave's reserve of claimed items, topped up a chunk
      * at a time by one atomic per wave */
-    bool need = !alive && !done;
-    unsigned long long m = wave_ballot(need);
-    if (m && __popcll(m) < kClaimMin && wave_ballot(alive) != 0ull) m = 0ull;
+    unsigned long long m = done ? 0ull : wave_ballot(!alive);
+    const int room = __popcll(m) - (64 - G.lane_cap);   /* lane_cap less the live lanes */
+    if (~m != 0ull && room < G.claim_min) m = 0ull;
     if (m) {
+      /* the first `room` idle lanes take an item each */
+      const bool need = !alive && __popcll(m & lanemask_lt) < room;
+      m = wave_ballot(need);
       const uint32_t cnt = (uint32_t)__popcll(m);
       uint32_t fresh = 0, want = 0;
       if (cnt > r_left) {
-        want = max(cnt - r_left, (uint32_t)kClaimChunk);
+        want = max(cnt - r_left, (uint32_t)G.claim_chunk);
         const int leader = __ffsll((long long)m) - 1;
         if (lane_id() == leader) fresh = atomicAdd(G.claim, want);
         fresh = __shfl(fresh, leader);
@@ -834,18 +843,20 @@ k_transport(DevScene S, GenDev G) {
             /* a queued electron is located again (the check opening its next step) */
             alive = idx < G.n_prim ? e.region >= 0 : locate(S, G.jobs, e, e.region);
           }
-        } else {
-          done = true;
         }
       }
+      /* items are handed out in order: one beyond the last means none are left */
+      done = wave_ballot(need && idx >= n_items) != 0ull;
     }
-    /* the wave leaves only once every lane has run past the launch's items: a
-     * claim round can hand out nothing but dead electrons (queued ones of a
-     * job the host stopped, or primaries that start outside the chamber),
-     * and the items after them must still be claimed */
-    if (wave_ballot(alive || !done) == 0ull) break;
     PT_END(PH_CLAIM, t_cl);
-    if (wave_ballot(alive) == 0ull) continue;
+    if (wave_ballot(alive) == 0ull) {
+      /* the wave leaves only once it has run past the launch's items: a claim
+       * round can hand out nothing but dead electrons (queued ones of a job
+       * the host stopped, or primaries that start outside the chamber), and
+       * the items after them must still be claimed */
+      if (done) break;
+      continue;
+    }
     /* start a step on every lane without one in progress; a step that may
      * reach a boundary waits for the wave's next findEndOfStep pass, which
      * runs once geo_batch lanes wait or no lane could move without it */
@@ -995,7 +1006,7 @@ k_transport(DevScene S, GenDev G) {
      * is redone there from the same state and draws. */
     if (G.tail_lanes > 0) {
       const unsigned long long ma = wave_ballot(alive);
-      if (ma && __popcll(ma) <= G.tail_lanes && wave_ballot(done) != 0ull) {
+      if (ma && done && __popcll(ma) <= G.tail_lanes) {
         queue_append(G, alive, e.px, e.py, e.pz, e.dx, e.dy, e.dz, e.E, e.region, e.primary, e.lin_lo, e.lin_hi,
                      e.job, e.steps, e.nchild, lanemask_lt, nover);
         alive = false;
@@ -1601,6 +1612,23 @@ int max_step_prims(const HostScene& H) {
 int geometry_batch_for(int tuned, int stepPrims, uint64_t items) {
   if (tuned > 0) return tuned;
   return stepPrims >= 3 && items >= kTailMinItems ? 8 : 1;
+}
+
+/* How a launch spreads its items over its waves.  A launch of fewer than
+ * kSpreadItems gives every wave the same share instead of filling the first
+ * ones: a wave's step costs it every path that some lane of it takes, so an
+ * electron in a wave of its own steps two to three times as fast as among 63
+ * others, and such a launch leaves most of the device idle anyway.  (One
+ * pixel of 100 primaries 6.2 -> 2.9 ms, 20,000 primaries on tabulated Si 25.5
+ * -> 19.9 ms; with the line at 16,384 items the latter stays at 26 ms, with
+ * launches of 65,536 to 262,144 items spread as well a line scan of 67,727
+ * primaries takes 25.8 ms instead of 23.1.)  The share leaves the other lanes
+ * of the wave to the secondaries its electrons spawn. */
+void spread_launch(GenDev& G, const monsel_tuning& T, uint64_t items, uint64_t waves) {
+  G.lane_cap = items < kSpreadItems ? (int)std::min<uint64_t>(64, std::max<uint64_t>(1, (items + waves - 1) / waves)) : 64;
+  G.claim_min = std::min(kClaimMin, G.lane_cap);
+  G.claim_chunk = std::min((int)kClaimChunk, G.lane_cap);
+  G.tail_lanes = T.tail_requeue < 0 || items < kTailMinItems ? 0 : (T.tail_requeue > 0 ? T.tail_requeue : kDefaultTailLanes);
 }
 
 /* New primaries per launch when the tuning leaves it open (0): 262,144, so
@@ -2596,11 +2624,9 @@ void run_generation(monsel_ctx_s* C) {
   G.steps_per_launch = C->tuning.steps_per_launch;
   G.geo_batch = geometry_batch_for(C->tuning.geometry_batch, C->batch.step_prims, nprim + C->in_count);
   G.handoff = C->tuning.spawn_handoff >= 0 ? 1 : 0;
-  G.tail_lanes = C->tuning.tail_requeue < 0 || nprim + C->in_count < kTailMinItems
-                     ? 0
-                     : (C->tuning.tail_requeue > 0 ? C->tuning.tail_requeue : kDefaultTailLanes);
   const int block = C->tuning.block_size > 0 ? C->tuning.block_size : 256;
   const int grid = C->n_cu * (C->blocks_per_cu > 0 ? C->blocks_per_cu : 4);
+  spread_launch(G, C->tuning, nprim + C->in_count, (uint64_t)grid * (block / 64));
   /* Event markers time the kernels; MONSEL_NO_EVENT_TIMING=1 leaves them out
    * (hardware-counter profiling sessions reject the marker packets). */
   const bool timing = !getenv("MONSEL_NO_EVENT_TIMING");
@@ -3307,9 +3333,7 @@ int monsel_run_static(monsel_ctx ctx, monsel_scene_id scene, const monsel_job_de
       G.steps_per_launch = T.steps_per_launch;
       G.geo_batch = geometry_batch_for(T.geometry_batch, sd->step_prims, n + in_count);
       G.handoff = T.spawn_handoff >= 0 ? 1 : 0;
-      G.tail_lanes = T.tail_requeue < 0 || n + in_count < kTailMinItems
-                         ? 0
-                         : (T.tail_requeue > 0 ? T.tail_requeue : kDefaultTailLanes);
+      spread_launch(G, T, n + in_count, (uint64_t)grid * (block / 64));
       g_hip_call = "launch k_transport";
       if (sd->dev.has_tabulated)
         hipLaunchKernelGGL(k_transport<true>, dim3(grid), dim3(block), 0, stream, sd->dev, G);

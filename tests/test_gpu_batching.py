@@ -69,6 +69,27 @@ def test_results_independent_of_tuning(M, tuning):
             _same(a, b)
 
 
+@pytest.mark.parametrize("primaries", [1, 63, 4095, 4096, 4097, 8193, 65535, 65536])
+def test_spread_launches_keep_results(M, primaries):
+    """A launch of fewer than 65,536 items gives each wave an equal share of
+    them (1 up to as many items as waves, 2 from one more on, ...); the same
+    job with fewer blocks (other shares), without handoff, and with a
+    regroup interval matches."""
+    from cudamonsel_amd import scenes
+    from cudamonsel_amd.abi import Engine
+    sc = scenes.line_on_substrate()
+    cs = sc.monte.compileScene()
+    cen = [[1e-9, 0.0, sc.beam_z]]
+    ref = None
+    for tuning in (dict(), dict(block_size=64, blocks_per_cu=1), dict(spawn_handoff=-1), dict(steps_per_launch=50)):
+        with Engine(**tuning) as eng:
+            r = eng.result(eng.submit(eng.upload(cs), cen, primaries, 200.0, 0.5e-9, 77))
+        assert r["stats"]["primaries"] == primaries and r["stats"]["queue_overflow"] == 0
+        if ref is None:
+            ref = r
+        _same(ref, r)
+
+
 def test_tail_compaction_keeps_results(M):
     """A launch large enough for tail compaction (>= 65536 items): waves down
     to a few live lanes queue them for the next launch; the results do not
