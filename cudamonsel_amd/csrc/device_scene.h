@@ -80,28 +80,35 @@ struct DCSD {
   int active;
   int nce;
   float breakE;  /* eV */
-  float gamma;   /* 1/(nm eV^1.5) */
+  float gamma15; /* 1.5 gamma, 1/(nm eV^1.5) */
   float minE;    /* eV (barrier height) */
-  float pad;
-  float recipJ[kMaxElem]; /* 1/eV */
-  float beta[kMaxElem];
-  float coef[kMaxElem];   /* eV^2/nm */
+  float pad[3];
+  struct Term {  /* one element's, read with one scalar load */
+    float recipJ; /* 1/eV */
+    float beta;
+    float coef;   /* eV^2/nm */
+    float pad;
+  } el[kMaxElem];
 };
 
-/* One element of an elastic (SelectableElasticSM) mechanism. */
+/* One element of an elastic (SelectableElasticSM) mechanism.  The first
+ * eight words are what a cross-section needs, read with one scalar load. */
 struct DElem {
-  int kind;     /* MONSEL_MECH_*_ELASTIC */
-  int mott;     /* table index or -1 */
-  int method;
-  int Z;
   float natoms; /* scalefactor * density * N_A, atoms / nm^3 */
-  float extrap; /* eV, NISTMottRS extrapolateBelowEnergy */
-  float mottAtMin; /* nm^2 */
   float sfBrowning;
-  float zp17, zp2, zp3, z;
+  float brNum;  /* Browning's 3e-4 Z^1.7, 0.005 Z^1.7 and 0.0007 Z^2 */
+  float brRoot;
+  float brInv;
+  int mott;     /* table index or -1 */
+  float mottAtMin; /* nm^2 */
+  float extrap; /* eV, NISTMottRS extrapolateBelowEnergy (one value per mechanism) */
+  int kind;     /* MONSEL_MECH_*_ELASTIC */
+  int method;
+  float zp3, z;
   float rz13;   /* Z^(1/3) */
   float rz23;   /* Z^(2/3) */
-  float pad[2];
+  int Z;
+  float pad;
 };
 
 struct DMech {

@@ -429,6 +429,7 @@ struct StepStart {
  * contains it).  A free path that ends at least a nudge short of the
  * safety bound (anchored at lane_anchor, less the distance moved since)
  * cannot reach a boundary; every other step needs the geometry. */
+template <bool TAB>
 __device__ __forceinline__ void begin_step_in(const DevScene& S, int region, Elec& e, StepStart& st) {
   PT_BEGIN(t_ra);
   const MONSEL_CS DMSM& msm = S.msms[S.regions[region].msm];
@@ -452,21 +453,19 @@ __device__ __forceinline__ void begin_step_in(const DevScene& S, int region, Ele
         float* esig = lane_esig();
         const bool keep = m.nelem <= kKeptTerms + 1;
         rk = 0.f;
-        for (int i = 0; i < m.nelem; ++i) {
-          const MONSEL_CS DElem& el = S.elems[m.elem0 + i];
-          const float c = elem_sigma(S, el, e.E) * el.natoms;
+        elastic_terms(S, m, e.E, [&](int i, float c) {
           if (keep && i < kKeptTerms) esig[i * kLaneBlock] = c;
           rk += c;
-        }
+        });
       } else {
-        rk = mech_rate(S, m, e.E);
+        rk = mech_rate<TAB>(S, m, e.E);
       }
       rates[k * kLaneBlock] = rk;
       total += rk;
     }
     PT_END(PH_RATE_LOOP, t_rl);
     if (total != 0.f) {
-      float fp = -flog(u[0]) / total;
+      float fp = fdiv(-flog(u[0]), total);
       freePath = fp > maxFreePath ? maxFreePath : fp;
     } else {
       freePath = maxFreePath;
@@ -500,9 +499,10 @@ __device__ __forceinline__ void by_region(const Elec& e, F body) {
   }
 }
 
+template <bool TAB>
 __device__ __forceinline__ void begin_step(const DevScene& S, Elec& e, StepStart& st) {
   PT_UNIFORM(PH_RATES_UNI, e.region);
-  by_region(e, [&](int r0) { begin_step_in(S, r0, e, st); });
+  by_region(e, [&](int r0) { begin_step_in<TAB>(S, r0, e, st); });
 }
 
 /* The check that opens MonteCarloSS::takeStep (MonteCarloSS.cu:107-115):
@@ -590,10 +590,13 @@ __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* j
       int idx = 0;
       float rate = rates[0];
       float cum = rate;
-      while (idx < msm.n_mech - 1 && cum < r) {
-        ++idx;
-        rate = rates[idx * kLaneBlock];
-        cum += rate;
+      for (int k = 1; k < msm.n_mech; ++k) {
+        const float rk = rates[k * kLaneBlock];
+        if (idx == k - 1 && cum < r) {
+          idx = k;
+          rate = rk;
+          cum += rk;
+        }
       }
       bool trapped = false;
       float u[kStepUniforms];
@@ -601,11 +604,22 @@ __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* j
       u[1] = st.u1;
       u[2] = st.u2;
       u[3] = st.u3;
-      step_uniforms_hi(e, kPhiloxKey0, kPhiloxKey1, u);
       PT_END(PH_SELECT, t_se);
-      sp = mech_scatter<TAB>(S, S.mechs[msm.mech0 + idx], e, prevE, rate, trapped, u,
-                             idx == msm.elastic_k && S.mechs[msm.mech0 + idx].nelem <= kKeptTerms + 1 ? lane_esig()
-                                                                                               : nullptr);
+      /* the mechanisms in turn, each for the lanes that chose it: its record
+       * is wave-uniform */
+      Deflect de;
+      de.has = false;
+      for (int k = 0; k < msm.n_mech; ++k) {
+        const unsigned long long turn = wave_ballot(idx == k);
+        if (!turn) continue;
+        const MONSEL_CS DMech& m = S.mechs[msm.mech0 + k];
+        if (lane_in(turn))
+          sp = mech_scatter<TAB>(
+              S, m, e, prevE, rate, trapped, u,
+              [&](float* v) { step_uniforms_hi(e, kPhiloxKey0, kPhiloxKey1, v); }, de,
+              k == msm.elastic_k && m.nelem <= kKeptTerms + 1 ? lane_esig() : nullptr);
+      }
+      if (de.has) deflect(e, de);
       if (sp.has) {
         /* trackSecondaryElectron (MonteCarloSS.cu:165-174) */
         if (!(sp.E > msm.minE)) sp.has = false;
@@ -861,7 +875,7 @@ k_transport(DevScene S, GenDev G) {
      * reach a boundary waits for the wave's next findEndOfStep pass, which
      * runs once geo_batch lanes wait or no lane could move without it */
     if (alive && !pending) {
-      begin_step(S, e, st);
+      begin_step<TAB>(S, e, st);
       pending = true;
     }
     const unsigned long long m_geo = wave_ballot(alive && st.geo);
@@ -1331,9 +1345,9 @@ __global__ void k_probe_elastic(DevScene S, int mech, int element, int n, const 
   float EeV = E[i], r1 = u[2 * i], r2 = u[2 * i + 1];
   float ca;
   if (el.kind == MONSEL_MECH_BROWNING_ELASTIC || (el.kind == MONSEL_MECH_NISTMOTT_ELASTIC && EeV < el.extrap))
-    ca = browning_cos(el, EeV, r1, r2);
+    ca = browning_cos(el.z, el.zp3, EeV, r1, r2);
   else if (el.kind == MONSEL_MECH_RUTHERFORD_ELASTIC || EeV >= kMaxNISTMott)
-    ca = rutherford_cos(el, EeV, r1);
+    ca = rutherford_cos(el.rz23, EeV, r1);
   else
     ca = mott_cos(S, el.mott, EeV, r1);
   out[i] = acosf(fminf(1.f, fmaxf(-1.f, ca)));
@@ -1360,7 +1374,10 @@ __global__ void k_probe_scatter(DevScene S, int mech, int n, const float* prevE,
   for (int k = 0; k < 6; ++k) uu[2 + k] = u[6 * i + k];
   bool trapped = false;
   const float rate = mech_rate(S, m, prevE[i]);
-  Spawn sp = mech_scatter(S, m, e, prevE[i], rate, trapped, uu);
+  Deflect de;
+  de.has = false;
+  Spawn sp = mech_scatter(S, m, e, prevE[i], rate, trapped, uu, [](float*) {}, de);
+  if (de.has) deflect(e, de);
   float* o = out + 11 * (size_t)i;
   o[0] = e.dx;
   o[1] = e.dy;
@@ -1662,12 +1679,12 @@ DCSD make_csd(const monsel_material_desc& m, double breakE) {
   }
   gamma /= pow(breakE, 3.5);
   for (int i = 0; i < c.nce; ++i) {
-    c.recipJ[i] = (float)(recipJ[i] * kE);
-    c.beta[i] = (float)beta[i];
-    c.coef[i] = (float)(coef[i] * 1e-9 / (kE * kE));
+    c.el[i].recipJ = (float)(recipJ[i] * kE);
+    c.el[i].beta = (float)beta[i];
+    c.el[i].coef = (float)(coef[i] * 1e-9 / (kE * kE));
   }
   c.breakE = (float)(breakE / kE);
-  c.gamma = (float)(gamma * 1e-9 * pow(kE, 1.5));
+  c.gamma15 = 1.5f * (float)(gamma * 1e-9 * pow(kE, 1.5));
   c.minE = (float)(bh / kE);
   return c;
 }
@@ -1786,8 +1803,10 @@ HostScene compile_scene(const monsel_scene_desc* d) {
             el.Z = Z;
             el.method = e.method < 1 ? 1 : e.method;
             el.z = (float)Z;
-            el.zp17 = (float)pow((double)Z, 1.7);
-            el.zp2 = (float)pow((double)Z, 2.0);
+            const float zp17 = (float)pow((double)Z, 1.7);
+            el.brNum = 3.0e-4f * zp17;
+            el.brRoot = 0.005f * zp17;
+            el.brInv = 0.0007f * (float)pow((double)Z, 2.0);
             el.zp3 = (float)pow((double)Z, 3.0);
             el.rz13 = (float)pow((double)Z, 1.0 / 3.0);
             el.rz23 = (float)pow((double)Z, 2.0 / 3.0);

@@ -50,6 +50,15 @@ MD float fsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 MD float flog(float x) { return __builtin_amdgcn_logf(x) * 0.693147180559945309f; }
 MD float fexp(float x) { return __builtin_amdgcn_exp2f(x * 1.442695040888963407f); }
 
+/* a / b as a times the hardware reciprocal: what the compiler's own division
+ * gives for |b| <= 2^96 (beyond it rescales b around the reciprocal's flush
+ * to zero: four more instructions for denominators no transport quantity
+ * reaches).  The product is not contracted into a following sum. */
+MD float fdiv(float a, float b) {
+#pragma clang fp contract(off)
+  return a * __builtin_amdgcn_rcpf(b);
+}
+
 /* Philox4x32-10 (Salmon et al., SC'11).  Counter words: (block, lineage lo,
  * lineage hi, primary index) under one fixed key; a job's seed enters
  * through the lineage of its primaries (splitmix64 of the seed), a
@@ -201,22 +210,20 @@ MD int u_index0(float reduced, int len) {
 
 /* ------------------------------------------------- elastic (per element) */
 
-/* BrowningEmpiricalCrossSection.cu:24-29 (nm^2) */
-MD float browning_sigma(const MONSEL_CS DElem& el, float EeV) {
-  float e = EeV * 1.0e-3f;
-  float re = fsqrt(e);
-  return 3.0e-4f * el.zp17 / (e + 0.005f * el.zp17 * re + 0.0007f * el.zp2 / re);
+/* BrowningEmpiricalCrossSection.cu:24-29 (nm^2); e in keV, re its root and
+ * inv_re the root's reciprocal */
+MD float browning_sigma(const MONSEL_CS DElem& el, float e, float re, float inv_re) {
+#pragma clang fp contract(off)
+  return el.brNum * __builtin_amdgcn_rcpf(__builtin_fmaf(re, el.brRoot, e) + el.brInv * inv_re);
 }
 
 /* BrowningEmpiricalCrossSection.cu:31-45 -> cos(theta) */
-MD float browning_cos(const MONSEL_CS DElem& el, float EeV, float r1, float r2) {
-  float e = EeV * 1.0e-3f;
-  float r = (300.0f * e / el.z) + (el.zp3 / (3.0e5f * e));
-  if (r1 <= r / (r + 1.f)) {
-    float alpha = 7.0e-3f / e;
-    return 1.0f - ((2.0f * alpha * r2) / (alpha - r2 + 1.f));
-  }
-  return 1.f - 2.0f * r2;
+MD float browning_cos(float z, float zp3, float EeV, float r1, float r2) {
+  const float e = EeV * 1.0e-3f;
+  const float r = fdiv(300.0f * e, z) + fdiv(zp3, 3.0e5f * e);
+  const float alpha = fdiv(7.0e-3f, e);
+  const bool screened = r1 <= fdiv(r, r + 1.f);
+  return 1.0f - (screened ? fdiv(2.0f * alpha * r2, alpha - r2 + 1.f) : 2.0f * r2);
 }
 
 /* ScreenedRutherfordScatteringAngle.cu:24-39 (sigma nm^2, cos theta) */
@@ -224,15 +231,15 @@ MD float rutherford_sigma(const MONSEL_CS DElem& el, float EeV) {
   const float K1 = 7.670843088080456e-38f / 1.60217653e-19f * 1.0e18f;
   const float K2 = 5.44967975966321e-19f / 1.60217653e-19f;
   float zp = el.rz13;
-  return K1 * zp * (1.f + el.z) / (EeV + K2 * zp * zp);
+  return fdiv(K1 * zp * (1.f + el.z), __builtin_fmaf(zp, K2 * zp, EeV));
 }
-MD float rutherford_cos(const MONSEL_CS DElem& el, float EeV, float r) {
+MD float rutherford_cos(float rz23, float EeV, float r) {
   const float K = 5.44968e-19f / 1.60217653e-19f;
-  float alpha = K * el.rz23 / EeV;
+  float alpha = fdiv(K * rz23, EeV);
   /* alpha - r + 1 summed as (1 - r) + alpha: 1 - r is exact for r >= 1/2,
    * so the denominator keeps its relative precision when alpha and 1 - r are
    * both small (E >= 20 keV, r near 1) */
-  return 1.f - 2.0f * alpha * r / ((1.f - r) + alpha);
+  return 1.f - fdiv(2.0f * alpha * r, (1.f - r) + alpha);
 }
 
 /* The hot tables: the cross-section nodes (Spwem, 61 floats) of the first
@@ -257,36 +264,67 @@ MD void stage_mott_sigma(const DevScene& S) {
   __syncthreads();
 }
 
-/* NISTMottRS::totalCrossSection (NISTMottRS.cu:103-119), nm^2 */
-MD float mott_table_sigma(const DevScene& S, int mott, float EeV) {
-  float red = (flog(EeV) - kMottLn50) * kMottInvParam;
-  int i0 = u_index0(red, kMottNE);
+/* NISTMottRS::totalCrossSection (NISTMottRS.cu:103-119), nm^2: the window
+ * of the energy grid and its weights, shared by the elements of a material */
+struct MottWindow {
+  int i0;
+  float l0, l1, l2, l3;
+};
+MD MottWindow mott_window(float EeV) {
+  MottWindow w;
+  const float red = (flog(EeV) - kMottLn50) * kMottInvParam;
+  w.i0 = u_index0(red, kMottNE);
+  lagrange4_w(red - (float)w.i0, w.l0, w.l1, w.l2, w.l3);
+  return w;
+}
+MD float mott_table_sigma(const DevScene& S, int mott, const MottWindow& w) {
   float f0, f1, f2, f3;
   if (mott < kLdsMott) {
-    const float* f = lds_spwem() + mott * kMottNE + i0;
+    const float* f = lds_spwem() + mott * kMottNE + w.i0;
     f0 = f[0];
     f1 = f[1];
     f2 = f[2];
     f3 = f[3];
   } else {
-    const MONSEL_CS float* f = S.mott_spwem + mott * kMottNE + i0;
+    const MONSEL_CS float* f = S.mott_spwem + mott * kMottNE + w.i0;
     f0 = f[0];
     f1 = f[1];
     f2 = f[2];
     f3 = f[3];
   }
-  return kA0nm2 * lagrange4(red - (float)i0, f0, f1, f2, f3);
+  return kA0nm2 * (w.l0 * f0 + w.l1 * f1 + w.l2 * f2 + w.l3 * f3);
 }
 
-MD float elem_sigma(const DevScene& S, const MONSEL_CS DElem& el, float EeV) {
-  if (el.kind == MONSEL_MECH_BROWNING_ELASTIC) return browning_sigma(el, EeV);
-  if (el.kind == MONSEL_MECH_RUTHERFORD_ELASTIC) return rutherford_sigma(el, EeV);
-  if (EeV < el.extrap) {
-    if (el.method == 3) return el.mottAtMin * EeV / el.extrap;
-    return el.sfBrowning * browning_sigma(el, EeV);
+/* The terms sigma_i * atoms_i of an elastic mechanism at energy EeV, given in
+ * element order to f(i, term).  The elements of a mechanism share its kind
+ * and extrapolation energy, so which formula holds depends on the energy
+ * alone and what the elements share is formed once. */
+template <class F>
+MD void elastic_terms(const DevScene& S, const MONSEL_CS DMech& m, float EeV, F f) {
+#pragma clang fp contract(off)
+  const int n = m.nelem;
+  if (n <= 0) return;
+  const MONSEL_CS DElem* el = S.elems + m.elem0;
+  const bool mott = m.kind == MONSEL_MECH_NISTMOTT_ELASTIC;
+  const bool low = mott && EeV < el[0].extrap;
+  if (m.kind == MONSEL_MECH_BROWNING_ELASTIC || low) {
+    if (mott && el[0].method == 3) {
+      for (int i = 0; i < n; ++i) f(i, fdiv(el[i].mottAtMin * EeV, el[i].extrap) * el[i].natoms);
+    } else {
+      const float e = EeV * 1.0e-3f;
+      const float re = fsqrt(e);
+      const float inv_re = __builtin_amdgcn_rcpf(re);
+      for (int i = 0; i < n; ++i) {
+        const float b = browning_sigma(el[i], e, re, inv_re);
+        f(i, (mott ? el[i].sfBrowning * b : b) * el[i].natoms);
+      }
+    }
+  } else if (mott && EeV < kMaxNISTMott) {
+    const MottWindow w = mott_window(EeV);
+    for (int i = 0; i < n; ++i) f(i, mott_table_sigma(S, el[i].mott, w) * el[i].natoms);
+  } else {
+    for (int i = 0; i < n; ++i) f(i, rutherford_sigma(el[i], EeV) * el[i].natoms);
   }
-  if (EeV < kMaxNISTMott) return mott_table_sigma(S, el.mott, EeV);
-  return rutherford_sigma(el, EeV);
 }
 
 /* NISTMottRS::randomScatteringAngle table branch: bicubic Lagrange on X1
@@ -319,8 +357,16 @@ MD float mott_cos(const DevScene& S, int mott, float EeV, float u) {
  * < 5e-13 relative), the hardware log2/exp2 above (relative error of the
  * result < 1e-4 there, where it is at least 6.7e-4 in size). */
 MD float nieminen_factor(float eps) {
-  if (eps < 1e-3f) return eps * (-2.f / 3.f + eps * (5.f / 9.f - eps * (40.f / 81.f)));
-  return __builtin_amdgcn_exp2f(-(2.f / 3.f) * __builtin_amdgcn_logf(1.f + eps)) - 1.f;
+  const float series = eps * (-2.f / 3.f + eps * (5.f / 9.f - eps * (40.f / 81.f)));
+  const float power = __builtin_amdgcn_exp2f(-(2.f / 3.f) * __builtin_amdgcn_logf(1.f + eps)) - 1.f;
+  return eps < 1e-3f ? series : power;
+}
+
+/* sum over the elements of coef ln(E / J + beta) */
+MD float joy_luo_sum(const MONSEL_CS DCSD& c, float kE) {
+  float s = 0.f;
+  for (int i = 0; i < c.nce; ++i) s += c.el[i].coef * flog(c.el[i].recipJ * kE + c.el[i].beta);
+  return s;
 }
 
 /* JoyLuoNieminenCSD::compute (JoyLuoNieminenCSD.cu:91-121) with the
@@ -333,20 +379,22 @@ MD float csd_compute_split(const MONSEL_CS DCSD& c, float len, float kE);
 /* The common case in straight-line code: one segment, no halving (the
  * first pass of csd_compute_split, with the same arithmetic). */
 MD float csd_compute(const MONSEL_CS DCSD& c, float len, float kE) {
+#pragma clang fp contract(off)
   if (!c.active || c.nce == 0) return 0.f;
   if (kE < c.minE || kE <= 0.f) return 0.f;
+  float dE;
   if (kE <= c.breakE) {
-    const float eps = 1.5f * c.gamma * len * kE * fsqrt(kE);
-    return kE * nieminen_factor(eps);
+    dE = kE * nieminen_factor(c.gamma15 * len * kE * fsqrt(kE));
+  } else {
+    const float loss = fdiv(joy_luo_sum(c, kE) * len, kE);
+    dE = -loss;
+    if (loss > 0.1f * kE) dE = csd_compute_split(c, len, kE);
   }
-  float s = 0.f;
-  for (int i = 0; i < c.nce; ++i) s += c.coef[i] * flog(c.recipJ[i] * kE + c.beta[i]);
-  const float loss = s * len / kE;
-  if (!(loss > 0.1f * kE)) return -loss;
-  return csd_compute_split(c, len, kE);
+  return dE;
 }
 
 MD float csd_compute_split(const MONSEL_CS DCSD& c, float len, float kE) {
+#pragma clang fp contract(off)
   float E = kE, total = 0.f;
   uint32_t pending = 0;
   int d = 0;
@@ -355,12 +403,9 @@ MD float csd_compute_split(const MONSEL_CS DCSD& c, float len, float kE) {
     float dE = 0.f;
     if (!(E < c.minE || E <= 0.f)) {
       if (E <= c.breakE) {
-        const float eps = 1.5f * c.gamma * seg * E * fsqrt(E);
-        dE = E * nieminen_factor(eps);
+        dE = E * nieminen_factor(c.gamma15 * seg * E * fsqrt(E));
       } else {
-        float s = 0.f;
-        for (int i = 0; i < c.nce; ++i) s += c.coef[i] * flog(c.recipJ[i] * E + c.beta[i]);
-        const float loss = s * seg / E;
+        const float loss = fdiv(joy_luo_sum(c, E) * seg, E);
         if (loss > 0.1f * E && d < 30) {
           pending |= 1u << (d + 1);
           d += 1;
@@ -563,14 +608,12 @@ MD double nu_interp(const DevScene& S, int table, int order, const double* x, bo
 
 MD float elastic_rate(const DevScene& S, const MONSEL_CS DMech& m, float EeV) {
   float tot = 0.f;
-  for (int i = 0; i < m.nelem; ++i) {
-    const MONSEL_CS DElem& el = S.elems[m.elem0 + i];
-    tot += elem_sigma(S, el, EeV) * el.natoms;
-  }
+  elastic_terms(S, m, EeV, [&](int, float c) { tot += c; });
   return tot;
 }
 
-/* ScatterMechanism::scatterRate (1/nm) */
+/* ScatterMechanism::scatterRate (1/nm); TAB as for mech_scatter */
+template <bool TAB = true>
 MD float mech_rate(const DevScene& S, const MONSEL_CS DMech& m, float EeV) {
   switch (m.kind) {
     case MONSEL_MECH_NISTMOTT_ELASTIC:
@@ -585,13 +628,13 @@ MD float mech_rate(const DevScene& S, const MONSEL_CS DMech& m, float EeV) {
       return m.p[0] * fexp(-m.p[1] * EeV);
     case MONSEL_MECH_PHONON: { /* GanachaudMokraniPhononInelasticSM.cu:46-72 */
       if (EeV < m.p[0]) return 0.f;
-      float x = m.p[0] / EeV;
-      if (x < 0.1f) return m.p[1] * x * flog(4.f / x);
-      if (x >= 1.f) return 0.f;
-      float temp = fsqrt(1.f - x);
-      return m.p[1] * x * flog((1.f + temp) / (1.f - temp));
+      const float x = fdiv(m.p[0], EeV);
+      const float temp = fsqrt(1.f - x);
+      const bool small = x < 0.1f;
+      const float rate = m.p[1] * x * flog(fdiv(small ? 4.f : 1.f + temp, small ? x : 1.f - temp));
+      return small || !(x >= 1.f) ? rate : 0.f;
     }
-    case MONSEL_MECH_TABULATED_INELASTIC: { /* TabulatedInelasticSM.cu:436-459 */
+    case MONSEL_MECH_TABULATED_INELASTIC: if constexpr (TAB) { /* TabulatedInelasticSM.cu:436-459 */
       float kE = (EeV + m.p[TP_OFFSET]) * kEcharge;
       if (kE < m.p[TP_IIMFPDOM0]) return 0.f;
       return m.p[TP_RATEMULT] * nu_d1<float, 1>(S, S.nu[m.table[0]], kE) * 1.0e-9f;
@@ -780,14 +823,33 @@ MD Spawn tabulated_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e,
   return se;
 }
 
-/* ScatterMechanism::scatter.  `rate` is this mechanism's scatterRate at
- * prevE, as summed when the step's free path was drawn. */
-/* TAB = false leaves the tabulated mechanism out of the code (its FP64
- * scatter sets the register budget of every kernel that contains it); only
- * for scenes without one. */
-template <bool TAB = true>
+/* A deflection of the electron's direction left for the end of the scatter:
+ * polar angle by its cosine, azimuth by its uniform. */
+struct Deflect {
+  bool has;
+  float cos_polar, u_azimuth;
+};
+
+/* Electron::updateDirection by d */
+MD void deflect(Elec& e, const Deflect& d) {
+  const float ca = fminf(1.f, fmaxf(-1.f, d.cos_polar));
+  const float sa = fsqrt(fmaxf(0.f, 1.f - ca * ca));
+  float sb, cb;
+  __sincosf(kTwoPI * d.u_azimuth, &sb, &cb);
+  rotate_dir(e.dx, e.dy, e.dz, ca, sa, cb, sb);
+}
+
+/* ScatterMechanism::scatter of mechanism m (the same one on every active
+ * lane).  `rate` is this mechanism's scatterRate at prevE, as summed when the
+ * step's free path was drawn; esig, if given, holds the elastic mechanism's
+ * first nelem - 1 terms (lane stride kLaneBlock); draw_hi(u) draws u[4..7].
+ * A deflection of the primary is left in `de` for the caller, which applies
+ * it once for every mechanism.  TAB = false leaves the tabulated mechanism
+ * out of the code (its FP64 scatter sets the register budget of every kernel
+ * that contains it); only for scenes without one. */
+template <bool TAB = true, class Draw>
 MD Spawn mech_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e, float prevE, float rate, bool& trapped,
-                      const float* u, const float* esig = nullptr) {
+                      float* u, Draw draw_hi, Deflect& de, const float* esig = nullptr) {
   Spawn se;
   se.has = false;
   switch (m.kind) {
@@ -797,36 +859,46 @@ MD Spawn mech_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e, floa
       PT_BEGIN(t_el);
       /* first element whose running sum of sigma * atoms reaches u * rate
        * (the last if none does); the sum is re-formed in the order
-       * elastic_rate formed it, from the rate's own terms when the caller
-       * kept them (esig: the first nelem - 1 terms, lane stride kLaneBlock) */
+       * elastic_rate formed it.  The elements pass by wave-uniformly, and a
+       * lane keeps the angle parameters of its choice. */
       const float r = u[2] * rate;
-      int idx = 0;
+      const MONSEL_CS DElem* el = S.elems + m.elem0;
+      const bool nist = m.kind == MONSEL_MECH_NISTMOTT_ELASTIC;
+      const float extrap = el[0].extrap;
+      int mott = el[0].mott;
+      float z = el[0].z, zp3 = el[0].zp3, rz23 = el[0].rz23;
       float cum = 0.f;
-      for (; idx < m.nelem - 1; ++idx) {
-        const MONSEL_CS DElem& el = S.elems[m.elem0 + idx];
-        cum += esig ? esig[idx * kLaneBlock] : elem_sigma(S, el, prevE) * el.natoms;
-        if (!(cum < r)) break;
+      bool open = true;
+      auto term = [&](int i, float c) {
+        if (i < m.nelem - 1) {
+          cum += c;
+          open = open && cum < r;
+          if (open) {
+            mott = el[i + 1].mott;
+            z = el[i + 1].z;
+            zp3 = el[i + 1].zp3;
+            rz23 = el[i + 1].rz23;
+          }
+        }
+      };
+      if (esig) {
+        for (int i = 0; i < m.nelem - 1; ++i) term(i, esig[i * kLaneBlock]);
+      } else {
+        elastic_terms(S, m, prevE, term);
       }
-      const MONSEL_CS DElem& el = S.elems[m.elem0 + idx];
+      draw_hi(u);
       /* the polar angle takes one uniform (two for Browning), the azimuth
        * the next one (SelectableElasticSM.cu:62-64) */
-      float ca, ub;
-      if (el.kind == MONSEL_MECH_BROWNING_ELASTIC ||
-          (el.kind == MONSEL_MECH_NISTMOTT_ELASTIC && prevE < el.extrap)) {
-        ca = browning_cos(el, prevE, u[3], u[4]);
-        ub = u[5];
-      } else if (el.kind == MONSEL_MECH_RUTHERFORD_ELASTIC || prevE >= kMaxNISTMott) {
-        ca = rutherford_cos(el, prevE, u[3]);
-        ub = u[4];
+      de.has = true;
+      de.u_azimuth = u[4];
+      if (m.kind == MONSEL_MECH_BROWNING_ELASTIC || (nist && prevE < extrap)) {
+        de.cos_polar = browning_cos(z, zp3, prevE, u[3], u[4]);
+        de.u_azimuth = u[5];
+      } else if (nist && !(prevE >= kMaxNISTMott)) {
+        de.cos_polar = mott_cos(S, mott, prevE, u[3]);
       } else {
-        ca = mott_cos(S, el.mott, prevE, u[3]);
-        ub = u[4];
+        de.cos_polar = rutherford_cos(rz23, prevE, u[3]);
       }
-      ca = fminf(1.f, fmaxf(-1.f, ca));
-      float sa = fsqrt(fmaxf(0.f, 1.f - ca * ca));
-      float sb, cb;
-      __sincosf(kTwoPI * ub, &sb, &cb);
-      rotate_dir(e.dx, e.dy, e.dz, ca, sa, cb, sb);
       PT_END(PH_ELASTIC, t_el);
       return se;
     }
@@ -854,23 +926,22 @@ MD Spawn mech_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e, floa
         PT_END(PH_PHONON, t_ph);
         return se;
       }
-      float x = m.p[0] / kE0;
+      float x = fdiv(m.p[0], kE0);
       const float r0 = u[2], r1 = u[3];
       float ct;
       /* x^a = 2^(a log2 x) for x > 0, on the hardware exp2/log2 */
       if (x < 0.1f)
-        ct = 1.f + ((x * x) - __builtin_amdgcn_exp2f(4.f * r0 + (2.f - 2.f * r0) * __builtin_amdgcn_logf(x))) / 8.f;
+        ct = 1.f + ((x * x) - __builtin_amdgcn_exp2f(
+                                  __builtin_fmaf(2.f - 2.f * r0, __builtin_amdgcn_logf(x), 4.f * r0))) / 8.f;
       else {
         float root = fsqrt(1.f - x);
         float temp = __builtin_amdgcn_exp2f(
-            r0 * __builtin_amdgcn_logf(((-2.f * (1.f + root)) + x) / ((-2.f * (1.f - root)) + x)));
-        ct = temp + (((x - 2.f) * (temp - 1.f)) / 2.f / root);
+            r0 * __builtin_amdgcn_logf(fdiv((-2.f * (1.f + root)) + x, (-2.f * (1.f - root)) + x)));
+        ct = temp + fdiv(((x - 2.f) * (temp - 1.f)) / 2.f, root);
       }
-      ct = fminf(1.f, fmaxf(-1.f, ct));
-      float st = fsqrt(fmaxf(0.f, 1.f - ct * ct));
-      float sb, cb;
-      __sincosf(kTwoPI * r1, &sb, &cb);
-      rotate_dir(e.dx, e.dy, e.dz, ct, st, cb, sb);
+      de.has = true;
+      de.cos_polar = ct;
+      de.u_azimuth = r1;
       e.E = kE0 - m.p[0];
       PT_END(PH_PHONON, t_ph);
       return se;
@@ -878,6 +949,7 @@ MD Spawn mech_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e, floa
     case MONSEL_MECH_TABULATED_INELASTIC:
       if constexpr (TAB) {
         PT_BEGIN(t_tb);
+        draw_hi(u);
         Spawn r = tabulated_scatter(S, m, e, u);
         PT_END(PH_TABULATED, t_tb);
         return r;
