@@ -38,6 +38,7 @@ struct DPrim {
   int kind;
   int first_plane;
   int n_planes;
+  int tie;       /* bit k: a line within plane k counts as inside (plane_tie_break) */
   float sdscale; /* planes: min over the planes of 1/|n| (distance bounds); 1 otherwise */
   float e0[3];   /* cylinder end0 / sphere centre (nm) */
   float ax[3];   /* cylinder unit axis */
@@ -45,6 +46,7 @@ struct DPrim {
   float r2;      /* radius^2 (nm^2) */
   float axv[3];  /* cylinder axis vector end1-end0 (nm), for point containment */
   float len2;    /* |axv|^2 */
+  float pad[3];
   float4 pl[4];  /* the first planes of a multi-plane primitive again, inline (one
                   * fewer dependent load for the common primitives) */
 };

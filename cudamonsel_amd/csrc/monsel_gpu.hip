@@ -313,7 +313,7 @@ __device__ __forceinline__ int barrier_core(const DevScene& S, const MONSEL_CS D
   if (compat) {
     nbx = e.dx; nby = e.dy; nbz = e.dz; /* ExpQMBarrierSM.cu:111 */
   } else {
-    float m2 = nbx * nbx + nby * nby + nbz * nbz;
+    const float m2 = dot3(nbx, nby, nbz, nbx, nby, nbz);
     if (m2 > 0.f) {
       float inv = __builtin_amdgcn_rsqf(m2);
       nbx *= inv; nby *= inv; nbz *= inv;
@@ -321,7 +321,7 @@ __device__ __forceinline__ int barrier_core(const DevScene& S, const MONSEL_CS D
       nbx = e.dx; nby = e.dy; nbz = e.dz;
     }
   }
-  const float cosalpha = compat ? 1.f : (e.dx * nbx + e.dy * nby + e.dz * nbz);
+  const float cosalpha = compat ? 1.f : dot3(e.dy, e.dx, e.dz, nby, nbx, nbz);
   const float dd = nudge_nm(e.px, e.py, e.pz);
   if (cosalpha <= 0.f) {
     e.px -= dd * nbx; e.py -= dd * nby; e.pz -= dd * nbz;
@@ -484,25 +484,13 @@ __device__ __forceinline__ void begin_step_in(const DevScene& S, int region, Ele
 
 /* The lanes of a wave take their turn by region (one pass per region present,
  * normally one): within a pass the region index is wave-uniform, so the
- * scene records it selects are read with scalar loads.  The loop runs over a
- * wave-uniform mask of the lanes still to do: a loop left lane by lane would
- * let the compiler run the body after it, where the region is a per-lane
- * value again and every scene read a vector load. */
-template <class F>
-__device__ __forceinline__ void by_region(const Elec& e, F body) {
-  unsigned long long todo = wave_ballot(true);
-  while (todo) {
-    const int r0 = __builtin_amdgcn_readlane(e.region, __ffsll((long long)todo) - 1);
-    const unsigned long long turn = wave_ballot(e.region == r0) & todo;
-    if (lane_in(turn)) body(r0);
-    todo &= ~turn;
-  }
-}
-
+ * scene records it selects are read with scalar loads.  (A loop left lane by
+ * lane instead would let the compiler run the body after it, where the region
+ * is a per-lane value again and every scene read a vector load.) */
 template <bool TAB>
 __device__ __forceinline__ void begin_step(const DevScene& S, Elec& e, StepStart& st) {
   PT_UNIFORM(PH_RATES_UNI, e.region);
-  by_region(e, [&](int r0) { begin_step_in<TAB>(S, r0, e, st); });
+  by_value(true, e.region, [&](int r0) { begin_step_in<TAB>(S, r0, e, st); });
 }
 
 /* The check that opens MonteCarloSS::takeStep (MonteCarloSS.cu:107-115):
@@ -512,8 +500,9 @@ __device__ __forceinline__ void begin_step(const DevScene& S, Elec& e, StepStart
 __device__ __forceinline__ bool locate(const DevScene& S, const JobRec* jobs, Elec& e, int r) {
   PT_BEGIN(t_co);
   e.safe = 0.f;
-  if (r < 0 || !shape_contains(S, S.regions[r].sh, e.px, e.py, e.pz))
-    e.region = containing_sub_region(S, jobs[e.job].root, e.px, e.py, e.pz);
+  bool in = false;
+  by_value(r >= 0, r, [&](int r0) { in = shape_contains(S, S.regions[r0].sh, e.px, e.py, e.pz); });
+  if (!in) e.region = containing_sub_region(S, jobs[e.job].root, e.px, e.py, e.pz);
   PT_END(PH_CONTAIN, t_co);
   return e.region >= 0;
 }
@@ -528,12 +517,14 @@ __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* j
                                               Spawn& sp, int maxSteps, const StepStart& st) {
   sp.has = false;
   const MONSEL_CS DMSM& msm = S.msms[S.regions[region].msm];
+  /* the reference's barrier ignores the surface normal in compat mode */
+  const bool normals = (S.compat & MONSEL_COMPAT_BARRIER_NORMAL) == 0u;
   const float freePath = st.freePath;
   const float px = e.px, py = e.py, pz = e.pz;
   StepEnd se;
   if (st.geo) {
     PT_BEGIN(t_ge);
-    se = find_end_of_step(S, region, px, py, pz, e.dx, e.dy, e.dz, freePath);
+    se = find_end_of_step(S, region, px, py, pz, e.dx, e.dy, e.dz, freePath, normals);
     PT_END(PH_GEOM, t_ge);
   } else {
     se.t = freePath;
@@ -638,22 +629,24 @@ __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* j
     } else {
       /* ExpQMBarrierSM.cu:77-96: outward normal of the struck shape, negated
        * when entering a child region (unused in compat mode) */
-      float nbx = 0.f, nby = 0.f, nbz = 0.f;
-      if (!(S.compat & MONSEL_COMPAT_BARRIER_NORMAL)) {
-        if (is_containing_region(S, region, next)) {
-          int struck = next;
-          while (S.regions[struck].parent != region) struck = S.regions[struck].parent;
-          if (struck == se.winner) {
-            nbx = -se.winNx; nby = -se.winNy; nbz = -se.winNz;
+      by_value(true, next, [&](int to) {
+        float nbx = 0.f, nby = 0.f, nbz = 0.f;
+        if (normals) {
+          if (is_containing_region(S, region, to)) {
+            int struck = to;
+            while (S.regions[struck].parent != region) struck = S.regions[struck].parent;
+            if (struck == se.winner) {
+              nbx = -se.winNx; nby = -se.winNy; nbz = -se.winNz;
+            } else {
+              ShapeHit h = shape_first(S, S.regions[struck].sh, px, py, pz, e.dx, e.dy, e.dz, freePath, true);
+              nbx = -h.nx; nby = -h.ny; nbz = -h.nz;
+            }
           } else {
-            ShapeHit h = shape_first(S, S.regions[struck].sh, px, py, pz, e.dx, e.dy, e.dz, freePath);
-            nbx = -h.nx; nby = -h.ny; nbz = -h.nz;
+            nbx = se.ownNx; nby = se.ownNy; nbz = se.ownNz;
           }
-        } else {
-          nbx = se.ownNx; nby = se.ownNy; nbz = se.ownNz;
         }
-      }
-      barrier_core(S, msm, S.msms[S.regions[next].msm], e, next, nbx, nby, nbz, st.u1);
+        barrier_core(S, msm, S.msms[S.regions[to].msm], e, to, nbx, nby, nbz, st.u1);
+      });
     }
     /* MonteCarloSS.cu:146-148: nudge along the new direction; the region is
      * re-located by the check that opens the next step */
@@ -685,7 +678,7 @@ __device__ __forceinline__ int finish_step(const DevScene& S, const JobRec* jobs
                                            const StepStart& st) {
   PT_UNIFORM(PH_GEOM_UNI, e.region);
   int res = STEP_CONTINUE;
-  by_region(e, [&](int r0) { res = finish_step_in<TAB>(S, jobs, r0, e, sp, maxSteps, st); });
+  by_value(true, e.region, [&](int r0) { res = finish_step_in<TAB>(S, jobs, r0, e, sp, maxSteps, st); });
   return res;
 }
 
@@ -1430,7 +1423,7 @@ __global__ void k_probe_step_end(DevScene S, int region, int n, const float* p0,
   float bx = p1[3 * i] - ax, by = p1[3 * i + 1] - ay, bz = p1[3 * i + 2] - az;
   float L = sqrtf(bx * bx + by * by + bz * bz);
   float inv = 1.f / L;
-  StepEnd se = find_end_of_step(S, region, ax, ay, az, bx * inv, by * inv, bz * inv, L);
+  StepEnd se = find_end_of_step(S, region, ax, ay, az, bx * inv, by * inv, bz * inv, L, true);
   out_u[i] = se.boundary ? se.t / L : kInf;
   out_next[i] = se.next;
   out_n[3 * i] = se.boundary ? se.winNx : 0.f;
@@ -1969,6 +1962,8 @@ HostScene compile_scene(const monsel_scene_desc* d) {
           double b = (n[0] * pl.point[0] + n[1] * pl.point[1] + n[2] * pl.point[2]) * 1e9;
           H.planes.push_back(make_float4((float)n[0], (float)n[1], (float)n[2], (float)b));
           if (k < kInlinePlanes) p.pl[k] = H.planes.back();
+          const float4& f = H.planes.back();
+          if (plane_tie_break(f.x, f.y, f.z)) p.tie |= 1 << k;
           maxn = std::max(maxn, sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]));
         }
         /* min over the planes of 1/|n|, rounded down (distance bounds) */

@@ -152,6 +152,12 @@ constexpr int kLaneBlock = 256;
 
 /* ----------------------------------------------------------- math ------ */
 
+/* dot product, its rounding fixed whatever surrounds it */
+MD float dot3(float ax, float ay, float az, float bx, float by, float bz) {
+#pragma clang fp contract(off)
+  return __builtin_fmaf(az, bz, __builtin_fmaf(ax, bx, ay * by));
+}
+
 /* Electron::updateDirection (Electron.cu:111-131) on a unit vector: deflect
  * by polar angle (ca = cos, sa = sin) and azimuth (cb, sb). */
 MD void rotate_dir(float& dx, float& dy, float& dz, float ca, float sa, float cb, float sb) {
@@ -966,8 +972,9 @@ struct Interval {
   int fin, fout; /* face codes: plane index, or -1 cap0 / -2 cap1 / -3 side */
 };
 
-MD bool plane_tie_break(float nx, float ny, float nz) {
-  /* NormalMultiPlaneShape.cu:26-38 */
+/* NormalMultiPlaneShape.cu:26-38: whether a line within the plane of normal
+ * (nx, ny, nz) counts as inside */
+inline __host__ __device__ bool plane_tie_break(float nx, float ny, float nz) {
   if (nx < 0.f) return false;
   if (nx == 0.f) {
     if (ny < 0.f) return false;
@@ -976,105 +983,85 @@ MD bool plane_tie_break(float nx, float ny, float nz) {
   return true;
 }
 
-/* plane k of a multi-plane primitive */
+/* plane k of a multi-plane primitive (k may differ by lane) */
 MD float4 prim_plane(const DevScene& S, const MONSEL_CS DPrim& pr, int k) {
   return k < kInlinePlanes ? pr.pl[k] : S.planes[pr.first_plane + k];
 }
 
-/* Parameter interval of the line p + t d inside a convex primitive. */
+/* Parameter interval of the line p + t d inside a convex primitive (empty
+ * intervals come back with tin > tout).  The primitive is the same on every
+ * active lane, so its kind and plane count branch uniformly; what differs by
+ * lane is selected, not branched on. */
 MD Interval prim_interval(const DevScene& S, const MONSEL_CS DPrim& pr, float px, float py, float pz, float dx, float dy,
                           float dz) {
   Interval iv;
   iv.tin = -kInf;
   iv.tout = kInf;
   iv.fin = iv.fout = -4;
+  bool miss = false;
   if (pr.kind == PRIM_PLANES) {
-    for (int k = 0; k < pr.n_planes; ++k) {
-      float4 pl = prim_plane(S, pr, k);
-      float num = pl.x * px + pl.y * py + pl.z * pz - pl.w;
-      float den = pl.x * dx + pl.y * dy + pl.z * dz;
-      if (den == 0.f) {
-        if (num < 0.f || (num == 0.f && plane_tie_break(pl.x, pl.y, pl.z))) continue;
-        iv.tin = kInf;
-        iv.tout = -kInf;
-        return iv;
-      }
-      float t = -num / den;
-      if (den > 0.f) {
-        if (t < iv.tout) {
-          iv.tout = t;
-          iv.fout = k;
-        }
-      } else if (t > iv.tin) {
-        iv.tin = t;
-        iv.fin = k;
-      }
-    }
-    return iv;
-  }
-  if (pr.kind == PRIM_CYLINDER) {
+    const int tie = pr.tie;
+    auto plane = [&](const float4& pl, int k) {
+      const float num = pl.x * px + pl.y * py + pl.z * pz - pl.w;
+      const float den = pl.x * dx + pl.y * dy + pl.z * dz;
+      const float t = fdiv(-num, den);
+      /* parallel: inside the half space, or outside of it for good */
+      const bool flat = den == 0.f;
+      const bool in = num < 0.f || (num == 0.f && ((tie >> k) & 1));
+      miss = miss || (flat && !in);
+      const bool leaves = den > 0.f && t < iv.tout;
+      const bool enters = !flat && !(den > 0.f) && t > iv.tin;
+      iv.tout = leaves ? t : iv.tout;
+      iv.fout = leaves ? k : iv.fout;
+      iv.tin = enters ? t : iv.tin;
+      iv.fin = enters ? k : iv.fin;
+    };
+    const int n = pr.n_planes;
+#pragma unroll
+    for (int k = 0; k < kInlinePlanes; ++k)
+      if (k < n) plane(pr.pl[k], k);
+    for (int k = kInlinePlanes; k < n; ++k) plane(S.planes[pr.first_plane + k], k);
+  } else if (pr.kind == PRIM_CYLINDER) {
     float wx = px - pr.e0[0], wy = py - pr.e0[1], wz = pz - pr.e0[2];
     float apar = wx * pr.ax[0] + wy * pr.ax[1] + wz * pr.ax[2];
     float dpar = dx * pr.ax[0] + dy * pr.ax[1] + dz * pr.ax[2];
-    float sin_ = -kInf, sout = kInf;
-    int fsin = -4, fsout = -4;
-    if (dpar != 0.f) {
-      float inv = 1.f / dpar;
-      float t0 = -apar * inv, t1 = (pr.len - apar) * inv;
-      if (dpar > 0.f) {
-        sin_ = t0; fsin = -1; sout = t1; fsout = -2;
-      } else {
-        sin_ = t1; fsin = -2; sout = t0; fsout = -1;
-      }
-    } else if (!(apar >= 0.f && apar <= pr.len)) {
-      iv.tin = kInf;
-      iv.tout = -kInf;
-      return iv;
-    }
+    const float inv = __builtin_amdgcn_rcpf(dpar);
+    const float t0 = -apar * inv, t1 = (pr.len - apar) * inv;
+    const bool along = dpar > 0.f, flat = dpar == 0.f;
+    const float sin_ = flat ? -kInf : (along ? t0 : t1), sout = flat ? kInf : (along ? t1 : t0);
+    const int fsin = along ? -1 : -2, fsout = along ? -2 : -1;
+    miss = flat && !(apar >= 0.f && apar <= pr.len);
     /* radial part from the components perpendicular to the axis */
     float qx = wx - apar * pr.ax[0], qy = wy - apar * pr.ax[1], qz = wz - apar * pr.ax[2];
     float vx = dx - dpar * pr.ax[0], vy = dy - dpar * pr.ax[1], vz = dz - dpar * pr.ax[2];
     float A = vx * vx + vy * vy + vz * vz;
     float B = qx * vx + qy * vy + qz * vz;
     float C = qx * qx + qy * qy + qz * qz - pr.r2;
-    float rin = -kInf, rout = kInf;
-    if (A > 1e-12f) {
-      float disc = B * B - A * C;
-      if (disc < 0.f) {
-        iv.tin = kInf;
-        iv.tout = -kInf;
-        return iv;
-      }
-      float sq = fsqrt(disc);
-      float q = -(B + (B >= 0.f ? sq : -sq));
-      float ra = q / A, rb = (q != 0.f) ? C * __builtin_amdgcn_rcpf(q) : ra;
-      rin = fminf(ra, rb);
-      rout = fmaxf(ra, rb);
-    } else if (C > 0.f) {
-      iv.tin = kInf;
-      iv.tout = -kInf;
-      return iv;
-    }
-    if (sin_ >= rin) { iv.tin = sin_; iv.fin = fsin; }
-    else { iv.tin = rin; iv.fin = -3; }
-    if (sout <= rout) { iv.tout = sout; iv.fout = fsout; }
-    else { iv.tout = rout; iv.fout = -3; }
-    return iv;
+    const bool slanted = A > 1e-12f;
+    const float disc = B * B - A * C;
+    miss = miss || (slanted ? disc < 0.f : C > 0.f);
+    const float sq = fsqrt(disc);
+    const float q = -(B + (B >= 0.f ? sq : -sq));
+    const float ra = fdiv(q, A), rb = (q != 0.f) ? C * __builtin_amdgcn_rcpf(q) : ra;
+    const float rin = slanted ? fminf(ra, rb) : -kInf, rout = slanted ? fmaxf(ra, rb) : kInf;
+    const bool cap_in = sin_ >= rin, cap_out = sout <= rout;
+    iv.tin = cap_in ? sin_ : rin;
+    iv.fin = cap_in ? fsin : -3;
+    iv.tout = cap_out ? sout : rout;
+    iv.fout = cap_out ? fsout : -3;
+  } else {
+    float cx = px - pr.e0[0], cy = py - pr.e0[1], cz = pz - pr.e0[2];
+    float B = cx * dx + cy * dy + cz * dz;
+    float C = cx * cx + cy * cy + cz * cz - pr.r2;
+    const float disc = B * B - C;
+    miss = disc < 0.f;
+    const float sq = fsqrt(disc);
+    iv.tin = -B - sq;
+    iv.tout = -B + sq;
+    iv.fin = iv.fout = -3;
   }
-  /* sphere */
-  float cx = px - pr.e0[0], cy = py - pr.e0[1], cz = pz - pr.e0[2];
-  float B = cx * dx + cy * dy + cz * dz;
-  float C = cx * cx + cy * cy + cz * cz - pr.r2;
-  float disc = B * B - C;
-  if (disc < 0.f) {
-    iv.tin = kInf;
-    iv.tout = -kInf;
-    return iv;
-  }
-  float sq = fsqrt(disc);
-  iv.tin = -B - sq;
-  iv.tout = -B + sq;
-  iv.fin = iv.fout = -3;
+  iv.tin = miss ? kInf : iv.tin;
+  iv.tout = miss ? -kInf : iv.tout;
   return iv;
 }
 
@@ -1112,63 +1099,53 @@ MD void prim_normal(const DevScene& S, const MONSEL_CS DPrim& pr, int f, float q
 MD bool prim_contains(const DevScene& S, const MONSEL_CS DPrim& pr, float px, float py, float pz) {
   if (pr.kind == PRIM_PLANES) {
     /* MultiPlaneShape.cu:23-27 for every plane */
-    for (int k = 0; k < pr.n_planes; ++k) {
-      float4 pl = prim_plane(S, pr, k);
-      if (!(pl.x * px + pl.y * py + pl.z * pz - pl.w <= 0.f)) return false;
+    bool in = true;
+    const int n = pr.n_planes;
+#pragma unroll
+    for (int k = 0; k < kInlinePlanes; ++k)
+      if (k < n) in = in && pr.pl[k].x * px + pr.pl[k].y * py + pr.pl[k].z * pz - pr.pl[k].w <= 0.f;
+    for (int k = kInlinePlanes; k < n; ++k) {
+      const float4 pl = S.planes[pr.first_plane + k];
+      in = in && pl.x * px + pl.y * py + pl.z * pz - pl.w <= 0.f;
     }
-    return true;
+    return in;
   }
   float wx = px - pr.e0[0], wy = py - pr.e0[1], wz = pz - pr.e0[2];
   if (pr.kind == PRIM_CYLINDER) {
     /* CylindricalShape.cu:41-45 */
-    float u = (pr.axv[0] * wx + pr.axv[1] * wy + pr.axv[2] * wz) / pr.len2;
+    float u = fdiv(pr.axv[0] * wx + pr.axv[1] * wy + pr.axv[2] * wz, pr.len2);
     float rx = wx - u * pr.axv[0], ry = wy - u * pr.axv[1], rz = wz - u * pr.axv[2];
     return u >= 0.f && u <= 1.f && (rx * rx + ry * ry + rz * rz) <= pr.r2;
   }
   return wx * wx + wy * wy + wz * wz <= pr.r2;
 }
 
+MD bool truth(const MONSEL_CS DShape& sh, uint32_t bits) { return (sh.truth[bits >> 5] >> (bits & 31u)) & 1u; }
+
 /* max_k g_k over a convex primitive's constraints, g_k the signed distance
  * to constraint k (plane rows scaled by sdscale <= 1/|n|): <= 0 inside.
  * Its magnitude bounds the distance from p to the primitive's surface from
  * below -- inside, -max g_k is the distance to the nearest face; outside,
- * max g_k is at most the distance to the primitive. */
-MD float prim_gmax(const DevScene& S, const MONSEL_CS DPrim& pr, float px, float py, float pz) {
-  if (pr.kind == PRIM_PLANES) {
-    float g = -kInf;
-    for (int k = 0; k < pr.n_planes; ++k) {
-      const float4 pl = prim_plane(S, pr, k);
-      g = fmaxf(g, pl.x * px + pl.y * py + pl.z * pz - pl.w);
-    }
-    return g * pr.sdscale;
-  }
-  const float wx = px - pr.e0[0], wy = py - pr.e0[1], wz = pz - pr.e0[2];
-  if (pr.kind == PRIM_CYLINDER) {
-    const float apar = wx * pr.ax[0] + wy * pr.ax[1] + wz * pr.ax[2];
-    const float qx = wx - apar * pr.ax[0], qy = wy - apar * pr.ax[1], qz = wz - apar * pr.ax[2];
-    const float radial = fsqrt(qx * qx + qy * qy + qz * qz) - fsqrt(pr.r2);
-    return fmaxf(radial, fmaxf(-apar, apar - pr.len));
-  }
-  return fsqrt(wx * wx + wy * wy + wz * wz) - fsqrt(pr.r2);
-}
-
-MD bool truth(const MONSEL_CS DShape& sh, uint32_t bits) { return (sh.truth[bits >> 5] >> (bits & 31u)) & 1u; }
-
-/* prim_gmax, and in `in` the primitive's inside bit as prim_contains
- * computes it.  Planes: the same row values.  A sphere or cylinder: the sign
- * of prim_gmax, except within a band of 1e-5 of the magnitudes involved
- * around the surface -- far wider than the few ulps by which the two
- * formulas can round apart -- where prim_contains itself decides. */
+ * max g_k is at most the distance to the primitive.  `in` receives the
+ * primitive's inside bit as prim_contains computes it.  Planes: the same row
+ * values.  A sphere or cylinder: the sign of the result, except within a band
+ * of 1e-5 of the magnitudes involved around the surface -- far wider than the
+ * few ulps by which the two formulas can round apart -- where prim_contains
+ * itself decides. */
 MD float prim_gmax_in(const DevScene& S, const MONSEL_CS DPrim& pr, float px, float py, float pz, bool& in) {
   if (pr.kind == PRIM_PLANES) {
     float g = -kInf;
     bool all = true;
-    for (int k = 0; k < pr.n_planes; ++k) {
-      const float4 pl = prim_plane(S, pr, k);
+    auto row = [&](const float4& pl) {
       const float v = pl.x * px + pl.y * py + pl.z * pz - pl.w;
       g = fmaxf(g, v);
       all = all && v <= 0.f;
-    }
+    };
+    const int n = pr.n_planes;
+#pragma unroll
+    for (int k = 0; k < kInlinePlanes; ++k)
+      if (k < n) row(pr.pl[k]);
+    for (int k = kInlinePlanes; k < n; ++k) row(S.planes[pr.first_plane + k]);
     in = all;
     return g * pr.sdscale;
   }
@@ -1198,6 +1175,9 @@ MD bool shape_contains(const DevScene& S, const MONSEL_CS DShape& sh, float px, 
   return truth(sh, bits);
 }
 
+/* whether some active lane of the wave has p */
+MD bool wave_any(bool p) { return __ballot(p) != 0ull; }
+
 struct ShapeHit {
   float t;      /* kInf if none within tmax */
   float nx, ny, nz;
@@ -1206,10 +1186,12 @@ struct ShapeHit {
 /* First boundary of the composite shape along p + t d, 0 < t <= tmax.
  * Each primitive's entry/exit parameters go to per-lane LDS slots; the walk
  * then visits the crossings in increasing t, toggling the primitives'
- * inside bits, until the truth table changes value.  Requires
- * blockDim.x <= kLaneBlock. */
+ * inside bits, until the truth table changes value.  The first crossing is
+ * found while the intervals are formed, so a segment that ends before it
+ * reads no slot back.  The normal is formed only when asked for.  Requires
+ * blockDim.x <= kLaneBlock and the same shape on every active lane. */
 MD ShapeHit shape_first(const DevScene& S, const MONSEL_CS DShape& sh, float px, float py, float pz, float dx,
-                        float dy, float dz, float tmax) {
+                        float dy, float dz, float tmax, bool want_normal) {
   __shared__ float l_tin[kMaxPrims][kLaneBlock];
   __shared__ float l_tout[kMaxPrims][kLaneBlock];
   __shared__ int8_t l_fin[kMaxPrims][kLaneBlock];
@@ -1218,102 +1200,119 @@ MD ShapeHit shape_first(const DevScene& S, const MONSEL_CS DShape& sh, float px,
   ShapeHit h;
   h.t = kInf;
   h.nx = h.ny = h.nz = 0.f;
-  uint32_t bits = 0;
+  uint32_t bits = 0, mask = 0;
+  float tnext = kInf;
   const int n = sh.n_prims;
-  auto one = [&](int k) {
+  PT_BEGIN(t_iv);
+  for (int k = 0; k < n; ++k) {
     Interval iv = prim_interval(S, S.prims[sh.first_prim + k], px, py, pz, dx, dy, dz);
-    if (!(iv.tin < iv.tout)) {
-      iv.tin = -kInf;
-      iv.tout = -kInf;
-    }
+    const bool empty = !(iv.tin < iv.tout);
+    iv.tin = empty ? -kInf : iv.tin;
+    iv.tout = empty ? -kInf : iv.tout;
     l_tin[k][tid] = iv.tin;
     l_tout[k][tid] = iv.tout;
-    l_fin[k][tid] = (int8_t)iv.fin;
-    l_fout[k][tid] = (int8_t)iv.fout;
-    if (iv.tin <= 0.f && iv.tout > 0.f) bits |= 1u << k;
-  };
-  /* the first four primitives unrolled, so that their records' loads and
-   * interval arithmetic can overlap */
-  PT_BEGIN(t_iv);
-#pragma unroll
-  for (int k = 0; k < 4; ++k)
-    if (k < n) one(k);
-  for (int k = 4; k < n; ++k) one(k);
+    if (want_normal) {
+      l_fin[k][tid] = (int8_t)iv.fin;
+      l_fout[k][tid] = (int8_t)iv.fout;
+    }
+    bits |= iv.tin <= 0.f && iv.tout > 0.f ? 1u << k : 0u;
+    /* the first crossing after 0 and the primitives crossing there */
+    const float nk = iv.tin > 0.f ? iv.tin : (iv.tout > 0.f ? iv.tout : kInf);
+    mask = nk < tnext ? 1u << k : (nk == tnext ? mask | (1u << k) : mask);
+    tnext = fminf(tnext, nk);
+  }
   PT_END(PH_GEOM_IV, t_iv);
   PT_BEGIN(t_wk);
-  bool state = truth(sh, bits);
-  float tcur = 0.f;
-  for (int it = 0; it < 2 * n; ++it) {
-    /* next crossing after tcur and the primitives crossing there */
-    float tnext = kInf;
-    uint32_t mask = 0;
-#pragma unroll
-    for (int k = 0; k < kMaxPrims; ++k) {
-      if (k >= n) break;
-      const float a = l_tin[k][tid], b = l_tout[k][tid];
-      const float nk = a > tcur ? a : (b > tcur ? b : kInf);
-      if (nk < tnext) {
-        tnext = nk;
-        mask = 1u << k;
-      } else if (nk == tnext) {
-        mask |= 1u << k;
+  const bool inside = truth(sh, bits);
+  bool open = tnext <= tmax;
+  for (int it = 0; it < 2 * n && wave_any(open); ++it) {
+    bits ^= open ? mask : 0u;
+    const bool hit = open && truth(sh, bits) != inside;
+    h.t = hit ? tnext : h.t;
+    open = open && !hit;
+    if (wave_any(open)) {
+      /* the next crossing after this one */
+      const float tcur = tnext;
+      float tn = kInf;
+      uint32_t mn = 0;
+      for (int k = 0; k < n; ++k) {
+        const float a = l_tin[k][tid], b = l_tout[k][tid];
+        const float nk = a > tcur ? a : (b > tcur ? b : kInf);
+        mn = nk < tn ? 1u << k : (nk == tn ? mn | (1u << k) : mn);
+        tn = fminf(tn, nk);
       }
+      tnext = open ? tn : tnext;
+      mask = open ? mn : mask;
+      open = open && tnext <= tmax;
     }
-    if (!(tnext <= tmax)) {
-      PT_END(PH_GEOM_WALK, t_wk);
-      return h;
+  }
+  if (want_normal && h.t < kInf) {
+    const float qx = px + tnext * dx, qy = py + tnext * dy, qz = pz + tnext * dz;
+    const int first = __ffs(mask) - 1;
+    const uint32_t rest = mask & (mask - 1u);
+    const int f1 = l_tin[first][tid] == tnext ? l_fin[first][tid] : l_fout[first][tid];
+    float nx, ny, nz;
+    prim_normal(S, S.prims[sh.first_prim + first], f1, qx, qy, qz, nx, ny, nz);
+    if (rest) {
+      /* simultaneous crossings: mean of the two lowest-index normals
+       * (NormalIntersectionShape.cu:229-236) */
+      const int second = __ffs(rest) - 1;
+      const int f2 = l_tin[second][tid] == tnext ? l_fin[second][tid] : l_fout[second][tid];
+      float mx, my, mz;
+      prim_normal(S, S.prims[sh.first_prim + second], f2, qx, qy, qz, mx, my, mz);
+      nx = 0.5f * (nx + mx);
+      ny = 0.5f * (ny + my);
+      nz = 0.5f * (nz + mz);
     }
-    bits ^= mask;
-    const bool ns = truth(sh, bits);
-    if (ns != state) {
-      const float qx = px + tnext * dx, qy = py + tnext * dy, qz = pz + tnext * dz;
-      const int first = __ffs(mask) - 1;
-      const uint32_t rest = mask & (mask - 1u);
-      const int f1 = l_tin[first][tid] == tnext ? l_fin[first][tid] : l_fout[first][tid];
-      float nx, ny, nz;
-      prim_normal(S, S.prims[sh.first_prim + first], f1, qx, qy, qz, nx, ny, nz);
-      if (rest) {
-        /* simultaneous crossings: mean of the two lowest-index normals
-         * (NormalIntersectionShape.cu:229-236) */
-        const int second = __ffs(rest) - 1;
-        const int f2 = l_tin[second][tid] == tnext ? l_fin[second][tid] : l_fout[second][tid];
-        float mx, my, mz;
-        prim_normal(S, S.prims[sh.first_prim + second], f2, qx, qy, qz, mx, my, mz);
-        nx = 0.5f * (nx + mx);
-        ny = 0.5f * (ny + my);
-        nz = 0.5f * (nz + mz);
-      }
-      h.t = tnext;
-      h.nx = nx;
-      h.ny = ny;
-      h.nz = nz;
-      PT_END(PH_GEOM_WALK, t_wk);
-      return h;
-    }
-    state = ns;
-    tcur = tnext;
+    h.nx = nx;
+    h.ny = ny;
+    h.nz = nz;
   }
   PT_END(PH_GEOM_WALK, t_wk);
   return h;
 }
 
-/* RegionBase::containingSubRegion (RegionBase.cu:50-60) from region r. */
-MD int containing_sub_region(const DevScene& S, int r, float px, float py, float pz) {
-  if (!shape_contains(S, S.regions[r].sh, px, py, pz)) return -1;
-  for (int guard = 0; guard < 64; ++guard) {
-    const MONSEL_CS DRegion& rg = S.regions[r];
+/* Runs body(r) once for each value r that `key` has among the lanes with
+ * `on`: r is wave-uniform (the loop runs over a uniform mask), so the scene
+ * records it selects are read with scalar loads; the body runs with those
+ * lanes active. */
+template <class F>
+MD void by_value(bool on, int key, F body) {
+  unsigned long long todo = __ballot(on);
+  while (todo) {
+    const int r0 = __builtin_amdgcn_readlane(key, __ffsll((long long)todo) - 1);
+    const unsigned long long turn = __ballot(key == r0) & todo;
+    if ((turn >> __lane_id()) & 1ull) body(r0);
+    todo &= ~turn;
+  }
+}
+
+/* The region among r (which contains the point) and its descendants that
+ * holds it: the descent of RegionBase::containingSubRegion. */
+MD int descend(const DevScene& S, int r, float px, float py, float pz) {
+  bool open = true;
+  for (int guard = 0; guard < 64 && wave_any(open); ++guard) {
     int next = -1;
-    for (int c = 0; c < rg.n_children; ++c) {
-      int ch = S.children[rg.first_child + c];
-      if (shape_contains(S, S.regions[ch].sh, px, py, pz)) {
-        next = ch;
-        break;
+    by_value(open, r, [&](int r0) {
+      const MONSEL_CS DRegion& rg = S.regions[r0];
+      for (int c = 0; c < rg.n_children; ++c) {
+        const int ch = S.children[rg.first_child + c];
+        const bool in = shape_contains(S, S.regions[ch].sh, px, py, pz);
+        if (next < 0 && in) next = ch;
       }
-    }
-    if (next < 0) return r;
-    r = next;
+    });
+    open = open && next >= 0;
+    r = open ? next : r;
   }
   return r;
+}
+
+/* RegionBase::containingSubRegion (RegionBase.cu:50-60) from region r (which
+ * may differ by lane). */
+MD int containing_sub_region(const DevScene& S, int r, float px, float py, float pz) {
+  bool in = false;
+  by_value(true, r, [&](int r0) { in = shape_contains(S, S.regions[r0].sh, px, py, pz); });
+  return in ? descend(S, r, px, py, pz) : -1;
 }
 
 MD bool is_containing_region(const DevScene& S, int r, int target) {
@@ -1433,7 +1432,7 @@ MD float nudge_nm(float px, float py, float pz) {
 /* RegionBase::findEndOfStep (RegionBase.cu:74-119) on the ray p + t d,
  * 0 < t <= s.  A crossing of the chamber's own boundary leaves the chamber. */
 MD StepEnd find_end_of_step(const DevScene& S, int r, float px, float py, float pz, float dx, float dy, float dz,
-                            float s) {
+                            float s, bool want_normal) {
   StepEnd se;
   const MONSEL_CS DRegion& rg = S.regions[r];
   float t = kInf;
@@ -1443,7 +1442,7 @@ MD StepEnd find_end_of_step(const DevScene& S, int r, float px, float py, float 
    * the nearest crossing found so far */
   for (int c = -1; c < rg.n_children; ++c) {
     const int reg = c < 0 ? r : S.children[rg.first_child + c];
-    ShapeHit h = shape_first(S, S.regions[reg].sh, px, py, pz, dx, dy, dz, c < 0 ? s : fminf(s, t));
+    ShapeHit h = shape_first(S, S.regions[reg].sh, px, py, pz, dx, dy, dz, c < 0 ? s : fminf(s, t), want_normal);
     if (c < 0) {
       se.ownNx = se.winNx = h.nx;
       se.ownNy = se.winNy = h.ny;
@@ -1471,11 +1470,21 @@ MD StepEnd find_end_of_step(const DevScene& S, int r, float px, float py, float 
     float ox = qx + dd * dx, oy = qy + dd * dy, oz = qz + dd * dz;
     int res = -1;
     PT_BEGIN(t_lo);
-    for (int guard = 0; guard < 64 && base >= 0; ++guard) {
-      res = containing_sub_region(S, base, ox, oy, oz);
-      if (res >= 0) break;
-      base = S.regions[base].parent;
+    /* up from the crossed shape's side until a region contains the point */
+    bool up = base >= 0;
+    for (int guard = 0; guard < 64 && wave_any(up); ++guard) {
+      by_value(up, base, [&](int r0) {
+        const MONSEL_CS DRegion& rb = S.regions[r0];
+        if (shape_contains(S, rb.sh, ox, oy, oz)) {
+          res = r0;
+          up = false;
+        } else {
+          base = rb.parent;
+          up = base >= 0;
+        }
+      });
     }
+    if (res >= 0) res = descend(S, res, ox, oy, oz);
     PT_END(PH_GEOM_LOC, t_lo);
     se.next = res;
     return se;
