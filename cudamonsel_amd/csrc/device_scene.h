@@ -93,8 +93,7 @@ struct DCSD {
   } el[kMaxElem];
 };
 
-/* One element of an elastic (SelectableElasticSM) mechanism.  The first
- * eight words are what a cross-section needs, read with one scalar load. */
+/* One element of an elastic (SelectableElasticSM) mechanism. */
 struct DElem {
   float natoms; /* scalefactor * density * N_A, atoms / nm^3 */
   float sfBrowning;
@@ -113,12 +112,30 @@ struct DElem {
   float pad;
 };
 
+/* The elements of an elastic mechanism of at most kFewElem, side by side:
+ * what their cross-sections and angles need, read with a few wide scalar
+ * loads and evaluated without a loop.  Slots beyond the last element have no
+ * atoms. */
+constexpr int kFewElem = 3;
+struct DFewElem {
+  float natoms[4];
+  float sfBrowning[4];
+  float brNum[4], brRoot[4], brInv[4];
+  int spwem[4];  /* offset of the element's cross-section nodes */
+  int x1[4];     /* and of its angle table */
+  float z[4], zp3[4];
+};
+
 struct DMech {
   int kind;
   int elem0;
   int nelem;
   int method;
   int table[4];
+  float extrap; /* elastic: eV, NISTMottRS extrapolateBelowEnergy (its elements share it) */
+  int few;      /* elastic: `el` holds its elements, and their Mott nodes are in LDS */
+  int pad[2];
+  DFewElem el;
   float p[24];
   DCSD csd; /* FittedInelSM's slowing-down algorithm */
   double q[24]; /* tabulated mechanism: the TP_* slots in SI units (J) for the FP64 scatter */

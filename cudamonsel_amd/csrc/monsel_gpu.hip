@@ -202,12 +202,12 @@ __device__ __forceinline__ int* lane_map() {
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
-__device__ __forceinline__ unsigned long long wave_ballot(bool p) { return __ballot(p); }
+__device__ __forceinline__ unsigned long long wave_ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 
 /* this lane's bit of a ballot.  Waterfall loops test membership this way
  * rather than by comparing with the readfirstlane value, which would let the
  * compiler substitute the per-lane value for the uniform one in the body. */
-__device__ __forceinline__ bool lane_in(unsigned long long m) { return (m >> lane_id()) & 1ull; }
+__device__ __forceinline__ bool lane_in(unsigned long long m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
 /* Histogram::bin with edges min + i*delta (Histogram.cu:73-79,
  * Algorithm.cu:5-14); compat = the reference's insertion-point semantics. */
@@ -383,12 +383,12 @@ __device__ __forceinline__ float* lane_rates() {
   return l_rate + threadIdx.x;
 }
 
-/* Per-lane terms sigma_i * atoms_i of the elastic mechanism's rate (the
- * region model's first elastic mechanism), kept between the step's start and
- * its scatter so that the element choice reuses them.  The choice needs all
- * terms but the last, so two slots serve materials of up to 3 elements
- * (larger ones recompute the terms at the scatter). */
-constexpr int kKeptTerms = 2;
+/* Per-lane first two terms sigma_i * atoms_i of the elastic mechanism's rate
+ * (the region model's first elastic mechanism, of at most kFewElem elements),
+ * kept between the step's start and its scatter so that the element choice,
+ * which needs all terms but the last, reuses them (larger materials recompute
+ * the terms at the scatter). */
+constexpr int kKeptTerms = kFewElem - 1;
 __device__ __forceinline__ float* lane_esig() {
   __shared__ float l_esig[kKeptTerms * kLaneBlock];
   return l_esig + threadIdx.x;
@@ -450,13 +450,18 @@ __device__ __forceinline__ void begin_step_in(const DevScene& S, int region, Ele
       float rk;
       if (k == msm.elastic_k) {
         /* elastic_rate, keeping its terms */
-        float* esig = lane_esig();
-        const bool keep = m.nelem <= kKeptTerms + 1;
-        rk = 0.f;
-        elastic_terms(S, m, e.E, [&](int i, float c) {
-          if (keep && i < kKeptTerms) esig[i * kLaneBlock] = c;
-          rk += c;
-        });
+        if (m.few) {
+          float c[kFewElem];
+          elastic_terms_few(S, m, e.E, c);
+          rk = (c[0] + c[1]) + c[2];
+          if (m.nelem > 1) {
+            float* esig = lane_esig();
+            esig[0] = c[0];
+            esig[kLaneBlock] = c[1];
+          }
+        } else {
+          rk = elastic_rate(S, m, e.E);
+        }
       } else {
         rk = mech_rate<TAB>(S, m, e.E);
       }
@@ -608,7 +613,7 @@ __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* j
           sp = mech_scatter<TAB>(
               S, m, e, prevE, rate, trapped, u,
               [&](float* v) { step_uniforms_hi(e, kPhiloxKey0, kPhiloxKey1, v); }, de,
-              k == msm.elastic_k && m.nelem <= kKeptTerms + 1 ? lane_esig() : nullptr);
+              k == msm.elastic_k ? lane_esig() : nullptr);
       }
       if (de.has) deflect(e, de);
       if (sp.has) {
@@ -756,12 +761,20 @@ __device__ __forceinline__ void flush_lane_stats(const GenDev& G, uint32_t job, 
   nsteps = nelec = nesc = nwd = nover = 0;
 }
 
-/* waves per SIMD the register allocation of k_transport targets */
+/* Waves per SIMD the register allocation of k_transport targets.  A wave
+ * issues at most one vector instruction in 5 cycles and one scalar one in 8
+ * here, so the SIMD's throughput comes from its waves.  Without the tabulated
+ * mechanism 5 (96 registers, 56 B of spills): 64 x 64 hole image 106.7 ms, 4:
+ * 117.0 ms, 256 x 256 image 816 and 897 ms; 6 (80 registers, more spills) is
+ * no faster.  The tabulated mechanism's FP64 scatter keeps that kernel at 4. */
+#ifndef MONSEL_TRANSPORT_WAVES_TAB
+#define MONSEL_TRANSPORT_WAVES_TAB 4
+#endif
 #ifndef MONSEL_TRANSPORT_WAVES_PER_EU
-#define MONSEL_TRANSPORT_WAVES_PER_EU 4
+#define MONSEL_TRANSPORT_WAVES_PER_EU 5
 #endif
 template <bool TAB>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MONSEL_TRANSPORT_WAVES_PER_EU)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TAB ? MONSEL_TRANSPORT_WAVES_TAB : MONSEL_TRANSPORT_WAVES_PER_EU)))
 k_transport(DevScene S, GenDev G) {
   Elec e;
   StepStart st;
@@ -1342,7 +1355,7 @@ __global__ void k_probe_elastic(DevScene S, int mech, int element, int n, const 
   else if (el.kind == MONSEL_MECH_RUTHERFORD_ELASTIC || EeV >= kMaxNISTMott)
     ca = rutherford_cos(el.rz23, EeV, r1);
   else
-    ca = mott_cos(S, el.mott, EeV, r1);
+    ca = mott_cos(S, el.mott * (kMottNE * kMottNQ), EeV, r1);
   out[i] = acosf(fminf(1.f, fmaxf(-1.f, ca)));
 }
 
@@ -1676,10 +1689,37 @@ DCSD make_csd(const monsel_material_desc& m, double breakE) {
     c.el[i].beta = (float)beta[i];
     c.el[i].coef = (float)(coef[i] * 1e-9 / (kE * kE));
   }
+  for (int i = c.nce; i < MONSEL_MAX_ELEMENTS; ++i) c.el[i].beta = 1.f;
   c.breakE = (float)(breakE / kE);
   c.gamma15 = 1.5f * (float)(gamma * 1e-9 * pow(kE, 1.5));
   c.minE = (float)(bh / kE);
   return c;
+}
+
+/* DMech::el of an elastic mechanism whose elements are in place; merging
+ * scenes, which moves the Mott tables, fills it again. */
+void fill_few(const HostScene& H, DMech& dm) {
+  memset(&dm.el, 0, sizeof(dm.el));
+  dm.few = dm.nelem >= 1 && dm.nelem <= kFewElem;
+  for (int i = 0; dm.few && i < dm.nelem; ++i) {
+    const DElem& el = H.elems[dm.elem0 + i];
+    if (el.mott >= kLdsMott) {
+      dm.few = 0;
+      break;
+    }
+    dm.el.natoms[i] = el.natoms;
+    dm.el.sfBrowning[i] = el.sfBrowning;
+    dm.el.brNum[i] = el.brNum;
+    dm.el.brRoot[i] = el.brRoot;
+    dm.el.brInv[i] = el.brInv;
+    dm.el.spwem[i] = std::max(el.mott, 0) * kMottNE;
+    dm.el.x1[i] = std::max(el.mott, 0) * kMottNE * kMottNQ;
+    dm.el.z[i] = el.z;
+    dm.el.zp3[i] = el.zp3;
+  }
+  /* slots beyond the last element: no atoms, and denominators that stay
+   * finite */
+  for (int i = std::max(dm.nelem, 0); i < 4; ++i) dm.el.brRoot[i] = dm.el.z[i] = 1.f;
 }
 
 /* collect the convex leaves of a CSG tree (deduplicated by shape index) */
@@ -1830,7 +1870,9 @@ HostScene compile_scene(const monsel_scene_desc* d) {
               el.sfBrowning = (float)(sig / brown);
             }
             H.elems.push_back(el);
+            dm.extrap = el.extrap;
           }
+          fill_few(H, dm);
           break;
         }
         case MONSEL_MECH_FITTED_INELASTIC: {
@@ -2139,16 +2181,17 @@ HostScene merge_scenes(const std::vector<const HostScene*>& parts, std::vector<i
       m.mech0 += o_me;
       M.msms.push_back(m);
     }
+    for (DElem el : P->elems) {
+      if (el.mott >= 0) el.mott += o_mott;
+      M.elems.push_back(el);
+    }
     for (DMech m : P->mechs) {
       m.elem0 += o_el;
+      if (m.kind <= MONSEL_MECH_RUTHERFORD_ELASTIC) fill_few(M, m);
       if (m.kind == MONSEL_MECH_TABULATED_INELASTIC)
         for (int q = 0; q < 4; ++q)
           if (m.table[q] >= 0) m.table[q] += o_nu;
       M.mechs.push_back(m);
-    }
-    for (DElem el : P->elems) {
-      if (el.mott >= 0) el.mott += o_mott;
-      M.elems.push_back(el);
     }
     M.spwem.insert(M.spwem.end(), P->spwem.begin(), P->spwem.end());
     M.x1.insert(M.x1.end(), P->x1.begin(), P->x1.end());
@@ -2288,7 +2331,7 @@ struct monsel_ctx_s {
   std::vector<std::shared_ptr<SceneDev>> batch_parts;
   std::vector<int> batch_roots;
   hipEvent_t ev0 = nullptr, ev1 = nullptr, evk0 = nullptr, evk1 = nullptr;
-  int blocks_per_cu = 0;
+  int blocks_per_cu[2] = {0, 0}; /* persistent blocks of k_transport<false> and <true> */
 };
 
 namespace {
@@ -2639,7 +2682,7 @@ void run_generation(monsel_ctx_s* C) {
   G.geo_batch = geometry_batch_for(C->tuning.geometry_batch, C->batch.step_prims, nprim + C->in_count);
   G.handoff = C->tuning.spawn_handoff >= 0 ? 1 : 0;
   const int block = C->tuning.block_size > 0 ? C->tuning.block_size : 256;
-  const int grid = C->n_cu * (C->blocks_per_cu > 0 ? C->blocks_per_cu : 4);
+  const int grid = C->n_cu * C->blocks_per_cu[C->batch.dev.has_tabulated ? 1 : 0];
   spread_launch(G, C->tuning, nprim + C->in_count, (uint64_t)grid * (block / 64));
   /* Event markers time the kernels; MONSEL_NO_EVENT_TIMING=1 leaves them out
    * (hardware-counter profiling sessions reject the marker packets). */
@@ -2928,13 +2971,11 @@ int monsel_create(int device_ordinal, const monsel_tuning* tuning, monsel_ctx* o
     int block = C->tuning.block_size > 0 ? C->tuning.block_size : 256;
     if (block % 64 != 0 || block > kLaneBlock)
       throw MonselError(MONSEL_E_INVALID, "block_size must be a multiple of 64, <= 256");
-    if (C->tuning.blocks_per_cu > 0) C->blocks_per_cu = C->tuning.blocks_per_cu;
-    else {
-      int occ_t = 0, occ_f = 0;
-      HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_t, k_transport<true>, block, 0));
-      HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_f, k_transport<false>, block, 0));
-      const int occ = std::min(occ_t, occ_f);
-      C->blocks_per_cu = occ > 0 ? occ : 1;
+    for (int tab = 0; tab < 2; ++tab) {
+      int occ = 0;
+      if (tab) HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_transport<true>, block, 0));
+      else HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_transport<false>, block, 0));
+      C->blocks_per_cu[tab] = C->tuning.blocks_per_cu > 0 ? C->tuning.blocks_per_cu : std::max(occ, 1);
     }
     monsel_ctx_s* raw = C.get();
     raw->worker = std::thread(worker_main, raw);
@@ -3304,7 +3345,7 @@ int monsel_run_static(monsel_ctx ctx, monsel_scene_id scene, const monsel_job_de
     const int maxGen = T.max_generations > 0 ? T.max_generations : 100000;
     const uint64_t perLaunch = primaries_per_launch_for(T.primaries_per_launch, cap);
     const int block = T.block_size > 0 ? T.block_size : 256;
-    const int grid = ctx->n_cu * (ctx->blocks_per_cu > 0 ? ctx->blocks_per_cu : 4);
+    const int grid = ctx->n_cu * ctx->blocks_per_cu[sd->dev.has_tabulated ? 1 : 0];
     uint64_t launched = 0, reserved = 0;
     uint32_t in_count = 0;
     int cur = 0, generations = 0;

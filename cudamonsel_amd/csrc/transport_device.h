@@ -50,6 +50,12 @@ MD float fsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 MD float flog(float x) { return __builtin_amdgcn_logf(x) * 0.693147180559945309f; }
 MD float fexp(float x) { return __builtin_amdgcn_exp2f(x * 1.442695040888963407f); }
 
+/* a product that is not contracted into a following sum */
+MD float fmul(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+
 /* a / b as a times the hardware reciprocal: what the compiler's own division
  * gives for |b| <= 2^96 (beyond it rescales b around the reciprocal's flush
  * to zero: four more instructions for denominators no transport quantity
@@ -188,17 +194,8 @@ MD void dir_from_angles(float ct, float st, float cph, float sph, float& dx, flo
   dz = ct;
 }
 
-/* Lagrange cubic through unit-spaced nodes 0..3 evaluated at t (the value
- * Neville's scheme in ULagrangeInterpolation.cu:5-33 produces). */
-MD float lagrange4(float t, float f0, float f1, float f2, float f3) {
-  float t1 = t - 1.f, t2 = t - 2.f, t3 = t - 3.f;
-  float l0 = -t1 * t2 * t3 * (1.f / 6.f);
-  float l1 = t * t2 * t3 * 0.5f;
-  float l2 = -t * t1 * t3 * 0.5f;
-  float l3 = t * t1 * t2 * (1.f / 6.f);
-  return l0 * f0 + l1 * f1 + l2 * f2 + l3 * f3;
-}
-
+/* Weights at t of the Lagrange cubic through unit-spaced nodes 0..3 (which
+ * Neville's scheme in ULagrangeInterpolation.cu:5-33 evaluates). */
 MD void lagrange4_w(float t, float& l0, float& l1, float& l2, float& l3) {
   float t1 = t - 1.f, t2 = t - 2.f, t3 = t - 3.f;
   l0 = -t1 * t2 * t3 * (1.f / 6.f);
@@ -218,9 +215,9 @@ MD int u_index0(float reduced, int len) {
 
 /* BrowningEmpiricalCrossSection.cu:24-29 (nm^2); e in keV, re its root and
  * inv_re the root's reciprocal */
-MD float browning_sigma(const MONSEL_CS DElem& el, float e, float re, float inv_re) {
+MD float browning_sigma(float num, float root, float inv, float e, float re, float inv_re) {
 #pragma clang fp contract(off)
-  return el.brNum * __builtin_amdgcn_rcpf(__builtin_fmaf(re, el.brRoot, e) + el.brInv * inv_re);
+  return num * __builtin_amdgcn_rcpf(__builtin_fmaf(re, root, e) + inv * inv_re);
 }
 
 /* BrowningEmpiricalCrossSection.cu:31-45 -> cos(theta) */
@@ -283,6 +280,9 @@ MD MottWindow mott_window(float EeV) {
   lagrange4_w(red - (float)w.i0, w.l0, w.l1, w.l2, w.l3);
   return w;
 }
+MD float mott_sigma(const MottWindow& w, float f0, float f1, float f2, float f3) {
+  return kA0nm2 * __builtin_fmaf(w.l3, f3, __builtin_fmaf(w.l2, f2, __builtin_fmaf(w.l1, f1, w.l0 * f0)));
+}
 MD float mott_table_sigma(const DevScene& S, int mott, const MottWindow& w) {
   float f0, f1, f2, f3;
   if (mott < kLdsMott) {
@@ -298,7 +298,58 @@ MD float mott_table_sigma(const DevScene& S, int mott, const MottWindow& w) {
     f2 = f[2];
     f3 = f[3];
   }
-  return kA0nm2 * (w.l0 * f0 + w.l1 * f1 + w.l2 * f2 + w.l3 * f3);
+  return mott_sigma(w, f0, f1, f2, f3);
+}
+
+/* The terms sigma_i * atoms_i of an elastic mechanism of at most kFewElem
+ * elements (m.few) at energy EeV: c[i], 0 beyond the last element.  The same
+ * arithmetic as elastic_terms, without its loops: one wave-uniform branch on
+ * the element count, one on the energy. */
+MD void elastic_terms_few(const DevScene& S, const MONSEL_CS DMech& m, float EeV, float* c) {
+#pragma clang fp contract(off)
+  const bool mott = m.kind == MONSEL_MECH_NISTMOTT_ELASTIC;
+  const bool one = m.nelem == 1;
+  const MONSEL_CS DFewElem& el = m.el;
+  c[0] = c[1] = c[2] = 0.f;
+  if (m.kind == MONSEL_MECH_BROWNING_ELASTIC || (mott && EeV < m.extrap)) {
+    if (mott && m.method == 3) {
+#pragma unroll
+      for (int i = 0; i < kFewElem; ++i)
+        if (i < m.nelem) {
+          const MONSEL_CS DElem& q = S.elems[m.elem0 + i];
+          c[i] = fdiv(q.mottAtMin * EeV, q.extrap) * q.natoms;
+        }
+    } else {
+      const float e = EeV * 1.0e-3f;
+      const float re = fsqrt(e);
+      const float inv_re = __builtin_amdgcn_rcpf(re);
+      auto term = [&](int i) {
+        const float b = browning_sigma(el.brNum[i], el.brRoot[i], el.brInv[i], e, re, inv_re);
+        c[i] = fmul(mott ? fmul(el.sfBrowning[i], b) : b, el.natoms[i]);
+      };
+      term(0);
+      if (!one) {
+        term(1);
+        term(2);
+      }
+    }
+  } else if (mott && EeV < kMaxNISTMott) {
+    const MottWindow w = mott_window(EeV);
+    const float* f = lds_spwem() + w.i0;
+    auto term = [&](int i) {
+      const float* q = f + el.spwem[i];
+      c[i] = fmul(mott_sigma(w, q[0], q[1], q[2], q[3]), el.natoms[i]);
+    };
+    term(0);
+    if (!one) {
+      term(1);
+      term(2);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < kFewElem; ++i)
+      if (i < m.nelem) c[i] = rutherford_sigma(S.elems[m.elem0 + i], EeV) * S.elems[m.elem0 + i].natoms;
+  }
 }
 
 /* The terms sigma_i * atoms_i of an elastic mechanism at energy EeV, given in
@@ -321,7 +372,7 @@ MD void elastic_terms(const DevScene& S, const MONSEL_CS DMech& m, float EeV, F 
       const float re = fsqrt(e);
       const float inv_re = __builtin_amdgcn_rcpf(re);
       for (int i = 0; i < n; ++i) {
-        const float b = browning_sigma(el[i], e, re, inv_re);
+        const float b = browning_sigma(el[i].brNum, el[i].brRoot, el[i].brInv, e, re, inv_re);
         f(i, (mott ? el[i].sfBrowning * b : b) * el[i].natoms);
       }
     }
@@ -334,9 +385,10 @@ MD void elastic_terms(const DevScene& S, const MONSEL_CS DMech& m, float EeV, F 
 }
 
 /* NISTMottRS::randomScatteringAngle table branch: bicubic Lagrange on X1
- * over (ln E, U) (NISTMottRS.cu:134-150, ULagrangeInterpolation.cu:55-78);
+ * over (ln E, U) (NISTMottRS.cu:134-150, ULagrangeInterpolation.cu:55-78) at
+ * offset x1 of the tables;
  * returns cos(theta) clamped as the reference does. */
-MD float mott_cos(const DevScene& S, int mott, float EeV, float u) {
+MD float mott_cos(const DevScene& S, int x1, float EeV, float u) {
   float rx = (flog(EeV) - kMottLn50) * kMottInvParam;
   int i0 = u_index0(rx, kMottNE);
   float ry = u * 200.0f;
@@ -344,14 +396,14 @@ MD float mott_cos(const DevScene& S, int mott, float EeV, float u) {
   float wx0, wx1, wx2, wx3, wy0, wy1, wy2, wy3;
   lagrange4_w(rx - (float)i0, wx0, wx1, wx2, wx3);
   lagrange4_w(ry - (float)j0, wy0, wy1, wy2, wy3);
-  const float* base = S.mott_x1 + (size_t)mott * (kMottNE * kMottNQ) + i0 * kMottNQ + j0;
+  const float* base = S.mott_x1 + (uint32_t)(x1 + i0 * kMottNQ + j0);
   float q = 0.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const float* row = base + i * kMottNQ;
-    float v = wy0 * row[0] + wy1 * row[1] + wy2 * row[2] + wy3 * row[3];
-    float wx = i == 0 ? wx0 : (i == 1 ? wx1 : (i == 2 ? wx2 : wx3));
-    q += wx * v;
+    const float v = __builtin_fmaf(wy3, row[3], __builtin_fmaf(wy2, row[2], __builtin_fmaf(wy0, row[0], wy1 * row[1])));
+    const float wx = i == 0 ? wx0 : (i == 1 ? wx1 : (i == 2 ? wx2 : wx3));
+    q = __builtin_fmaf(wx, v, q);
   }
   float com = 1.0f - 2.0f * q * q;
   return com > -1.0f ? (com < 1.0f ? com : 1.0f) : -1.0f;
@@ -371,7 +423,14 @@ MD float nieminen_factor(float eps) {
 /* sum over the elements of coef ln(E / J + beta) */
 MD float joy_luo_sum(const MONSEL_CS DCSD& c, float kE) {
   float s = 0.f;
-  for (int i = 0; i < c.nce; ++i) s += c.el[i].coef * flog(c.el[i].recipJ * kE + c.el[i].beta);
+  auto term = [&](int i) { s += c.el[i].coef * flog(c.el[i].recipJ * kE + c.el[i].beta); };
+  term(0);
+  if (c.nce > 1) {
+    /* slots beyond the last element add 0 */
+    term(1);
+    term(2);
+    for (int i = 3; i < c.nce; ++i) term(i);
+  }
   return s;
 }
 
@@ -614,7 +673,13 @@ MD double nu_interp(const DevScene& S, int table, int order, const double* x, bo
 
 MD float elastic_rate(const DevScene& S, const MONSEL_CS DMech& m, float EeV) {
   float tot = 0.f;
-  elastic_terms(S, m, EeV, [&](int, float c) { tot += c; });
+  if (m.few) {
+    float c[kFewElem];
+    elastic_terms_few(S, m, EeV, c);
+    tot = (c[0] + c[1]) + c[2];
+  } else {
+    elastic_terms(S, m, EeV, [&](int, float c) { tot += c; });
+  }
   return tot;
 }
 
@@ -829,6 +894,17 @@ MD Spawn tabulated_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e,
   return se;
 }
 
+/* The pick-th of three wave-uniform values.  They are held in scalar
+ * registers first: left to itself the compiler selects among their addresses
+ * and loads per lane. */
+template <class T>
+MD T of_three(int pick, T a, T b, T c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("" : "+s"(a), "+s"(b), "+s"(c));
+#endif
+  return pick == 0 ? a : (pick == 1 ? b : c);
+}
+
 /* A deflection of the electron's direction left for the end of the scatter:
  * polar angle by its cosine, azimuth by its uniform. */
 struct Deflect {
@@ -848,7 +924,8 @@ MD void deflect(Elec& e, const Deflect& d) {
 /* ScatterMechanism::scatter of mechanism m (the same one on every active
  * lane).  `rate` is this mechanism's scatterRate at prevE, as summed when the
  * step's free path was drawn; esig, if given, holds the elastic mechanism's
- * first nelem - 1 terms (lane stride kLaneBlock); draw_hi(u) draws u[4..7].
+ * first two terms if it has no more than kFewElem elements (lane stride
+ * kLaneBlock); draw_hi(u) draws u[4..7].
  * A deflection of the primary is left in `de` for the caller, which applies
  * it once for every mechanism.  TAB = false leaves the tabulated mechanism
  * out of the code (its FP64 scatter sets the register budget of every kernel
@@ -865,45 +942,53 @@ MD Spawn mech_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e, floa
       PT_BEGIN(t_el);
       /* first element whose running sum of sigma * atoms reaches u * rate
        * (the last if none does); the sum is re-formed in the order
-       * elastic_rate formed it.  The elements pass by wave-uniformly, and a
-       * lane keeps the angle parameters of its choice. */
+       * elastic_rate formed it */
       const float r = u[2] * rate;
-      const MONSEL_CS DElem* el = S.elems + m.elem0;
       const bool nist = m.kind == MONSEL_MECH_NISTMOTT_ELASTIC;
-      const float extrap = el[0].extrap;
-      int mott = el[0].mott;
-      float z = el[0].z, zp3 = el[0].zp3, rz23 = el[0].rz23;
-      float cum = 0.f;
-      bool open = true;
-      auto term = [&](int i, float c) {
-        if (i < m.nelem - 1) {
-          cum += c;
-          open = open && cum < r;
-          if (open) {
-            mott = el[i + 1].mott;
-            z = el[i + 1].z;
-            zp3 = el[i + 1].zp3;
-            rz23 = el[i + 1].rz23;
+      int pick = 0;
+      if (m.few) {
+        if (m.nelem > 1) {
+          float c[kFewElem];
+          if (esig) {
+            c[0] = esig[0];
+            c[1] = esig[kLaneBlock];
+          } else {
+            elastic_terms_few(S, m, prevE, c);
           }
+          const bool past0 = c[0] < r, past1 = past0 & (m.nelem > 2) & (c[0] + c[1] < r);
+          pick = past1 ? 2 : (past0 ? 1 : 0);
         }
-      };
-      if (esig) {
-        for (int i = 0; i < m.nelem - 1; ++i) term(i, esig[i * kLaneBlock]);
       } else {
-        elastic_terms(S, m, prevE, term);
+        float cum = 0.f;
+        elastic_terms(S, m, prevE, [&](int i, float c) {
+          if (i < m.nelem - 1) {
+            cum += c;
+            if (pick == i && cum < r) pick = i + 1;
+          }
+        });
       }
       draw_hi(u);
       /* the polar angle takes one uniform (two for Browning), the azimuth
        * the next one (SelectableElasticSM.cu:62-64) */
       de.has = true;
       de.u_azimuth = u[4];
-      if (m.kind == MONSEL_MECH_BROWNING_ELASTIC || (nist && prevE < extrap)) {
+      if (m.kind == MONSEL_MECH_BROWNING_ELASTIC || (nist && prevE < m.extrap)) {
+        float z, zp3;
+        if (m.few) {
+          z = of_three(pick, m.el.z[0], m.el.z[1], m.el.z[2]);
+          zp3 = of_three(pick, m.el.zp3[0], m.el.zp3[1], m.el.zp3[2]);
+        } else {
+          z = S.elems[m.elem0 + pick].z;
+          zp3 = S.elems[m.elem0 + pick].zp3;
+        }
         de.cos_polar = browning_cos(z, zp3, prevE, u[3], u[4]);
         de.u_azimuth = u[5];
       } else if (nist && !(prevE >= kMaxNISTMott)) {
-        de.cos_polar = mott_cos(S, mott, prevE, u[3]);
+        const int x1 = m.few ? of_three(pick, m.el.x1[0], m.el.x1[1], m.el.x1[2])
+                             : S.elems[m.elem0 + pick].mott * (kMottNE * kMottNQ);
+        de.cos_polar = mott_cos(S, x1, prevE, u[3]);
       } else {
-        de.cos_polar = rutherford_cos(rz23, prevE, u[3]);
+        de.cos_polar = rutherford_cos(S.elems[m.elem0 + pick].rz23, prevE, u[3]);
       }
       PT_END(PH_ELASTIC, t_el);
       return se;
@@ -1007,10 +1092,10 @@ MD Interval prim_interval(const DevScene& S, const MONSEL_CS DPrim& pr, float px
       const float t = fdiv(-num, den);
       /* parallel: inside the half space, or outside of it for good */
       const bool flat = den == 0.f;
-      const bool in = num < 0.f || (num == 0.f && ((tie >> k) & 1));
-      miss = miss || (flat && !in);
-      const bool leaves = den > 0.f && t < iv.tout;
-      const bool enters = !flat && !(den > 0.f) && t > iv.tin;
+      const bool in = (num < 0.f) | ((num == 0.f) & (((tie >> k) & 1) != 0));
+      miss = miss | (flat & !in);
+      const bool leaves = (den > 0.f) & (t < iv.tout);
+      const bool enters = !flat & !(den > 0.f) & (t > iv.tin);
       iv.tout = leaves ? t : iv.tout;
       iv.fout = leaves ? k : iv.fout;
       iv.tin = enters ? t : iv.tin;
@@ -1030,7 +1115,7 @@ MD Interval prim_interval(const DevScene& S, const MONSEL_CS DPrim& pr, float px
     const bool along = dpar > 0.f, flat = dpar == 0.f;
     const float sin_ = flat ? -kInf : (along ? t0 : t1), sout = flat ? kInf : (along ? t1 : t0);
     const int fsin = along ? -1 : -2, fsout = along ? -2 : -1;
-    miss = flat && !(apar >= 0.f && apar <= pr.len);
+    miss = flat & !((apar >= 0.f) & (apar <= pr.len));
     /* radial part from the components perpendicular to the axis */
     float qx = wx - apar * pr.ax[0], qy = wy - apar * pr.ax[1], qz = wz - apar * pr.ax[2];
     float vx = dx - dpar * pr.ax[0], vy = dy - dpar * pr.ax[1], vz = dz - dpar * pr.ax[2];
@@ -1039,7 +1124,7 @@ MD Interval prim_interval(const DevScene& S, const MONSEL_CS DPrim& pr, float px
     float C = qx * qx + qy * qy + qz * qz - pr.r2;
     const bool slanted = A > 1e-12f;
     const float disc = B * B - A * C;
-    miss = miss || (slanted ? disc < 0.f : C > 0.f);
+    miss = miss | (slanted ? disc < 0.f : C > 0.f);
     const float sq = fsqrt(disc);
     const float q = -(B + (B >= 0.f ? sq : -sq));
     const float ra = fdiv(q, A), rb = (q != 0.f) ? C * __builtin_amdgcn_rcpf(q) : ra;
@@ -1103,10 +1188,10 @@ MD bool prim_contains(const DevScene& S, const MONSEL_CS DPrim& pr, float px, fl
     const int n = pr.n_planes;
 #pragma unroll
     for (int k = 0; k < kInlinePlanes; ++k)
-      if (k < n) in = in && pr.pl[k].x * px + pr.pl[k].y * py + pr.pl[k].z * pz - pr.pl[k].w <= 0.f;
+      if (k < n) in = in & (pr.pl[k].x * px + pr.pl[k].y * py + pr.pl[k].z * pz - pr.pl[k].w <= 0.f);
     for (int k = kInlinePlanes; k < n; ++k) {
       const float4 pl = S.planes[pr.first_plane + k];
-      in = in && pl.x * px + pl.y * py + pl.z * pz - pl.w <= 0.f;
+      in = in & (pl.x * px + pl.y * py + pl.z * pz - pl.w <= 0.f);
     }
     return in;
   }
@@ -1115,7 +1200,7 @@ MD bool prim_contains(const DevScene& S, const MONSEL_CS DPrim& pr, float px, fl
     /* CylindricalShape.cu:41-45 */
     float u = fdiv(pr.axv[0] * wx + pr.axv[1] * wy + pr.axv[2] * wz, pr.len2);
     float rx = wx - u * pr.axv[0], ry = wy - u * pr.axv[1], rz = wz - u * pr.axv[2];
-    return u >= 0.f && u <= 1.f && (rx * rx + ry * ry + rz * rz) <= pr.r2;
+    return (u >= 0.f) & (u <= 1.f) & ((rx * rx + ry * ry + rz * rz) <= pr.r2);
   }
   return wx * wx + wy * wy + wz * wz <= pr.r2;
 }
@@ -1139,7 +1224,7 @@ MD float prim_gmax_in(const DevScene& S, const MONSEL_CS DPrim& pr, float px, fl
     auto row = [&](const float4& pl) {
       const float v = pl.x * px + pl.y * py + pl.z * pz - pl.w;
       g = fmaxf(g, v);
-      all = all && v <= 0.f;
+      all = all & (v <= 0.f);
     };
     const int n = pr.n_planes;
 #pragma unroll
@@ -1176,90 +1261,76 @@ MD bool shape_contains(const DevScene& S, const MONSEL_CS DShape& sh, float px, 
 }
 
 /* whether some active lane of the wave has p */
-MD bool wave_any(bool p) { return __ballot(p) != 0ull; }
+MD bool wave_any(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0ull; }
 
 struct ShapeHit {
   float t;      /* kInf if none within tmax */
   float nx, ny, nz;
 };
 
-/* First boundary of the composite shape along p + t d, 0 < t <= tmax.
- * Each primitive's entry/exit parameters go to per-lane LDS slots; the walk
- * then visits the crossings in increasing t, toggling the primitives'
- * inside bits, until the truth table changes value.  The first crossing is
- * found while the intervals are formed, so a segment that ends before it
- * reads no slot back.  The normal is formed only when asked for.  Requires
- * blockDim.x <= kLaneBlock and the same shape on every active lane. */
+/* First boundary of the composite shape along p + t d, 0 < t <= tmax: the
+ * walk visits the primitives' crossings in increasing t, toggling their
+ * inside bits, until the truth table changes value.  Each pass over the
+ * primitives forms their intervals and finds the next crossing after tcur;
+ * a segment that ends before the first one, or crosses the boundary there,
+ * takes one pass.  Forming the intervals again for a later crossing keeps
+ * them out of LDS (20 KB per block of 256 lanes), which held the kernel to 4
+ * waves per SIMD.  The normal is formed only when asked for.  Requires the
+ * same shape on every active lane. */
 MD ShapeHit shape_first(const DevScene& S, const MONSEL_CS DShape& sh, float px, float py, float pz, float dx,
                         float dy, float dz, float tmax, bool want_normal) {
-  __shared__ float l_tin[kMaxPrims][kLaneBlock];
-  __shared__ float l_tout[kMaxPrims][kLaneBlock];
-  __shared__ int8_t l_fin[kMaxPrims][kLaneBlock];
-  __shared__ int8_t l_fout[kMaxPrims][kLaneBlock];
-  const int tid = threadIdx.x;
   ShapeHit h;
   h.t = kInf;
   h.nx = h.ny = h.nz = 0.f;
-  uint32_t bits = 0, mask = 0;
-  float tnext = kInf;
   const int n = sh.n_prims;
+  const MONSEL_CS DPrim* prims = S.prims + sh.first_prim;
+  uint32_t bits = 0;
+  float tcur = 0.f;
+  bool inside = false, open = true;
+  /* primitive and face of the lowest two indices crossing at the hit */
+  int k1 = 0, f1 = 0, k2 = -1, f2 = 0;
   PT_BEGIN(t_iv);
-  for (int k = 0; k < n; ++k) {
-    Interval iv = prim_interval(S, S.prims[sh.first_prim + k], px, py, pz, dx, dy, dz);
-    const bool empty = !(iv.tin < iv.tout);
-    iv.tin = empty ? -kInf : iv.tin;
-    iv.tout = empty ? -kInf : iv.tout;
-    l_tin[k][tid] = iv.tin;
-    l_tout[k][tid] = iv.tout;
-    if (want_normal) {
-      l_fin[k][tid] = (int8_t)iv.fin;
-      l_fout[k][tid] = (int8_t)iv.fout;
+  for (int it = 0; it < 2 * n; ++it) {
+    uint32_t mask = 0;
+    float tnext = kInf;
+    for (int k = 0; k < n; ++k) {
+      const Interval iv = prim_interval(S, prims[k], px, py, pz, dx, dy, dz);
+      const bool empty = !(iv.tin < iv.tout);
+      const float a = empty ? -kInf : iv.tin, b = empty ? -kInf : iv.tout;
+      if (it == 0) bits |= (a <= 0.f) & (b > 0.f) ? 1u << k : 0u;
+      const bool at_in = a > tcur;
+      const float nk = at_in ? a : (b > tcur ? b : kInf);
+      const bool nearer = nk < tnext, same = nk == tnext;
+      if (want_normal && open) {
+        const int f = at_in ? iv.fin : iv.fout;
+        k2 = nearer ? -1 : (same & (k2 < 0) ? k : k2);
+        f2 = k2 == k ? f : f2;
+        k1 = nearer ? k : k1;
+        f1 = nearer ? f : f1;
+      }
+      mask = nearer ? 1u << k : (same ? mask | (1u << k) : mask);
+      tnext = nearer ? nk : tnext;
     }
-    bits |= iv.tin <= 0.f && iv.tout > 0.f ? 1u << k : 0u;
-    /* the first crossing after 0 and the primitives crossing there */
-    const float nk = iv.tin > 0.f ? iv.tin : (iv.tout > 0.f ? iv.tout : kInf);
-    mask = nk < tnext ? 1u << k : (nk == tnext ? mask | (1u << k) : mask);
-    tnext = fminf(tnext, nk);
+    if (it == 0) inside = truth(sh, bits);
+    open = open & (tnext <= tmax);
+    bits ^= open ? mask : 0u;
+    const bool hit = open & (truth(sh, bits) != inside);
+    h.t = hit ? tnext : h.t;
+    open = open & !hit;
+    tcur = tnext;
+    if (!wave_any(open)) break;
   }
   PT_END(PH_GEOM_IV, t_iv);
   PT_BEGIN(t_wk);
-  const bool inside = truth(sh, bits);
-  bool open = tnext <= tmax;
-  for (int it = 0; it < 2 * n && wave_any(open); ++it) {
-    bits ^= open ? mask : 0u;
-    const bool hit = open && truth(sh, bits) != inside;
-    h.t = hit ? tnext : h.t;
-    open = open && !hit;
-    if (wave_any(open)) {
-      /* the next crossing after this one */
-      const float tcur = tnext;
-      float tn = kInf;
-      uint32_t mn = 0;
-      for (int k = 0; k < n; ++k) {
-        const float a = l_tin[k][tid], b = l_tout[k][tid];
-        const float nk = a > tcur ? a : (b > tcur ? b : kInf);
-        mn = nk < tn ? 1u << k : (nk == tn ? mn | (1u << k) : mn);
-        tn = fminf(tn, nk);
-      }
-      tnext = open ? tn : tnext;
-      mask = open ? mn : mask;
-      open = open && tnext <= tmax;
-    }
-  }
   if (want_normal && h.t < kInf) {
-    const float qx = px + tnext * dx, qy = py + tnext * dy, qz = pz + tnext * dz;
-    const int first = __ffs(mask) - 1;
-    const uint32_t rest = mask & (mask - 1u);
-    const int f1 = l_tin[first][tid] == tnext ? l_fin[first][tid] : l_fout[first][tid];
+    const float qx = px + h.t * dx, qy = py + h.t * dy, qz = pz + h.t * dz;
     float nx, ny, nz;
-    prim_normal(S, S.prims[sh.first_prim + first], f1, qx, qy, qz, nx, ny, nz);
-    if (rest) {
+    prim_normal(S, prims[k1], f1, qx, qy, qz, nx, ny, nz);
+    if (k2 >= 0) {
       /* simultaneous crossings: mean of the two lowest-index normals
        * (NormalIntersectionShape.cu:229-236) */
-      const int second = __ffs(rest) - 1;
-      const int f2 = l_tin[second][tid] == tnext ? l_fin[second][tid] : l_fout[second][tid];
       float mx, my, mz;
-      prim_normal(S, S.prims[sh.first_prim + second], f2, qx, qy, qz, mx, my, mz);
+      prim_normal(S, prims[k2], f2, qx, qy, qz, mx, my, mz);
       nx = 0.5f * (nx + mx);
       ny = 0.5f * (ny + my);
       nz = 0.5f * (nz + mz);
@@ -1278,11 +1349,11 @@ MD ShapeHit shape_first(const DevScene& S, const MONSEL_CS DShape& sh, float px,
  * lanes active. */
 template <class F>
 MD void by_value(bool on, int key, F body) {
-  unsigned long long todo = __ballot(on);
+  unsigned long long todo = __builtin_amdgcn_ballot_w64(on);
   while (todo) {
     const int r0 = __builtin_amdgcn_readlane(key, __ffsll((long long)todo) - 1);
-    const unsigned long long turn = __ballot(key == r0) & todo;
-    if ((turn >> __lane_id()) & 1ull) body(r0);
+    const unsigned long long turn = __builtin_amdgcn_ballot_w64(key == r0) & todo;
+    if (__builtin_amdgcn_inverse_ballot_w64(turn)) body(r0);
     todo &= ~turn;
   }
 }
@@ -1348,6 +1419,12 @@ MD uint32_t xor_permute(uint32_t T, uint32_t B, int n) {
  * nearest primitive surface. */
 MD float shape_safety(const DevScene& S, const MONSEL_CS DShape& sh, float px, float py, float pz, bool& inside) {
   const int n = sh.n_prims;
+  if (n == 1) {
+    bool in;
+    const float d = fabsf(prim_gmax_in(S, S.prims[sh.first_prim], px, py, pz, in));
+    inside = truth(sh, in ? 1u : 0u);
+    return truth(sh, 0u) != truth(sh, 1u) ? d : kInf;
+  }
   if (n > kMaxCstPrims) {
     float d = kInf;
     uint32_t bits = 0;

@@ -69,6 +69,25 @@ def test_results_independent_of_tuning(M, tuning):
             _same(a, b)
 
 
+def test_many_mott_tables_in_one_batch(M):
+    """A batch of seven line scenes holds 28 Mott tables, more than the 16 kept
+    in LDS: the jobs on the later scenes take their cross-sections from device
+    memory, element by element, and match the same jobs alone, whose elements
+    are evaluated side by side from LDS."""
+    from cudamonsel_amd import scenes
+    from cudamonsel_amd.abi import Engine
+    scs = [scenes.line_on_substrate(w_nm=18.0 + k) for k in range(7)]
+    cs = [sc.monte.compileScene() for sc in scs]
+    cen = scenes.scan_centers(np.linspace(-15, 15, 4), [0.0], scs[0].beam_z)
+    with Engine() as eng:
+        sids = [eng.upload(c) for c in cs]
+        alone = [eng.result(eng.submit(s, cen, 300, 600.0, 0.5e-9, 40 + k)) for k, s in enumerate(sids)]
+        ids = [eng.submit(s, cen, 300, 600.0, 0.5e-9, 40 + k) for k, s in enumerate(sids)]
+        mixed = [eng.result(i) for i in ids]
+    for a, b in zip(alone, mixed):
+        _same(a, b)
+
+
 @pytest.mark.parametrize("primaries", [1, 63, 4095, 4096, 4097, 8193, 65535, 65536])
 def test_spread_launches_keep_results(M, primaries):
     """A launch of fewer than 65,536 items gives each wave an equal share of
