@@ -417,10 +417,10 @@ __device__ __forceinline__ float from_anchor(float x, float y, float z) {
 
 /* What the start of a step leaves for its end. */
 struct StepStart {
-  float freePath;
+  uint32_t path; /* the free path's bits; the sign bit: the step may reach a
+                  * boundary, findEndOfStep must run */
   float total;   /* summed mechanism rates (0 in a null material) */
   float u1, u2, u3;
-  bool geo;      /* the step may reach a boundary: findEndOfStep must run */
 };
 
 /* MonteCarloSS::takeStep (MonteCarloSS.cu:107-163), first half: the
@@ -476,14 +476,14 @@ __device__ __forceinline__ void begin_step_in(const DevScene& S, int region, Ele
       freePath = maxFreePath;
     }
   }
-  st.freePath = freePath;
   st.total = total;
   st.u1 = u[1];
   st.u2 = u[2];
   st.u3 = u[3];
   const float margin = nudge_nm(e.px, e.py, e.pz);
   const float current = e.safe > 0.f ? e.safe - from_anchor(e.px, e.py, e.pz) : 0.f;  /* bound here */
-  st.geo = !(freePath + margin <= current);
+  const bool near_surface = !(freePath + margin <= current);
+  st.path = (__float_as_uint(freePath) & 0x7FFFFFFFu) | (near_surface ? 0x80000000u : 0u);
   PT_END(PH_RATES, t_ra);
 }
 
@@ -520,161 +520,171 @@ __device__ __forceinline__ bool locate(const DevScene& S, const JobRec* jobs, El
 template <bool TAB>
 __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* jobs, const int region, Elec& e,
                                               Spawn& sp, int maxSteps, const StepStart& st) {
-  sp.has = false;
-  const MONSEL_CS DMSM& msm = S.msms[S.regions[region].msm];
+  const MONSEL_CS DRegion& rg = S.regions[region];
+  const MONSEL_CS DMSM& msm = S.msms[rg.msm];
   /* the reference's barrier ignores the surface normal in compat mode */
   const bool normals = (S.compat & MONSEL_COMPAT_BARRIER_NORMAL) == 0u;
-  const float freePath = st.freePath;
+  const bool geo = (int)st.path < 0;
+  const float freePath = __uint_as_float(st.path & 0x7FFFFFFFu);
   const float px = e.px, py = e.py, pz = e.pz;
   StepEnd se;
-  if (st.geo) {
-    PT_BEGIN(t_ge);
-    se = find_end_of_step(S, region, px, py, pz, e.dx, e.dy, e.dz, freePath, normals);
-    PT_END(PH_GEOM, t_ge);
-  } else {
-    se.t = freePath;
-    se.next = region;
-    se.boundary = false;
-    se.winner = -1;
-  }
-  float len = se.t;
-  e.px = px + len * e.dx;
-  e.py = py + len * e.dy;
-  e.pz = pz + len * e.dz;
-  /* the safety bound: a geometry step's is its end point's; a step within
-   * the bound keeps the anchored one.  Where findEndOfStep found no boundary
-   * for some lane, the wave computes the end point's bound; the pass costs
-   * the wave the same whichever lanes take part, so every lane of it that
-   * crossed no boundary refreshes its bound (and keeps the better one). */
-  if (st.geo || se.boundary) e.safe = 0.f;
-  if (!msm.is_null && wave_ballot(st.geo && !se.boundary) != 0ull && !se.boundary) {
-    PT_BEGIN(t_sf);
-    const float fresh = region_safety(S, region, e.px, e.py, e.pz);
-    const float kept = e.safe > 0.f ? e.safe - from_anchor(e.px, e.py, e.pz) : 0.f;
-    if (fresh > kept) {
-      e.safe = fresh;
-      set_anchor(e.px, e.py, e.pz);
+  se.t = freePath;
+  se.next = region;
+  se.winner = -1;
+  const bool any_geo = wave_any(geo);
+  if (any_geo) {
+    bool boundary = false;
+    if (geo) {
+      PT_BEGIN(t_ge);
+      se = find_end_of_step(S, region, px, py, pz, e.dx, e.dy, e.dz, freePath, normals);
+      boundary = se.boundary;
+      e.safe = 0.f;
+      PT_END(PH_GEOM, t_ge);
     }
-    PT_END(PH_SAFETY, t_sf);
+    e.px = px + se.t * e.dx;
+    e.py = py + se.t * e.dy;
+    e.pz = pz + se.t * e.dz;
+    /* the safety bound: a geometry step's is its end point's; a step within
+     * the bound keeps the anchored one.  Where findEndOfStep found no boundary
+     * for some lane, the wave computes the end point's bound; the pass costs
+     * the wave the same whichever lanes take part, so every lane of it that
+     * crossed no boundary refreshes its bound (and keeps the better one). */
+    if (!msm.is_null && wave_any(geo & !boundary) && !boundary) {
+      PT_BEGIN(t_sf);
+      const float fresh = region_safety(S, region, e.px, e.py, e.pz);
+      const float kept = e.safe > 0.f ? e.safe - from_anchor(e.px, e.py, e.pz) : 0.f;
+      if (fresh > kept) {
+        e.safe = fresh;
+        set_anchor(e.px, e.py, e.pz);
+      }
+      PT_END(PH_SAFETY, t_sf);
+    }
+    if (boundary & (se.next == region)) {
+      /* a grazing crossing: the point a nudge beyond the boundary is back in
+       * this region (a corner clipped within the nudge, or FP32 rounding
+       * between the crossing walk and the containment test).  The step still
+       * ends there as in RegionBase::findEndOfStep, but the electron is carried
+       * past the feature so that the next step cannot stop at it again. */
+      const float dd = nudge_nm(e.px, e.py, e.pz);
+      e.px += dd * e.dx;
+      e.py += dd * e.dy;
+      e.pz += dd * e.dz;
+    }
+  } else {
+    e.px = px + freePath * e.dx;
+    e.py = py + freePath * e.dy;
+    e.pz = pz + freePath * e.dz;
   }
-  if (se.boundary && se.next == region) {
-    /* a grazing crossing: the point a nudge beyond the boundary is back in
-     * this region (a corner clipped within the nudge, or FP32 rounding
-     * between the crossing walk and the containment test).  The step still
-     * ends there as in RegionBase::findEndOfStep, but the electron is carried
-     * past the feature so that the next step cannot stop at it again. */
-    const float dd = nudge_nm(e.px, e.py, e.pz);
-    e.px += dd * e.dx;
-    e.py += dd * e.dy;
-    e.pz += dd * e.dz;
-  }
-  float prevE = e.E;
+  const float prevE = e.E;
   PT_BEGIN(t_cs);
-  if (!msm.is_null) e.E += csd_compute(msm.csd, len, e.E);
+  if (!msm.is_null) e.E += csd_compute(msm.csd, se.t, e.E);
   PT_END(PH_CSD, t_cs);
   e.steps++;
-  if ((int)e.steps > maxSteps || !(e.E == e.E)) return STEP_WATCHDOG;
-  if (e.E < msm.minE) return STEP_DEAD;
-  if (se.next == region) {
-    /* MONSEL_MaterialScatterModel::scatter (:93-134), rates at prevE */
-    if (!msm.is_null && st.total != 0.f) {
-      PT_BEGIN(t_se);
-      const float* rates = lane_rates();
-      const float r = st.u1 * st.total;
-      /* first mechanism whose cumulative rate reaches r (MONSEL_MaterialScatterModel.cu:129-131);
-       * the running sum repeats the order of `total` */
-      int idx = 0;
-      float rate = rates[0];
-      float cum = rate;
-      for (int k = 1; k < msm.n_mech; ++k) {
-        const float rk = rates[k * kLaneBlock];
-        if (idx == k - 1 && cum < r) {
-          idx = k;
-          rate = rk;
-          cum += rk;
-        }
-      }
-      bool trapped = false;
-      float u[kStepUniforms];
-      u[0] = 0.f;
-      u[1] = st.u1;
-      u[2] = st.u2;
-      u[3] = st.u3;
-      PT_END(PH_SELECT, t_se);
-      /* the mechanisms in turn, each for the lanes that chose it: its record
-       * is wave-uniform */
-      Deflect de;
-      de.has = false;
-      for (int k = 0; k < msm.n_mech; ++k) {
-        const unsigned long long turn = wave_ballot(idx == k);
-        if (!turn) continue;
-        const MONSEL_CS DMech& m = S.mechs[msm.mech0 + k];
-        if (lane_in(turn))
-          sp = mech_scatter<TAB>(
-              S, m, e, prevE, rate, trapped, u,
-              [&](float* v) { step_uniforms_hi(e, kPhiloxKey0, kPhiloxKey1, v); }, de,
-              k == msm.elastic_k ? lane_esig() : nullptr);
-      }
-      if (de.has) deflect(e, de);
-      if (sp.has) {
-        /* trackSecondaryElectron (MonteCarloSS.cu:165-174) */
-        if (!(sp.E > msm.minE)) sp.has = false;
-      }
-      if (trapped || e.E < msm.minE) return STEP_DEAD;
-    }
-    if (st.geo && !(e.safe > nudge_nm(e.px, e.py, e.pz)) && !locate(S, jobs, e, region)) return STEP_DEAD;
-    return STEP_CONTINUE;
-  }
-  if (se.next >= 0) {
-    /* ExpQMBarrierSM::barrierScatter (ExpQMBarrierSM.cu:50-219) */
-    PT_BEGIN(t_ba);
-    int next = se.next;
-    if (msm.is_null || msm.barrier_kind == MONSEL_BARRIER_NONE) {
-      e.region = next;
-    } else {
-      /* ExpQMBarrierSM.cu:77-96: outward normal of the struck shape, negated
-       * when entering a child region (unused in compat mode) */
-      by_value(true, next, [&](int to) {
-        float nbx = 0.f, nby = 0.f, nbz = 0.f;
-        if (normals) {
-          if (is_containing_region(S, region, to)) {
-            int struck = to;
-            while (S.regions[struck].parent != region) struck = S.regions[struck].parent;
-            if (struck == se.winner) {
-              nbx = -se.winNx; nby = -se.winNy; nbz = -se.winNz;
+  int res = STEP_CONTINUE;
+  if (e.E < msm.minE) res = STEP_DEAD;
+  if (((int)e.steps > maxSteps) | !(e.E == e.E)) res = STEP_WATCHDOG;
+  const bool crossed = se.next != region;
+  uint32_t check = 0u;   /* the containment check that opens the next step is due */
+  if (any_geo) {
+    check = geo & (res == STEP_CONTINUE) ? 1u : 0u;
+    if (check && !crossed) {
+      /* the electron may have left its region only within a nudge of a surface */
+      check = !(e.safe > nudge_nm(e.px, e.py, e.pz)) ? 1u : 0u;
+    } else if (check && se.next >= 0) {
+      /* ExpQMBarrierSM::barrierScatter (ExpQMBarrierSM.cu:50-219) */
+      PT_BEGIN(t_ba);
+      const int next = se.next;
+      if (msm.is_null || msm.barrier_kind == MONSEL_BARRIER_NONE) {
+        e.region = next;
+      } else {
+        /* ExpQMBarrierSM.cu:77-96: outward normal of the struck shape, negated
+         * when entering a child region (unused in compat mode) */
+        by_value(true, next, [&](int to) {
+          float nbx = 0.f, nby = 0.f, nbz = 0.f;
+          if (normals) {
+            if (is_containing_region(S, region, to)) {
+              int struck = to;
+              while (S.regions[struck].parent != region) struck = S.regions[struck].parent;
+              if (struck == se.winner) {
+                nbx = -se.winNx; nby = -se.winNy; nbz = -se.winNz;
+              } else {
+                ShapeHit h = shape_first(S, S.regions[struck].sh, px, py, pz, e.dx, e.dy, e.dz, freePath, true);
+                nbx = -h.nx; nby = -h.ny; nbz = -h.nz;
+              }
             } else {
-              ShapeHit h = shape_first(S, S.regions[struck].sh, px, py, pz, e.dx, e.dy, e.dz, freePath, true);
-              nbx = -h.nx; nby = -h.ny; nbz = -h.nz;
+              nbx = se.ownNx; nby = se.ownNy; nbz = se.ownNz;
             }
-          } else {
-            nbx = se.ownNx; nby = se.ownNy; nbz = se.ownNz;
           }
-        }
-        barrier_core(S, msm, S.msms[S.regions[to].msm], e, to, nbx, nby, nbz, st.u1);
-      });
+          barrier_core(S, msm, S.msms[S.regions[to].msm], e, to, nbx, nby, nbz, st.u1);
+        });
+      }
+      /* MonteCarloSS.cu:146-148: nudge along the new direction; the region is
+       * re-located by the check that opens the next step */
+      const float dd = nudge_nm(e.px, e.py, e.pz);
+      e.px += dd * e.dx;
+      e.py += dd * e.dy;
+      e.pz += dd * e.dz;
+      PT_END(PH_BARRIER, t_ba);
+    } else if (check) {
+      /* left the chamber: BackscatterEvent.  The escape is recorded for
+       * k_tally_escapes: through the chamber wall the tally point is recomputed
+       * in FP64 from the step's start, so that start replaces the position and
+       * e.region carries the flag. */
+      check = 0u;
+      const bool fromRoot = (rg.parent < 0) & (se.winner < 0);
+      e.px = fromRoot ? px : e.px;
+      e.py = fromRoot ? py : e.py;
+      e.pz = fromRoot ? pz : e.pz;
+      e.region = fromRoot ? 1 : 0;
+      res = STEP_ESCAPED;
     }
-    /* MonteCarloSS.cu:146-148: nudge along the new direction; the region is
-     * re-located by the check that opens the next step */
-    float dd = nudge_nm(e.px, e.py, e.pz);
-    e.px += dd * e.dx;
-    e.py += dd * e.dy;
-    e.pz += dd * e.dz;
-    PT_END(PH_BARRIER, t_ba);
-    if (!locate(S, jobs, e, e.region)) return STEP_DEAD;
-    return STEP_CONTINUE;
   }
-  /* left the chamber: BackscatterEvent.  The escape is recorded for
-   * k_tally_escapes: through the chamber wall the tally point is recomputed
-   * in FP64 from the step's start, so that start replaces the position and
-   * e.region carries the flag. */
-  const bool fromRoot = S.regions[region].parent < 0 && se.winner < 0;
-  if (fromRoot) {
-    e.px = px;
-    e.py = py;
-    e.pz = pz;
+  if ((res == STEP_CONTINUE) & !crossed & (st.total != 0.f)) {
+    /* MONSEL_MaterialScatterModel::scatter (:93-134), rates at prevE (their
+     * sum is 0 in a null material) */
+    PT_BEGIN(t_se);
+    const float* rates = lane_rates();
+    const float r = st.u1 * st.total;
+    /* first mechanism whose cumulative rate reaches r (MONSEL_MaterialScatterModel.cu:129-131);
+     * the running sum repeats the order of `total` */
+    int idx = 0;
+    float rate = rates[0];
+    float cum = rate;
+    for (int k = 1; k < msm.n_mech; ++k) {
+      const float rk = rates[k * kLaneBlock];
+      const bool past = (idx == k - 1) & (cum < r);
+      idx = past ? k : idx;
+      rate = past ? rk : rate;
+      cum = past ? cum + rk : cum;
+    }
+    bool trapped = false;
+    float u[kStepUniforms];
+    u[0] = 0.f;
+    u[1] = st.u1;
+    u[2] = st.u2;
+    u[3] = st.u3;
+    PT_END(PH_SELECT, t_se);
+    /* the mechanisms in turn, each for the lanes that chose it: its record
+     * is wave-uniform */
+    Deflect de;
+    de.has = 0u;
+    for (int k = 0; k < msm.n_mech; ++k) {
+      const unsigned long long turn = wave_ballot(idx == k);
+      if (!turn) continue;
+      const MONSEL_CS DMech& m = S.mechs[msm.mech0 + k];
+      if (lane_in(turn))
+        sp = mech_scatter<TAB>(
+            S, m, e, prevE, rate, trapped, u,
+            [&](float* v) { step_uniforms_hi(e, kPhiloxKey0, kPhiloxKey1, v); }, de,
+            k == msm.elastic_k ? lane_esig() : nullptr);
+    }
+    if (de.has) deflect(e, de);
+    /* trackSecondaryElectron (MonteCarloSS.cu:165-174) */
+    sp.has = sp.has && sp.E > msm.minE ? 1u : 0u;
+    if (trapped | (e.E < msm.minE)) res = STEP_DEAD;
   }
-  e.region = fromRoot ? 1 : 0;
-  return STEP_ESCAPED;
+  if (check && res == STEP_CONTINUE && !locate(S, jobs, e, e.region)) res = STEP_DEAD;
+  return res;
 }
 
 /* finish_step_in by region, as begin_step */
@@ -715,50 +725,84 @@ __device__ __forceinline__ void make_primary(const DevScene& S, const JobRec& J,
   e.region = containing_sub_region(S, J.root, e.px, e.py, e.pz);
 }
 
-/* Appends electrons to the next launch's queue: one atomic per wave. */
-__device__ __forceinline__ void queue_append(const GenDev& G, bool has, float px, float py, float pz, float dx, float dy,
-                                             float dz, float E, int region, uint32_t primary, uint32_t lin_lo,
-                                             uint32_t lin_hi, uint32_t job, uint32_t steps, uint32_t nchild,
-                                             unsigned long long lanemask_lt, uint32_t& nover) {
-  const unsigned long long m = wave_ballot(has);
+/* a pointer known to address global memory (one read from a record would
+ * otherwise compile to flat accesses) */
+template <class T>
+__device__ __forceinline__ T* in_global(T* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (T*)(__attribute__((address_space(1))) T*)p;
+#else
+  return p;
+#endif
+}
+
+/* Appends the electrons of the lanes in m to the next launch's queue: one
+ * atomic per wave. */
+__device__ __forceinline__ void queue_append(const MONSEL_CS GenDev& G, unsigned long long m, float px, float py,
+                                             float pz, float dx, float dy, float dz, float E, int region,
+                                             uint32_t primary, uint32_t lin_lo, uint32_t lin_hi, uint32_t job,
+                                             uint32_t steps, uint32_t nchild, unsigned long long lanemask_lt,
+                                             uint32_t& nover) {
   if (!m) return;
   const int leader = __ffsll((long long)m) - 1;
   uint32_t base = 0;
-  if (lane_id() == leader) base = atomicAdd(G.out_count, (unsigned int)__popcll(m));
-  base = __shfl(base, leader);
-  if (!has) return;
+  if (lane_id() == leader) base = atomicAdd(in_global(G.out_count), (unsigned int)__popcll(m));
+  base = __builtin_amdgcn_readlane(base, leader);
+  if (!lane_in(m)) return;
   const uint32_t slot = base + (uint32_t)__popcll(m & lanemask_lt);
-  if (slot >= G.out_cap) {
+  const uint32_t cap = G.out_cap;
+  if (slot >= cap) {
     nover++;
     return;
   }
-  const uint32_t cap = G.out_cap;
-  G.out_f[0 * cap + slot] = px;
-  G.out_f[1 * cap + slot] = py;
-  G.out_f[2 * cap + slot] = pz;
-  G.out_f[3 * cap + slot] = dx;
-  G.out_f[4 * cap + slot] = dy;
-  G.out_f[5 * cap + slot] = dz;
-  G.out_f[6 * cap + slot] = E;
-  G.out_u[0 * cap + slot] = (uint32_t)region;
-  G.out_u[1 * cap + slot] = primary;
-  G.out_u[2 * cap + slot] = lin_lo;
-  G.out_u[3 * cap + slot] = lin_hi;
-  G.out_u[4 * cap + slot] = job;
-  G.out_u[5 * cap + slot] = steps;
-  G.out_u[6 * cap + slot] = nchild;
+  float* f = in_global(G.out_f) + slot;
+  uint32_t* q = in_global(G.out_u) + slot;
+  const size_t c = cap;
+  f[0] = px;
+  f[c] = py;
+  f[2 * c] = pz;
+  f[3 * c] = dx;
+  f[4 * c] = dy;
+  f[5 * c] = dz;
+  f[6 * c] = E;
+  q[0] = (uint32_t)region;
+  q[c] = primary;
+  q[2 * c] = lin_lo;
+  q[3 * c] = lin_hi;
+  q[4 * c] = job;
+  q[5 * c] = steps;
+  q[6 * c] = nchild;
 }
 
 /* adds one lane's counters to its job's statistics (per-lane atomics) */
-__device__ __forceinline__ void flush_lane_stats(const GenDev& G, uint32_t job, uint32_t& nsteps, uint32_t& nelec,
+__device__ __forceinline__ void flush_lane_stats(const JobRec* jobs, uint32_t job, uint32_t& nsteps, uint32_t& nelec,
                                                  uint32_t& nesc, uint32_t& nwd, uint32_t& nover) {
-  unsigned long long* st = stat_stripe(G.jobs[job].stats);
+  unsigned long long* st = stat_stripe(jobs[job].stats);
   if (nsteps) atomicAdd(&st[kStatSteps], (unsigned long long)nsteps);
   if (nelec) atomicAdd(&st[kStatElectrons], (unsigned long long)nelec);
   if (nesc) atomicAdd(&st[kStatEscapes], (unsigned long long)nesc);
   if (nwd) atomicAdd(&st[kStatWatchdog], (unsigned long long)nwd);
   if (nover) atomicAdd(&st[kStatOverflow], (unsigned long long)nover);
   nsteps = nelec = nesc = nwd = nover = 0;
+}
+
+struct TransportArgs {
+  DevScene S;
+  GenDev G;
+};
+
+/* The transport kernel's arguments where they are used: read from the
+ * kernel-argument segment on the spot.  Taken as plain arguments, the launch
+ * record's two dozen fields are loaded at the kernel's start and held for its
+ * whole length, for the most part spilled to vector-register lanes. */
+__device__ __forceinline__ const MONSEL_CS TransportArgs* launch_args() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const MONSEL_CS TransportArgs* a = (const MONSEL_CS TransportArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  return a;
+#else
+  return nullptr;
+#endif
 }
 
 /* Waves per SIMD the register allocation of k_transport targets.  A wave
@@ -775,18 +819,24 @@ __device__ __forceinline__ void flush_lane_stats(const GenDev& G, uint32_t job, 
 #endif
 template <bool TAB>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TAB ? MONSEL_TRANSPORT_WAVES_TAB : MONSEL_TRANSPORT_WAVES_PER_EU)))
-k_transport(DevScene S, GenDev G) {
+k_transport(TransportArgs args) {
+  const DevScene& S = args.S;
   Elec e;
   StepStart st;
-  bool alive = false, pending = false;
+  /* Wave-uniform lane masks: the lanes with an electron, and those of them
+   * whose step has begun.  As masks they need no merging where lanes diverge. */
+  unsigned long long alive = 0ull, pending = 0ull;
   bool done = false;                   /* wave-uniform: the launch's items are all claimed */
   uint32_t r_base = 0, r_left = 0;     /* wave-uniform reserve of claimed item indices */
   int maxSteps = 0;
   uint32_t steps0 = 0;                 /* step count when the lane took the electron */
   uint32_t cur_job = 0xFFFFFFFFu;      /* job the lane's counters belong to */
   uint32_t nsteps = 0, nelec = 0, nesc = 0, nwd = 0, nover = 0;
-  const uint32_t n_items = G.n_prim + G.in_n;
   const unsigned long long lanemask_lt = (1ull << lane_id()) - 1ull;
+  const int geo_batch = args.G.geo_batch, lane_cap = args.G.lane_cap, claim_min = args.G.claim_min;
+  const int tail_lanes = args.G.tail_lanes, regroup = args.G.steps_per_launch;
+  const JobRec* jobs = args.G.jobs;
+  st.path = 0u;
   stage_mott_sigma(S);
   PT_INIT();
   for (;;) {
@@ -794,20 +844,22 @@ k_transport(DevScene S, GenDev G) {
     /* claim work for idle lanes (once kClaimMin of them wait, or no lane
      * steps): from the wave's reserve of claimed items, topped up a chunk
      * at a time by one atomic per wave */
-    unsigned long long m = done ? 0ull : wave_ballot(!alive);
-    const int room = __popcll(m) - (64 - G.lane_cap);   /* lane_cap less the live lanes */
-    if (~m != 0ull && room < G.claim_min) m = 0ull;
+    unsigned long long m = done ? 0ull : ~alive;
+    const int room = __popcll(m) - (64 - lane_cap);   /* lane_cap less the live lanes */
+    if (alive != 0ull && room < claim_min) m = 0ull;
     if (m) {
+      const MONSEL_CS GenDev& G = launch_args()->G;
+      const uint32_t n_prim = G.n_prim, n_items = n_prim + G.in_n;
       /* the first `room` idle lanes take an item each */
-      const bool need = !alive && __popcll(m & lanemask_lt) < room;
+      const bool need = lane_in(m) && __popcll(m & lanemask_lt) < room;
       m = wave_ballot(need);
       const uint32_t cnt = (uint32_t)__popcll(m);
       uint32_t fresh = 0, want = 0;
       if (cnt > r_left) {
         want = max(cnt - r_left, (uint32_t)G.claim_chunk);
         const int leader = __ffsll((long long)m) - 1;
-        if (lane_id() == leader) fresh = atomicAdd(G.claim, want);
-        fresh = __shfl(fresh, leader);
+        if (lane_id() == leader) fresh = atomicAdd(in_global(G.claim), want);
+        fresh = __builtin_amdgcn_readlane(fresh, leader);
       }
       const uint32_t rank = (uint32_t)__popcll(m & lanemask_lt);
       const uint32_t idx = rank < r_left ? r_base + rank : fresh + (rank - r_left);
@@ -818,58 +870,61 @@ k_transport(DevScene S, GenDev G) {
         r_base += cnt;
         r_left -= cnt;
       }
-      if (need) {
-        if (idx < n_items) {
-          if (idx < G.n_prim) {
-            /* segment holding item idx (binary search over the running ends) */
-            int lo = 0, hi = G.n_seg - 1;
-            while (lo < hi) {
-              const int mid = (lo + hi) >> 1;
-              if (G.seg_end[mid] > idx) hi = mid;
-              else lo = mid + 1;
-            }
-            const uint32_t start = lo > 0 ? G.seg_end[lo - 1] : 0u;
-            const uint32_t job = G.seg_job[lo];
-            make_primary(S, G.jobs[job], job, G.seg_first[lo] + (idx - start), e);
-          } else {
-            const uint32_t q = idx - G.n_prim;
-            const uint32_t cap = G.in_cap;
-            e.px = G.in_f[0 * cap + q];
-            e.py = G.in_f[1 * cap + q];
-            e.pz = G.in_f[2 * cap + q];
-            e.dx = G.in_f[3 * cap + q];
-            e.dy = G.in_f[4 * cap + q];
-            e.dz = G.in_f[5 * cap + q];
-            e.E = G.in_f[6 * cap + q];
-            e.region = (int)G.in_u[0 * cap + q];
-            e.primary = G.in_u[1 * cap + q];
-            e.lin_lo = G.in_u[2 * cap + q];
-            e.lin_hi = G.in_u[3 * cap + q];
-            e.job = G.in_u[4 * cap + q];
-            e.steps = G.in_u[5 * cap + q];
-            e.nchild = G.in_u[6 * cap + q];
-            e.safe = 0.f;
+      uint32_t took = 0u;
+      if (need && idx < n_items) {
+        if (idx < n_prim) {
+          /* segment holding item idx (binary search over the running ends) */
+          const uint32_t* seg_end = in_global(G.seg_end);
+          int lo = 0, hi = G.n_seg - 1;
+          while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (seg_end[mid] > idx) hi = mid;
+            else lo = mid + 1;
           }
-          if (e.job != cur_job) {
-            if (cur_job != 0xFFFFFFFFu) flush_lane_stats(G, cur_job, nsteps, nelec, nesc, nwd, nover);
-            cur_job = e.job;
-          }
-          const JobRec& J = G.jobs[e.job];
-          if (J.killed) {
-            nover++;
-          } else {
-            maxSteps = J.max_steps;
-            steps0 = e.steps;
-            /* a queued electron is located again (the check opening its next step) */
-            alive = idx < G.n_prim ? e.region >= 0 : locate(S, G.jobs, e, e.region);
-          }
+          const uint32_t start = lo > 0 ? seg_end[lo - 1] : 0u;
+          const uint32_t job = in_global(G.seg_job)[lo];
+          make_primary(S, jobs[job], job, in_global(G.seg_first)[lo] + (idx - start), e);
+        } else {
+          const uint32_t q = idx - n_prim;
+          const size_t cap = G.in_cap;
+          const float* f = in_global(G.in_f) + q;
+          const uint32_t* u = in_global(G.in_u) + q;
+          e.px = f[0];
+          e.py = f[cap];
+          e.pz = f[2 * cap];
+          e.dx = f[3 * cap];
+          e.dy = f[4 * cap];
+          e.dz = f[5 * cap];
+          e.E = f[6 * cap];
+          e.region = (int)u[0];
+          e.primary = u[cap];
+          e.lin_lo = u[2 * cap];
+          e.lin_hi = u[3 * cap];
+          e.job = u[4 * cap];
+          e.steps = u[5 * cap];
+          e.nchild = u[6 * cap];
+          e.safe = 0.f;
+        }
+        if (e.job != cur_job) {
+          if (cur_job != 0xFFFFFFFFu) flush_lane_stats(jobs, cur_job, nsteps, nelec, nesc, nwd, nover);
+          cur_job = e.job;
+        }
+        const JobRec& J = jobs[e.job];
+        if (J.killed) {
+          nover++;
+        } else {
+          maxSteps = J.max_steps;
+          steps0 = e.steps;
+          /* a queued electron is located again (the check opening its next step) */
+          took = (idx < n_prim ? e.region >= 0 : locate(S, jobs, e, e.region)) ? 1u : 0u;
         }
       }
+      alive |= wave_ballot(took != 0u);
       /* items are handed out in order: one beyond the last means none are left */
       done = wave_ballot(need && idx >= n_items) != 0ull;
     }
     PT_END(PH_CLAIM, t_cl);
-    if (wave_ballot(alive) == 0ull) {
+    if (alive == 0ull) {
       /* the wave leaves only once it has run past the launch's items: a claim
        * round can hand out nothing but dead electrons (queued ones of a job
        * the host stopped, or primaries that start outside the chamber), and
@@ -880,120 +935,123 @@ k_transport(DevScene S, GenDev G) {
     /* start a step on every lane without one in progress; a step that may
      * reach a boundary waits for the wave's next findEndOfStep pass, which
      * runs once geo_batch lanes wait or no lane could move without it */
-    if (alive && !pending) {
-      begin_step<TAB>(S, e, st);
-      pending = true;
-    }
-    const unsigned long long m_geo = wave_ballot(alive && st.geo);
-    const unsigned long long m_free = wave_ballot(alive && !st.geo);
-    const bool run_geo = m_free == 0ull || __popcll(m_geo) >= G.geo_batch;
+    if (lane_in(alive & ~pending)) begin_step<TAB>(S, e, st);
+    const unsigned long long m_geo = wave_ballot((int)st.path < 0) & alive;
+    const bool run_geo = m_geo == alive || __popcll(m_geo) >= geo_batch;
+    const unsigned long long step = run_geo ? alive : alive & ~m_geo;
+    pending = alive & ~step;
     Spawn sp;
-    sp.has = false;
+    sp.has = 0u;
     int res = STEP_CONTINUE;
-    const bool stepped = alive && (!st.geo || run_geo);
-    if (stepped) {
+    if (lane_in(step)) {
       PT_BEGIN(t_st);
-      res = finish_step<TAB>(S, G.jobs, e, sp, maxSteps, st);
-      pending = false;
+      res = finish_step<TAB>(S, jobs, e, sp, maxSteps, st);
       nsteps++;
       /* an electron is counted once, at its first step (it may be queued
        * again before taking one) */
-      if (e.steps == 1u) nelec++;
+      nelec += e.steps == 1u ? 1u : 0u;
       PT_END(PH_STEP, t_st);
     }
     PT_BEGIN(t_ta);
-    /* a new secondary starts where its parent's step ended, in the region
-     * the parent is in (trackSecondaryElectron, MonteCarloSS.cu:165-174);
-     * its state is set aside before any lane takes a new electron below */
-    uint32_t clo = 0, chi = 0;
-    if (sp.has) {
-      const uint64_t lin = child_lineage(((uint64_t)e.lin_hi << 32) | e.lin_lo, e.nchild++);
-      clo = (uint32_t)lin;
-      chi = (uint32_t)(lin >> 32);
-    }
-    const float cpx = e.px, cpy = e.py, cpz = e.pz;
-    const float csafe = sp.has && e.safe > 0.f ? fmaxf(0.f, e.safe - from_anchor(cpx, cpy, cpz)) : 0.f;
-    const int creg = e.region;
-    const uint32_t cprim = e.primary, cjob = e.job;
+    unsigned long long ends = wave_ballot(res != STEP_CONTINUE);
+    const unsigned long long born = wave_ballot(sp.has != 0u);
     /* regroup: an electron past its step budget for this launch continues in the next one */
-    const bool requeue = stepped && res == STEP_CONTINUE && G.steps_per_launch > 0 &&
-                         (int)(e.steps - steps0) >= G.steps_per_launch;
-    queue_append(G, requeue, e.px, e.py, e.pz, e.dx, e.dy, e.dz, e.E, e.region, e.primary, e.lin_lo, e.lin_hi, e.job,
-                 e.steps, e.nchild, lanemask_lt, nover);
-    /* escape records: one atomic per wave */
-    const bool esc = stepped && res == STEP_ESCAPED;
-    unsigned long long em = wave_ballot(esc);
-    if (em) {
-      int leader = __ffsll((long long)em) - 1;
-      uint32_t base = 0;
-      if (lane_id() == leader) base = atomicAdd(G.esc_count, (unsigned int)__popcll(em));
-      base = __shfl(base, leader);
-      if (esc) {
-        uint32_t slot = base + (uint32_t)__popcll(em & lanemask_lt);
-        if (slot < G.esc_cap) {
-          const uint32_t cap = G.esc_cap;
-          G.esc_f[0 * cap + slot] = e.px;
-          G.esc_f[1 * cap + slot] = e.py;
-          G.esc_f[2 * cap + slot] = e.pz;
-          G.esc_f[3 * cap + slot] = e.dx;
-          G.esc_f[4 * cap + slot] = e.dy;
-          G.esc_f[5 * cap + slot] = e.dz;
-          G.esc_f[6 * cap + slot] = e.E;
-          G.esc_u[0 * cap + slot] = e.primary;
-          G.esc_u[1 * cap + slot] = (e.job << 1) | (uint32_t)e.region;
-          G.esc_u[2 * cap + slot] = e.lin_lo;
-          G.esc_u[3 * cap + slot] = e.lin_hi;
-          G.esc_u[4 * cap + slot] = e.steps;
-        } else {
-          nover++;
-        }
+    unsigned long long requeue = 0ull;
+    if (regroup > 0) requeue = wave_ballot((int)(e.steps - steps0) >= regroup) & step & ~ends;
+    uint32_t clo = 0, chi = 0;
+    if (born) {
+      /* the lineage of a new secondary (trackSecondaryElectron, MonteCarloSS.cu:165-174) */
+      if (sp.has) {
+        const uint64_t lin = child_lineage(((uint64_t)e.lin_hi << 32) | e.lin_lo, e.nchild++);
+        clo = (uint32_t)lin;
+        chi = (uint32_t)(lin >> 32);
       }
     }
-    const bool ends = stepped && (res != STEP_CONTINUE || requeue);
-    if (ends) {
-      PT_END_ELECTRON(e.steps - steps0);
-      alive = false;
-      if (res == STEP_ESCAPED) nesc++;
-      if (res == STEP_WATCHDOG) {
-        nwd++;
-        const JobRec& J = G.jobs[e.job];
-        if (J.wd_log) {
-          const unsigned int k = atomicAdd(J.wd_count, 1u);
-          if (k < (unsigned int)kWatchdogLog) {
-            float* w = J.wd_log + (size_t)k * kWatchdogFields;
-            w[0] = e.px; w[1] = e.py; w[2] = e.pz;
-            w[3] = e.dx; w[4] = e.dy; w[5] = e.dz;
-            w[6] = e.E; w[7] = (float)e.region; w[8] = (float)e.steps; w[9] = (float)e.primary;
+    if (ends | requeue) {
+      const MONSEL_CS GenDev& G = launch_args()->G;
+      queue_append(G, requeue, e.px, e.py, e.pz, e.dx, e.dy, e.dz, e.E, e.region, e.primary, e.lin_lo, e.lin_hi, e.job,
+                   e.steps, e.nchild, lanemask_lt, nover);
+      /* escape records: one atomic per wave */
+      const unsigned long long em = wave_ballot(res == STEP_ESCAPED);
+      if (em) {
+        const int leader = __ffsll((long long)em) - 1;
+        uint32_t base = 0;
+        if (lane_id() == leader) base = atomicAdd(in_global(G.esc_count), (unsigned int)__popcll(em));
+        base = __builtin_amdgcn_readlane(base, leader);
+        if (lane_in(em)) {
+          nesc++;
+          const uint32_t slot = base + (uint32_t)__popcll(em & lanemask_lt);
+          const size_t cap = G.esc_cap;
+          if (slot < (uint32_t)cap) {
+            float* f = in_global(G.esc_f) + slot;
+            uint32_t* u = in_global(G.esc_u) + slot;
+            f[0] = e.px;
+            f[cap] = e.py;
+            f[2 * cap] = e.pz;
+            f[3 * cap] = e.dx;
+            f[4 * cap] = e.dy;
+            f[5 * cap] = e.dz;
+            f[6 * cap] = e.E;
+            u[0] = e.primary;
+            u[cap] = (e.job << 1) | (uint32_t)e.region;
+            u[2 * cap] = e.lin_lo;
+            u[3 * cap] = e.lin_hi;
+            u[4 * cap] = e.steps;
+          } else {
+            nover++;
           }
         }
       }
+      if (wave_ballot(res == STEP_WATCHDOG)) {
+        if (res == STEP_WATCHDOG) {
+          nwd++;
+          const JobRec& J = jobs[e.job];
+          if (J.wd_log) {
+            const unsigned int k = atomicAdd(J.wd_count, 1u);
+            if (k < (unsigned int)kWatchdogLog) {
+              float* w = J.wd_log + (size_t)k * kWatchdogFields;
+              w[0] = e.px; w[1] = e.py; w[2] = e.pz;
+              w[3] = e.dx; w[4] = e.dy; w[5] = e.dz;
+              w[6] = e.E; w[7] = (float)e.region; w[8] = (float)e.steps; w[9] = (float)e.primary;
+            }
+          }
+        }
+      }
+      ends |= requeue;
+#ifdef MONSEL_PHASE_TIMING
+      if (lane_in(ends)) PT_END_ELECTRON(e.steps - steps0);
+#endif
+      alive &= ~ends;
     }
-    /* new secondaries: the k-th spawning lane hands its secondary to the
+    /* new secondaries start where their parent's step ended, in the region
+     * the parent is in: the k-th spawning lane hands its secondary to the
      * k-th lane without an electron; the rest go to the queue for the next
      * launch.  An electron's stream depends only on its lineage, so which
      * lane runs it changes nothing. */
-    bool queue_spawn = sp.has;
-    if (G.handoff) {
+    if (born) {
+      const MONSEL_CS GenDev& G = launch_args()->G;
       /* a secondary whose parent left the chamber (region -1) goes to the
        * queue, whose containment check at the claim ends it */
-      const bool give = sp.has && creg >= 0;
-      const unsigned long long mg = wave_ballot(give);
-      const unsigned long long mt = wave_ballot(!alive);
-      if (mg && mt) {
-        const int n = min(__popcll(mg), __popcll(mt));
-        const int grank = __popcll(mg & lanemask_lt);
-        const int trank = __popcll(mt & lanemask_lt);
+      const unsigned long long mg = G.handoff ? wave_ballot((sp.has != 0u) & (e.region >= 0)) : 0ull;
+      const int n = min(__popcll(mg), __popcll(~alive));
+      const int grank = __popcll(mg & lanemask_lt);
+      const bool give = lane_in(mg) & (grank < n);
+      queue_append(G, born & ~wave_ballot(give), e.px, e.py, e.pz, sp.dx, sp.dy, sp.dz, sp.E, e.region, e.primary, clo,
+                   chi, e.job, 0u, 0u, lanemask_lt, nover);
+      if (n > 0) {
+        const float csafe = give && e.safe > 0.f ? fmaxf(0.f, e.safe - from_anchor(e.px, e.py, e.pz)) : 0.f;
         int* giver = lane_map();
-        if (give && grank < n) giver[grank] = lane_id();
+        if (give) giver[grank] = lane_id();
         __builtin_amdgcn_wave_barrier();
-        const bool take = !alive && trank < n;
+        const int trank = __popcll(~alive & lanemask_lt);
+        const bool take = lane_in(~alive) & (trank < n);
         const int src = take ? giver[trank] : lane_id();
-        const float tpx = __shfl(cpx, src), tpy = __shfl(cpy, src), tpz = __shfl(cpz, src);
+        const float tpx = __shfl(e.px, src), tpy = __shfl(e.py, src), tpz = __shfl(e.pz, src);
         const float tdx = __shfl(sp.dx, src), tdy = __shfl(sp.dy, src), tdz = __shfl(sp.dz, src);
         const float tE = __shfl(sp.E, src), tsafe = __shfl(csafe, src);
-        const int treg = __shfl(creg, src), tmax = __shfl(maxSteps, src);
-        const uint32_t tprim = __shfl(cprim, src), tlo = __shfl(clo, src), thi = __shfl(chi, src);
-        const uint32_t tjob = __shfl(cjob, src);
+        const int treg = __shfl(e.region, src), tmax = __shfl(maxSteps, src);
+        const uint32_t tprim = __shfl(e.primary, src), tlo = __shfl(clo, src), thi = __shfl(chi, src);
+        const uint32_t tjob = __shfl(e.job, src);
         if (take) {
           e.px = tpx; e.py = tpy; e.pz = tpz;
           e.dx = tdx; e.dy = tdy; e.dz = tdz;
@@ -1008,30 +1066,24 @@ k_transport(DevScene S, GenDev G) {
           e.safe = tsafe;
           set_anchor(tpx, tpy, tpz);
           if (e.job != cur_job) {
-            if (cur_job != 0xFFFFFFFFu) flush_lane_stats(G, cur_job, nsteps, nelec, nesc, nwd, nover);
+            if (cur_job != 0xFFFFFFFFu) flush_lane_stats(jobs, cur_job, nsteps, nelec, nesc, nwd, nover);
             cur_job = e.job;
           }
           maxSteps = tmax;
           steps0 = 0;
-          alive = true;
         }
-        if (give && grank < n) queue_spawn = false;
+        alive |= wave_ballot(take);
       }
     }
-    queue_append(G, queue_spawn, cpx, cpy, cpz, sp.dx, sp.dy, sp.dz, sp.E, creg, cprim, clo, chi, cjob, 0u, 0u,
-                 lanemask_lt, nover);
     /* tail compaction: once the launch's own items are all claimed, a wave
      * down to tail_lanes live lanes queues them for the next launch (which
      * packs them into full waves) and leaves.  A step begun but not finished
      * is redone there from the same state and draws. */
-    if (G.tail_lanes > 0) {
-      const unsigned long long ma = wave_ballot(alive);
-      if (ma && done && __popcll(ma) <= G.tail_lanes) {
-        queue_append(G, alive, e.px, e.py, e.pz, e.dx, e.dy, e.dz, e.E, e.region, e.primary, e.lin_lo, e.lin_hi,
-                     e.job, e.steps, e.nchild, lanemask_lt, nover);
-        alive = false;
-        pending = false;
-      }
+    if (done && alive && __popcll(alive) <= tail_lanes) {
+      queue_append(launch_args()->G, alive, e.px, e.py, e.pz, e.dx, e.dy, e.dz, e.E, e.region, e.primary, e.lin_lo,
+                   e.lin_hi, e.job, e.steps, e.nchild, lanemask_lt, nover);
+      alive = 0ull;
+      pending = 0ull;
     }
     PT_END(PH_TAIL, t_ta);
   }
@@ -1051,7 +1103,7 @@ k_transport(DevScene S, GenDev G) {
       wover += __shfl_down(wover, off);
     }
     if (lane_id() == 0) {
-      unsigned long long* st = stat_stripe(G.jobs[j0].stats);
+      unsigned long long* st = stat_stripe(jobs[j0].stats);
       atomicAdd(&st[kStatSteps], wsteps);
       atomicAdd(&st[kStatElectrons], welec);
       if (wesc) atomicAdd(&st[kStatEscapes], wesc);
@@ -1059,7 +1111,7 @@ k_transport(DevScene S, GenDev G) {
       if (wover) atomicAdd(&st[kStatOverflow], wover);
     }
   } else if (cur_job != 0xFFFFFFFFu) {
-    flush_lane_stats(G, cur_job, nsteps, nelec, nesc, nwd, nover);
+    flush_lane_stats(jobs, cur_job, nsteps, nelec, nesc, nwd, nover);
   }
 }
 
@@ -1381,7 +1433,7 @@ __global__ void k_probe_scatter(DevScene S, int mech, int n, const float* prevE,
   bool trapped = false;
   const float rate = mech_rate(S, m, prevE[i]);
   Deflect de;
-  de.has = false;
+  de.has = 0u;
   Spawn sp = mech_scatter(S, m, e, prevE[i], rate, trapped, uu, [](float*) {}, de);
   if (de.has) deflect(e, de);
   float* o = out + 11 * (size_t)i;
@@ -2691,9 +2743,9 @@ void run_generation(monsel_ctx_s* C) {
   g_hip_call = "launch k_transport";
   /* scenes without a tabulated mechanism run the kernel built without it */
   if (C->batch.dev.has_tabulated)
-    hipLaunchKernelGGL(k_transport<true>, dim3(grid), dim3(block), 0, C->stream, C->batch.dev, G);
+    hipLaunchKernelGGL(k_transport<true>, dim3(grid), dim3(block), 0, C->stream, TransportArgs{C->batch.dev, G});
   else
-    hipLaunchKernelGGL(k_transport<false>, dim3(grid), dim3(block), 0, C->stream, C->batch.dev, G);
+    hipLaunchKernelGGL(k_transport<false>, dim3(grid), dim3(block), 0, C->stream, TransportArgs{C->batch.dev, G});
   HIP_TRY(hipGetLastError());
   if (timing) HIP_TRY(hipEventRecord(C->evk1, C->stream));
   /* escape tallies: the histograms go through LDS when one job is in flight */
@@ -3391,9 +3443,9 @@ int monsel_run_static(monsel_ctx ctx, monsel_scene_id scene, const monsel_job_de
       spread_launch(G, T, n + in_count, (uint64_t)grid * (block / 64));
       g_hip_call = "launch k_transport";
       if (sd->dev.has_tabulated)
-        hipLaunchKernelGGL(k_transport<true>, dim3(grid), dim3(block), 0, stream, sd->dev, G);
+        hipLaunchKernelGGL(k_transport<true>, dim3(grid), dim3(block), 0, stream, TransportArgs{sd->dev, G});
       else
-        hipLaunchKernelGGL(k_transport<false>, dim3(grid), dim3(block), 0, stream, sd->dev, G);
+        hipLaunchKernelGGL(k_transport<false>, dim3(grid), dim3(block), 0, stream, TransportArgs{sd->dev, G});
       HIP_TRY(hipGetLastError());
       g_hip_call = "launch k_tally_escapes";
       hipLaunchKernelGGL(k_tally_escapes, dim3(ctx->n_cu * 4), dim3(256), (size_t)lj.off[lj.n] * 4, stream, sd->dev,

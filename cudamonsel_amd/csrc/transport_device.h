@@ -717,7 +717,7 @@ MD float mech_rate(const DevScene& S, const MONSEL_CS DMech& m, float EeV) {
 /* secondary produced by a scatter event (new Electron(*pe, theta, phi, E)
  * followed by an optional relative rotation) */
 struct Spawn {
-  bool has;
+  uint32_t has; /* 0 or 1 (a bool kept across branches costs scalar mask merges) */
   float dx, dy, dz;
   float E;
 };
@@ -782,7 +782,7 @@ MD void isotropic_dir(float u1, float u2, float& dx, float& dy, float& dz) {
  * parameters come from DMech::q (J). */
 MD Spawn tabulated_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e, const float* u) {
   Spawn se;
-  se.has = false;
+  se.has = 0u;
   const bool cd3 = (S.compat & MONSEL_COMPAT_D3_ABSCISSAE) != 0;
   const double J = 1.60217653e-19;
   const double kE0 = (double)e.E * J;
@@ -889,7 +889,7 @@ MD Spawn tabulated_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e,
       }
     }
   }
-  se.has = true;
+  se.has = 1u;
   se.E = (float)(energySE / J);
   return se;
 }
@@ -908,7 +908,7 @@ MD T of_three(int pick, T a, T b, T c) {
 /* A deflection of the electron's direction left for the end of the scatter:
  * polar angle by its cosine, azimuth by its uniform. */
 struct Deflect {
-  bool has;
+  uint32_t has;
   float cos_polar, u_azimuth;
 };
 
@@ -934,7 +934,7 @@ template <bool TAB = true, class Draw>
 MD Spawn mech_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e, float prevE, float rate, bool& trapped,
                       float* u, Draw draw_hi, Deflect& de, const float* esig = nullptr) {
   Spawn se;
-  se.has = false;
+  se.has = 0u;
   switch (m.kind) {
     case MONSEL_MECH_NISTMOTT_ELASTIC:
     case MONSEL_MECH_BROWNING_ELASTIC:
@@ -970,7 +970,7 @@ MD Spawn mech_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e, floa
       draw_hi(u);
       /* the polar angle takes one uniform (two for Browning), the azimuth
        * the next one (SelectableElasticSM.cu:62-64) */
-      de.has = true;
+      de.has = 1u;
       de.u_azimuth = u[4];
       if (m.kind == MONSEL_MECH_BROWNING_ELASTIC || (nist && prevE < m.extrap)) {
         float z, zp3;
@@ -999,7 +999,7 @@ MD Spawn mech_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e, floa
       float u_th = u[3];
       isotropic_dir(u_th, u_phi, se.dx, se.dy, se.dz);
       se.E = m.p[1];
-      se.has = true;
+      se.has = 1u;
       PT_END(PH_FITTED, t_fi);
       return se;
     }
@@ -1030,7 +1030,7 @@ MD Spawn mech_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e, floa
             r0 * __builtin_amdgcn_logf(fdiv((-2.f * (1.f + root)) + x, (-2.f * (1.f - root)) + x)));
         ct = temp + fdiv(((x - 2.f) * (temp - 1.f)) / 2.f, root);
       }
-      de.has = true;
+      de.has = 1u;
       de.cos_polar = ct;
       de.u_azimuth = r1;
       e.E = kE0 - m.p[0];
