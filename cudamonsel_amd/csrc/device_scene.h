@@ -35,20 +35,23 @@ enum PrimKind { PRIM_PLANES = 0, PRIM_CYLINDER = 1, PRIM_SPHERE = 2 };
 
 /* One convex primitive.  Planes: inside is n.p - b <= 0. */
 struct DPrim {
+  /* 16 words: what a cylinder or a sphere needs, and a multi-plane
+   * primitive's counts */
   int kind;
-  int first_plane;
   int n_planes;
   int tie;       /* bit k: a line within plane k counts as inside (plane_tie_break) */
-  float sdscale; /* planes: min over the planes of 1/|n| (distance bounds); 1 otherwise */
+  int first_plane;
   float e0[3];   /* cylinder end0 / sphere centre (nm) */
+  float r2;      /* radius^2 (nm^2) */
   float ax[3];   /* cylinder unit axis */
   float len;     /* cylinder length (nm) */
-  float r2;      /* radius^2 (nm^2) */
-  float axv[3];  /* cylinder axis vector end1-end0 (nm), for point containment */
+  float sdscale; /* planes: min over the planes of 1/|n| (distance bounds); 1 otherwise */
   float len2;    /* |axv|^2 */
-  float pad[3];
+  float pad[2];
   float4 pl[4];  /* the first planes of a multi-plane primitive again, inline (one
                   * fewer dependent load for the common primitives) */
+  float axv[3];  /* cylinder axis vector end1-end0 (nm), for point containment */
+  float pad2;
 };
 constexpr int kInlinePlanes = 4;
 
@@ -62,19 +65,8 @@ struct DShape {
   int first_prim;
   int n_prims;
   int is_sphere; /* the chamber sphere: a single primitive */
-  int pad;
+  int region;    /* the region of this shape, in the list of a region's children */
   uint32_t truth[8];
-};
-
-struct DRegion {
-  int parent;
-  int shape;
-  int msm;
-  int first_child;
-  int n_children;
-  int depth;
-  int pad[2];
-  DShape sh;    /* its shape's record again, inline (one fewer dependent load) */
 };
 
 /* JoyLuoNieminenCSD (eV, nm). */
@@ -84,13 +76,12 @@ struct DCSD {
   float breakE;  /* eV */
   float gamma15; /* 1.5 gamma, 1/(nm eV^1.5) */
   float minE;    /* eV (barrier height) */
-  float pad[3];
-  struct Term {  /* one element's, read with one scalar load */
+  struct Term {  /* one element's; the first three end the record's first 16 words */
     float recipJ; /* 1/eV */
     float beta;
     float coef;   /* eV^2/nm */
-    float pad;
   } el[kMaxElem];
+  float pad[3];
 };
 
 /* One element of an elastic (SelectableElasticSM) mechanism. */
@@ -118,26 +109,27 @@ struct DElem {
  * atoms. */
 constexpr int kFewElem = 3;
 struct DFewElem {
-  float natoms[4];
-  float sfBrowning[4];
-  float brNum[4], brRoot[4], brInv[4];
-  int spwem[4];  /* offset of the element's cross-section nodes */
-  int x1[4];     /* and of its angle table */
-  float z[4], zp3[4];
+  float natoms[kFewElem];
+  float sfBrowning[kFewElem];
+  float brNum[kFewElem], brRoot[kFewElem], brInv[kFewElem];
+  float extrap;          /* eV, NISTMottRS extrapolateBelowEnergy (the elements share it) */
+  int spwem[kFewElem];   /* offset of the element's cross-section nodes */
+  int x1[kFewElem];      /* and of its angle table */
+  float z[kFewElem], zp3[kFewElem];
 };
 
 struct DMech {
   int kind;
-  int elem0;
   int nelem;
-  int method;
-  int table[4];
-  float extrap; /* elastic: eV, NISTMottRS extrapolateBelowEnergy (its elements share it) */
   int few;      /* elastic: `el` holds its elements, and their Mott nodes are in LDS */
+  int method;
+  float extrap; /* elastic: eV, NISTMottRS extrapolateBelowEnergy (its elements share it) */
+  int elem0;
   int pad[2];
-  DFewElem el;
   float p[24];
   DCSD csd; /* FittedInelSM's slowing-down algorithm */
+  DFewElem el;
+  int table[4];
   double q[24]; /* tabulated mechanism: the TP_* slots in SI units (J) for the FP64 scatter */
 };
 
@@ -162,6 +154,20 @@ struct DMSM {
   DCSD csd;
 };
 
+/* One region.  Its scatter model's and its shape's records are inline, so
+ * that a step reads them at an offset of one address. */
+struct DRegion {
+  DMSM m;
+  int parent;
+  int shape;
+  int msm;
+  int first_child;
+  int n_children;
+  int depth;
+  int pad[2];
+  DShape sh;
+};
+
 /* Non-uniform table (NUTableInterpolation) in the file's own units. */
 struct DNUTable {
   int dim;
@@ -178,7 +184,7 @@ struct DevScene {
   float chamber_r;        /* nm */
   float chamber_c[3];     /* nm */
   const MONSEL_CS DRegion* regions;
-  const MONSEL_CS int* children;
+  const MONSEL_CS DShape* children;   /* the shapes of each region's children, in a run */
   const MONSEL_CS DShape* shapes;
   const MONSEL_CS DPrim* prims;
   const MONSEL_CS float4* planes;   /* (nx, ny, nz, b) */

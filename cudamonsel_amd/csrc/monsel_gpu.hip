@@ -432,7 +432,8 @@ struct StepStart {
 template <bool TAB>
 __device__ __forceinline__ void begin_step_in(const DevScene& S, int region, Elec& e, StepStart& st) {
   PT_BEGIN(t_ra);
-  const MONSEL_CS DMSM& msm = S.msms[S.regions[region].msm];
+  const MONSEL_CS DMSM& msm = S.regions[region].m;
+  int is_null = msm.is_null, n_mech = msm.n_mech, mech0 = msm.mech0, elastic_k = msm.elastic_k;
   float u[4];
   PT_BEGIN(t_un);
   step_uniforms_lo(e, kPhiloxKey0, kPhiloxKey1, u);
@@ -441,14 +442,15 @@ __device__ __forceinline__ void begin_step_in(const DevScene& S, int region, Ele
   float total = 0.f;
   float freePath;
   const float maxFreePath = 2.f * S.chamber_r;
-  if (msm.is_null) {
+  pin(is_null, n_mech, mech0, elastic_k);
+  if (is_null) {
     freePath = 1.0e9f; /* NullMaterialScatterModel.cu:32-35: 1 m */
   } else {
     PT_BEGIN(t_rl);
-    for (int k = 0; k < msm.n_mech; ++k) {
-      const MONSEL_CS DMech& m = S.mechs[msm.mech0 + k];
+    for (int k = 0; k < n_mech; ++k) {
+      const MONSEL_CS DMech& m = S.mechs[mech0 + k];
       float rk;
-      if (k == msm.elastic_k) {
+      if (k == elastic_k) {
         /* elastic_rate, keeping its terms */
         if (m.few) {
           float c[kFewElem];
@@ -521,7 +523,10 @@ template <bool TAB>
 __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* jobs, const int region, Elec& e,
                                               Spawn& sp, int maxSteps, const StepStart& st) {
   const MONSEL_CS DRegion& rg = S.regions[region];
-  const MONSEL_CS DMSM& msm = S.msms[rg.msm];
+  const MONSEL_CS DMSM& msm = rg.m;
+  int is_null = msm.is_null, n_mech = msm.n_mech, mech0 = msm.mech0, elastic_k = msm.elastic_k;
+  float minE = msm.minE;
+  pin(is_null, n_mech, mech0, elastic_k, minE);
   /* the reference's barrier ignores the surface normal in compat mode */
   const bool normals = (S.compat & MONSEL_COMPAT_BARRIER_NORMAL) == 0u;
   const bool geo = (int)st.path < 0;
@@ -549,7 +554,7 @@ __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* j
      * for some lane, the wave computes the end point's bound; the pass costs
      * the wave the same whichever lanes take part, so every lane of it that
      * crossed no boundary refreshes its bound (and keeps the better one). */
-    if (!msm.is_null && wave_any(geo & !boundary) && !boundary) {
+    if (!is_null && wave_any(geo & !boundary) && !boundary) {
       PT_BEGIN(t_sf);
       const float fresh = region_safety(S, region, e.px, e.py, e.pz);
       const float kept = e.safe > 0.f ? e.safe - from_anchor(e.px, e.py, e.pz) : 0.f;
@@ -577,11 +582,11 @@ __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* j
   }
   const float prevE = e.E;
   PT_BEGIN(t_cs);
-  if (!msm.is_null) e.E += csd_compute(msm.csd, se.t, e.E);
+  if (!is_null) e.E += csd_compute(msm.csd, se.t, e.E);
   PT_END(PH_CSD, t_cs);
   e.steps++;
   int res = STEP_CONTINUE;
-  if (e.E < msm.minE) res = STEP_DEAD;
+  if (e.E < minE) res = STEP_DEAD;
   if (((int)e.steps > maxSteps) | !(e.E == e.E)) res = STEP_WATCHDOG;
   const bool crossed = se.next != region;
   uint32_t check = 0u;   /* the containment check that opens the next step is due */
@@ -594,7 +599,7 @@ __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* j
       /* ExpQMBarrierSM::barrierScatter (ExpQMBarrierSM.cu:50-219) */
       PT_BEGIN(t_ba);
       const int next = se.next;
-      if (msm.is_null || msm.barrier_kind == MONSEL_BARRIER_NONE) {
+      if (is_null || msm.barrier_kind == MONSEL_BARRIER_NONE) {
         e.region = next;
       } else {
         /* ExpQMBarrierSM.cu:77-96: outward normal of the struck shape, negated
@@ -615,7 +620,7 @@ __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* j
               nbx = se.ownNx; nby = se.ownNy; nbz = se.ownNz;
             }
           }
-          barrier_core(S, msm, S.msms[S.regions[to].msm], e, to, nbx, nby, nbz, st.u1);
+          barrier_core(S, msm, S.regions[to].m, e, to, nbx, nby, nbz, st.u1);
         });
       }
       /* MonteCarloSS.cu:146-148: nudge along the new direction; the region is
@@ -650,7 +655,7 @@ __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* j
     int idx = 0;
     float rate = rates[0];
     float cum = rate;
-    for (int k = 1; k < msm.n_mech; ++k) {
+    for (int k = 1; k < n_mech; ++k) {
       const float rk = rates[k * kLaneBlock];
       const bool past = (idx == k - 1) & (cum < r);
       idx = past ? k : idx;
@@ -668,20 +673,20 @@ __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* j
      * is wave-uniform */
     Deflect de;
     de.has = 0u;
-    for (int k = 0; k < msm.n_mech; ++k) {
+    for (int k = 0; k < n_mech; ++k) {
       const unsigned long long turn = wave_ballot(idx == k);
       if (!turn) continue;
-      const MONSEL_CS DMech& m = S.mechs[msm.mech0 + k];
+      const MONSEL_CS DMech& m = S.mechs[mech0 + k];
       if (lane_in(turn))
         sp = mech_scatter<TAB>(
             S, m, e, prevE, rate, trapped, u,
             [&](float* v) { step_uniforms_hi(e, kPhiloxKey0, kPhiloxKey1, v); }, de,
-            k == msm.elastic_k ? lane_esig() : nullptr);
+            k == elastic_k ? lane_esig() : nullptr);
     }
     if (de.has) deflect(e, de);
     /* trackSecondaryElectron (MonteCarloSS.cu:165-174) */
-    sp.has = sp.has && sp.E > msm.minE ? 1u : 0u;
-    if (trapped | (e.E < msm.minE)) res = STEP_DEAD;
+    sp.has = sp.has && sp.E > minE ? 1u : 0u;
+    if (trapped | (e.E < minE)) res = STEP_DEAD;
   }
   if (check && res == STEP_CONTINUE && !locate(S, jobs, e, e.region)) res = STEP_DEAD;
   return res;
@@ -1635,7 +1640,7 @@ struct HBuf {
 
 struct HostScene {
   std::vector<DRegion> regions;
-  std::vector<int> children;
+  std::vector<DShape> children;
   std::vector<DShape> shapes;
   std::vector<DPrim> prims;
   std::vector<float4> planes;
@@ -1657,36 +1662,41 @@ struct SceneDev {
   DBuf blob;
   DevScene dev{};
   size_t bytes = 0;
-  int step_prims = 0; /* the most primitives one findEndOfStep call tests */
+  int step_cost = 0; /* what one findEndOfStep call costs at most (max_step_cost) */
   HostScene host;     /* kept to assemble batch scenes */
 };
 
-/* The most primitives one findEndOfStep call tests in the scene: a region's
- * own shape and its children's, the chamber's sphere aside (an electron
- * meets it once, on its way out). */
-int max_step_prims(const HostScene& H) {
-  auto prims = [&](int region) {
+/* What one findEndOfStep call costs in the scene at most: the primitives of a
+ * region's own shape and its children's, a cylinder counted as two, the
+ * chamber's sphere aside (an electron meets it once, on its way out). */
+int max_step_cost(const HostScene& H) {
+  auto cost = [&](int region) {
     const DShape& sh = H.shapes[H.regions[region].shape];
-    return sh.is_sphere ? 0 : sh.n_prims;
+    int n = 0;
+    for (int k = 0; k < sh.n_prims; ++k) n += H.prims[sh.first_prim + k].kind == PRIM_CYLINDER ? 2 : 1;
+    return sh.is_sphere ? 0 : n;
   };
   int most = 0;
   for (int r = 0; r < (int)H.regions.size(); ++r) {
-    int n = prims(r);
-    for (int c = 0; c < H.regions[r].n_children; ++c) n += prims(H.children[H.regions[r].first_child + c]);
+    int n = cost(r);
+    for (int c = 0; c < H.regions[r].n_children; ++c) n += cost(H.children[H.regions[r].first_child + c].region);
     most = std::max(most, n);
   }
   return most;
 }
 
 /* Lanes a wave gathers for findEndOfStep when the tuning leaves it open (0):
- * gathering pays where a call tests several primitives (line and image
- * scenes, 3 or more: 11 to 14 % more primaries/s with 8) and costs where it
- * tests one or two (flat and step-edge yield jobs: 2 to 4 % slower).  A
- * launch of few items (a small job alone) leaves most of the device idle and
- * lasts as long as its longest cascade, which waiting only lengthens. */
-int geometry_batch_for(int tuned, int stepPrims, uint64_t items) {
+ * gathering pays the more the call costs.  256 x 256 image of three lines
+ * (cost above 6): 8 lanes 723 ms, 12: 701, 16: 692 (1: 20 % more than 8), six
+ * requests of mixed sizes and scenes 278, 281 and 288 ms; contact hole image
+ * (cost 3): 1: 92.5 ms, 8: 86.7, 16: 91.2; flat and step-edge yield jobs (cost
+ * 1 and 2): 1: 539 ms, 4: 554.  A launch of few items (a small job
+ * alone) leaves most of the device idle and lasts as long as its longest
+ * cascade, which waiting only lengthens. */
+int geometry_batch_for(int tuned, int stepCost, uint64_t items) {
   if (tuned > 0) return tuned;
-  return stepPrims >= 3 && items >= kTailMinItems ? 8 : 1;
+  if (items < kTailMinItems) return 1;
+  return stepCost >= 6 ? 12 : (stepCost >= 3 ? 8 : 1);
 }
 
 /* How a launch spreads its items over its waves.  A launch of fewer than
@@ -1771,7 +1781,8 @@ void fill_few(const HostScene& H, DMech& dm) {
   }
   /* slots beyond the last element: no atoms, and denominators that stay
    * finite */
-  for (int i = std::max(dm.nelem, 0); i < 4; ++i) dm.el.brRoot[i] = dm.el.z[i] = 1.f;
+  dm.el.extrap = dm.extrap;
+  for (int i = std::max(dm.nelem, 0); i < kFewElem; ++i) dm.el.brRoot[i] = dm.el.z[i] = 1.f;
 }
 
 /* collect the convex leaves of a CSG tree (deduplicated by shape index) */
@@ -2118,11 +2129,15 @@ HostScene compile_scene(const monsel_scene_desc* d) {
     dr.first_child = (int)H.children.size();
     dr.n_children = (int)kids[r].size();
     dr.depth = dr.parent < 0 ? 0 : H.regions[dr.parent].depth + 1;
+    dr.m = H.msms[dr.msm];
     dr.sh = H.shapes[dr.shape];
-    for (int c : kids[r]) H.children.push_back(c);
+    for (int c : kids[r]) {
+      H.children.push_back(H.shapes[shapeIdx[d->regions[c].shape]]);
+      H.children.back().region = c;
+    }
     H.regions.push_back(dr);
   }
-  if (H.children.empty()) H.children.push_back(0);
+  if (H.children.empty()) H.children.push_back(DShape{});
   return H;
 }
 
@@ -2139,7 +2154,7 @@ size_t host_scene_bytes(const HostScene& H) {
   size_t total = 0;
   auto add = [&](size_t bytes) { total = ((total + 255) & ~(size_t)255) + bytes; };
   add(H.regions.size() * sizeof(DRegion));
-  add(H.children.size() * sizeof(int));
+  add(H.children.size() * sizeof(DShape));
   add(H.shapes.size() * sizeof(DShape));
   add(H.prims.size() * sizeof(DPrim));
   add(H.planes.size() * sizeof(float4));
@@ -2194,7 +2209,7 @@ void upload_scene(const HostScene& H, SceneDev& sd) {
   S.nu_data = (decltype(S.nu_data))(b + o_nd);
   S.nu_data64 = (decltype(S.nu_data64))(b + o_nd64);
   sd.bytes = blob.size();
-  sd.step_prims = max_step_prims(H);
+  sd.step_cost = max_step_cost(H);
 }
 
 /* One device scene holding several scenes side by side: every index is
@@ -2216,10 +2231,15 @@ HostScene merge_scenes(const std::vector<const HostScene*>& parts, std::vector<i
       r.shape += o_sh;
       r.sh.first_prim += o_pr;
       r.msm += o_msm;
+      r.m.mech0 += o_me;
       r.first_child += o_ch;
       M.regions.push_back(r);
     }
-    for (int c : P->children) M.children.push_back(c + o_reg);
+    for (DShape c : P->children) {
+      c.first_prim += o_pr;
+      c.region += o_reg;
+      M.children.push_back(c);
+    }
     for (DShape sh : P->shapes) {
       sh.first_prim += o_pr;
       M.shapes.push_back(sh);
@@ -2430,7 +2450,7 @@ void rebuild_batch_scene(monsel_ctx_s* C) {
   C->batch.blob = std::move(fresh.blob);
   C->batch.dev = fresh.dev;
   C->batch.bytes = fresh.bytes;
-  C->batch.step_prims = fresh.step_prims;
+  C->batch.step_cost = fresh.step_cost;
 }
 
 void finish_job(monsel_ctx_s* C, const std::shared_ptr<Job>& job, int st, const std::string& msg) {
@@ -2731,7 +2751,7 @@ void run_generation(monsel_ctx_s* C) {
   G.esc_cap = cap;
   G.esc_count = counts + 2;
   G.steps_per_launch = C->tuning.steps_per_launch;
-  G.geo_batch = geometry_batch_for(C->tuning.geometry_batch, C->batch.step_prims, nprim + C->in_count);
+  G.geo_batch = geometry_batch_for(C->tuning.geometry_batch, C->batch.step_cost, nprim + C->in_count);
   G.handoff = C->tuning.spawn_handoff >= 0 ? 1 : 0;
   const int block = C->tuning.block_size > 0 ? C->tuning.block_size : 256;
   const int grid = C->n_cu * C->blocks_per_cu[C->batch.dev.has_tabulated ? 1 : 0];
@@ -3438,7 +3458,7 @@ int monsel_run_static(monsel_ctx ctx, monsel_scene_id scene, const monsel_job_de
       G.esc_cap = (uint32_t)cap;
       G.esc_count = d_cnt + 2;
       G.steps_per_launch = T.steps_per_launch;
-      G.geo_batch = geometry_batch_for(T.geometry_batch, sd->step_prims, n + in_count);
+      G.geo_batch = geometry_batch_for(T.geometry_batch, sd->step_cost, n + in_count);
       G.handoff = T.spawn_handoff >= 0 ? 1 : 0;
       spread_launch(G, T, n + in_count, (uint64_t)grid * (block / 64));
       g_hip_call = "launch k_transport";

@@ -50,6 +50,19 @@ MD float fsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 MD float flog(float x) { return __builtin_amdgcn_logf(x) * 0.693147180559945309f; }
 MD float fexp(float x) { return __builtin_amdgcn_exp2f(x * 1.442695040888963407f); }
 
+/* Holds wave-uniform values in scalar registers from here on: the loads that
+ * feed several of them are then issued together and waited for once, instead
+ * of each sinking to its first use behind a branch (a step waited for some 80
+ * scalar loads one by one). */
+MD void pin() {}
+template <class T, class... Rest>
+MD void pin(T& v, Rest&... rest) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(v));
+#endif
+  pin(rest...);
+}
+
 /* a product that is not contracted into a following sum */
 MD float fmul(float a, float b) {
 #pragma clang fp contract(off)
@@ -310,8 +323,16 @@ MD void elastic_terms_few(const DevScene& S, const MONSEL_CS DMech& m, float EeV
   const bool mott = m.kind == MONSEL_MECH_NISTMOTT_ELASTIC;
   const bool one = m.nelem == 1;
   const MONSEL_CS DFewElem& el = m.el;
+  float n0 = el.natoms[0], n1 = el.natoms[1], n2 = el.natoms[2];
+  float s0 = el.sfBrowning[0], s1 = el.sfBrowning[1], s2 = el.sfBrowning[2];
+  float a0 = el.brNum[0], a1 = el.brNum[1], a2 = el.brNum[2];
+  float b0 = el.brRoot[0], b1 = el.brRoot[1], b2 = el.brRoot[2];
+  float d0 = el.brInv[0], d1 = el.brInv[1], d2 = el.brInv[2];
+  float extrap = el.extrap;
+  int t0 = el.spwem[0], t1 = el.spwem[1], t2 = el.spwem[2];
+  pin(n0, n1, n2, s0, s1, s2, a0, a1, a2, b0, b1, b2, d0, d1, d2, extrap, t0, t1, t2);
   c[0] = c[1] = c[2] = 0.f;
-  if (m.kind == MONSEL_MECH_BROWNING_ELASTIC || (mott && EeV < m.extrap)) {
+  if (m.kind == MONSEL_MECH_BROWNING_ELASTIC || (mott && EeV < extrap)) {
     if (mott && m.method == 3) {
 #pragma unroll
       for (int i = 0; i < kFewElem; ++i)
@@ -323,27 +344,24 @@ MD void elastic_terms_few(const DevScene& S, const MONSEL_CS DMech& m, float EeV
       const float e = EeV * 1.0e-3f;
       const float re = fsqrt(e);
       const float inv_re = __builtin_amdgcn_rcpf(re);
-      auto term = [&](int i) {
-        const float b = browning_sigma(el.brNum[i], el.brRoot[i], el.brInv[i], e, re, inv_re);
-        c[i] = fmul(mott ? fmul(el.sfBrowning[i], b) : b, el.natoms[i]);
+      auto term = [&](float num, float root, float inv, float sf, float n) {
+        const float b = browning_sigma(num, root, inv, e, re, inv_re);
+        return fmul(mott ? fmul(sf, b) : b, n);
       };
-      term(0);
+      c[0] = term(a0, b0, d0, s0, n0);
       if (!one) {
-        term(1);
-        term(2);
+        c[1] = term(a1, b1, d1, s1, n1);
+        c[2] = term(a2, b2, d2, s2, n2);
       }
     }
   } else if (mott && EeV < kMaxNISTMott) {
     const MottWindow w = mott_window(EeV);
     const float* f = lds_spwem() + w.i0;
-    auto term = [&](int i) {
-      const float* q = f + el.spwem[i];
-      c[i] = fmul(mott_sigma(w, q[0], q[1], q[2], q[3]), el.natoms[i]);
-    };
-    term(0);
+    auto term = [&](int t, float n) { return fmul(mott_sigma(w, f[t], f[t + 1], f[t + 2], f[t + 3]), n); };
+    c[0] = term(t0, n0);
     if (!one) {
-      term(1);
-      term(2);
+      c[1] = term(t1, n1);
+      c[2] = term(t2, n2);
     }
   } else {
 #pragma unroll
@@ -420,16 +438,30 @@ MD float nieminen_factor(float eps) {
   return eps < 1e-3f ? series : power;
 }
 
+/* A stopping-power record's head and its first three elements, in scalar
+ * registers: one 16-word load. */
+struct CSDHead {
+  int active, nce;
+  float breakE, gamma15, minE;
+  float r0, b0, k0, r1, b1, k1, r2, b2, k2;
+};
+MD CSDHead csd_head(const MONSEL_CS DCSD& c) {
+  CSDHead h = {c.active,      c.nce,      c.breakE,   c.gamma15,      c.minE,     c.el[0].recipJ, c.el[0].beta,
+               c.el[0].coef, c.el[1].recipJ, c.el[1].beta, c.el[1].coef, c.el[2].recipJ, c.el[2].beta, c.el[2].coef};
+  pin(h.active, h.nce, h.breakE, h.gamma15, h.minE, h.r0, h.b0, h.k0, h.r1, h.b1, h.k1, h.r2, h.b2, h.k2);
+  return h;
+}
+
 /* sum over the elements of coef ln(E / J + beta) */
-MD float joy_luo_sum(const MONSEL_CS DCSD& c, float kE) {
+MD float joy_luo_sum(const MONSEL_CS DCSD& c, const CSDHead& h, float kE) {
   float s = 0.f;
-  auto term = [&](int i) { s += c.el[i].coef * flog(c.el[i].recipJ * kE + c.el[i].beta); };
-  term(0);
-  if (c.nce > 1) {
+  auto term = [&](float recipJ, float beta, float coef) { s += coef * flog(recipJ * kE + beta); };
+  term(h.r0, h.b0, h.k0);
+  if (h.nce > 1) {
     /* slots beyond the last element add 0 */
-    term(1);
-    term(2);
-    for (int i = 3; i < c.nce; ++i) term(i);
+    term(h.r1, h.b1, h.k1);
+    term(h.r2, h.b2, h.k2);
+    for (int i = 3; i < h.nce; ++i) term(c.el[i].recipJ, c.el[i].beta, c.el[i].coef);
   }
   return s;
 }
@@ -439,26 +471,27 @@ MD float joy_luo_sum(const MONSEL_CS DCSD& c, float kE) {
  * `pending` marks a second half at depth d.  Below breakE the Nieminen form
  * kE (1 + 1.5 gamma len kE^1.5)^(-2/3) - kE; above it the Joy-Luo loss,
  * halved while it exceeds 10% of the energy. */
-MD float csd_compute_split(const MONSEL_CS DCSD& c, float len, float kE);
+MD float csd_compute_split(const MONSEL_CS DCSD& c, const CSDHead& h, float len, float kE);
 
 /* The common case in straight-line code: one segment, no halving (the
  * first pass of csd_compute_split, with the same arithmetic). */
 MD float csd_compute(const MONSEL_CS DCSD& c, float len, float kE) {
 #pragma clang fp contract(off)
-  if (!c.active || c.nce == 0) return 0.f;
-  if (kE < c.minE || kE <= 0.f) return 0.f;
+  const CSDHead h = csd_head(c);
+  if (!h.active || h.nce == 0) return 0.f;
+  if ((kE < h.minE) | (kE <= 0.f)) return 0.f;
   float dE;
-  if (kE <= c.breakE) {
-    dE = kE * nieminen_factor(c.gamma15 * len * kE * fsqrt(kE));
+  if (kE <= h.breakE) {
+    dE = kE * nieminen_factor(h.gamma15 * len * kE * fsqrt(kE));
   } else {
-    const float loss = fdiv(joy_luo_sum(c, kE) * len, kE);
+    const float loss = fdiv(joy_luo_sum(c, h, kE) * len, kE);
     dE = -loss;
-    if (loss > 0.1f * kE) dE = csd_compute_split(c, len, kE);
+    if (loss > 0.1f * kE) dE = csd_compute_split(c, h, len, kE);
   }
   return dE;
 }
 
-MD float csd_compute_split(const MONSEL_CS DCSD& c, float len, float kE) {
+MD float csd_compute_split(const MONSEL_CS DCSD& c, const CSDHead& h, float len, float kE) {
 #pragma clang fp contract(off)
   float E = kE, total = 0.f;
   uint32_t pending = 0;
@@ -466,11 +499,11 @@ MD float csd_compute_split(const MONSEL_CS DCSD& c, float len, float kE) {
   for (int it = 0; it < 128; ++it) {
     const float seg = ldexpf(len, -d);
     float dE = 0.f;
-    if (!(E < c.minE || E <= 0.f)) {
-      if (E <= c.breakE) {
-        dE = E * nieminen_factor(c.gamma15 * seg * E * fsqrt(E));
+    if (!((E < h.minE) | (E <= 0.f))) {
+      if (E <= h.breakE) {
+        dE = E * nieminen_factor(h.gamma15 * seg * E * fsqrt(E));
       } else {
-        const float loss = fdiv(joy_luo_sum(c, E) * seg, E);
+        const float loss = fdiv(joy_luo_sum(c, h, E) * seg, E);
         if (loss > 0.1f * E && d < 30) {
           pending |= 1u << (d + 1);
           d += 1;
@@ -686,23 +719,26 @@ MD float elastic_rate(const DevScene& S, const MONSEL_CS DMech& m, float EeV) {
 /* ScatterMechanism::scatterRate (1/nm); TAB as for mech_scatter */
 template <bool TAB = true>
 MD float mech_rate(const DevScene& S, const MONSEL_CS DMech& m, float EeV) {
-  switch (m.kind) {
+  int kind = m.kind;
+  float p0 = m.p[0], p1 = m.p[1], p2 = m.p[2];
+  pin(kind, p0, p1, p2);
+  switch (kind) {
     case MONSEL_MECH_NISTMOTT_ELASTIC:
     case MONSEL_MECH_BROWNING_ELASTIC:
     case MONSEL_MECH_RUTHERFORD_ELASTIC:
       return elastic_rate(S, m, EeV);
     case MONSEL_MECH_FITTED_INELASTIC: /* FittedInelSM.cu:20-25 */
-      if (EeV <= m.p[0]) return 0.f;
-      return -csd_compute(m.csd, 0.1f, EeV) * 10.f * m.p[2];
+      if (EeV <= p0) return 0.f;
+      return -csd_compute(m.csd, 0.1f, EeV) * 10.f * p2;
     case MONSEL_MECH_POLARON_TRAP: /* GanachaudMokraniPolaronTrapSM.cu:21-27 */
-      if (EeV > m.p[2]) return 0.f;
-      return m.p[0] * fexp(-m.p[1] * EeV);
+      if (EeV > p2) return 0.f;
+      return p0 * fexp(-p1 * EeV);
     case MONSEL_MECH_PHONON: { /* GanachaudMokraniPhononInelasticSM.cu:46-72 */
-      if (EeV < m.p[0]) return 0.f;
-      const float x = fdiv(m.p[0], EeV);
+      if (EeV < p0) return 0.f;
+      const float x = fdiv(p0, EeV);
       const float temp = fsqrt(1.f - x);
       const bool small = x < 0.1f;
-      const float rate = m.p[1] * x * flog(fdiv(small ? 4.f : 1.f + temp, small ? x : 1.f - temp));
+      const float rate = p1 * x * flog(fdiv(small ? 4.f : 1.f + temp, small ? x : 1.f - temp));
       return small || !(x >= 1.f) ? rate : 0.f;
     }
     case MONSEL_MECH_TABULATED_INELASTIC: if constexpr (TAB) { /* TabulatedInelasticSM.cu:436-459 */
@@ -1073,6 +1109,20 @@ MD float4 prim_plane(const DevScene& S, const MONSEL_CS DPrim& pr, int k) {
   return k < kInlinePlanes ? pr.pl[k] : S.planes[pr.first_plane + k];
 }
 
+/* f(plane, k) for every plane of a wave-uniform multi-plane primitive; the
+ * first four are loaded together (a slot beyond the last plane is 0) */
+template <class F>
+MD void for_planes(const DevScene& S, const MONSEL_CS DPrim& pr, F f) {
+  float4 a = pr.pl[0], b = pr.pl[1], c = pr.pl[2], d = pr.pl[3];
+  const int n = pr.n_planes;
+  pin(a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, c.x, c.y, c.z, c.w, d.x, d.y, d.z, d.w);
+  f(a, 0);
+  if (n > 1) f(b, 1);
+  if (n > 2) f(c, 2);
+  if (n > 3) f(d, 3);
+  for (int k = kInlinePlanes; k < n; ++k) f(S.planes[pr.first_plane + k], k);
+}
+
 /* Parameter interval of the line p + t d inside a convex primitive (empty
  * intervals come back with tin > tout).  The primitive is the same on every
  * active lane, so its kind and plane count branch uniformly; what differs by
@@ -1101,11 +1151,7 @@ MD Interval prim_interval(const DevScene& S, const MONSEL_CS DPrim& pr, float px
       iv.tin = enters ? t : iv.tin;
       iv.fin = enters ? k : iv.fin;
     };
-    const int n = pr.n_planes;
-#pragma unroll
-    for (int k = 0; k < kInlinePlanes; ++k)
-      if (k < n) plane(pr.pl[k], k);
-    for (int k = kInlinePlanes; k < n; ++k) plane(S.planes[pr.first_plane + k], k);
+    for_planes(S, pr, plane);
   } else if (pr.kind == PRIM_CYLINDER) {
     float wx = px - pr.e0[0], wy = py - pr.e0[1], wz = pz - pr.e0[2];
     float apar = wx * pr.ax[0] + wy * pr.ax[1] + wz * pr.ax[2];
@@ -1185,14 +1231,7 @@ MD bool prim_contains(const DevScene& S, const MONSEL_CS DPrim& pr, float px, fl
   if (pr.kind == PRIM_PLANES) {
     /* MultiPlaneShape.cu:23-27 for every plane */
     bool in = true;
-    const int n = pr.n_planes;
-#pragma unroll
-    for (int k = 0; k < kInlinePlanes; ++k)
-      if (k < n) in = in & (pr.pl[k].x * px + pr.pl[k].y * py + pr.pl[k].z * pz - pr.pl[k].w <= 0.f);
-    for (int k = kInlinePlanes; k < n; ++k) {
-      const float4 pl = S.planes[pr.first_plane + k];
-      in = in & (pl.x * px + pl.y * py + pl.z * pz - pl.w <= 0.f);
-    }
+    for_planes(S, pr, [&](const float4& pl, int) { in = in & (pl.x * px + pl.y * py + pl.z * pz - pl.w <= 0.f); });
     return in;
   }
   float wx = px - pr.e0[0], wy = py - pr.e0[1], wz = pz - pr.e0[2];
@@ -1205,7 +1244,13 @@ MD bool prim_contains(const DevScene& S, const MONSEL_CS DPrim& pr, float px, fl
   return wx * wx + wy * wy + wz * wz <= pr.r2;
 }
 
-MD bool truth(const MONSEL_CS DShape& sh, uint32_t bits) { return (sh.truth[bits >> 5] >> (bits & 31u)) & 1u; }
+/* the shape's truth value for the primitives' inside bits; a shape of at most
+ * five primitives has its table in one (scalar) word */
+MD bool truth(const MONSEL_CS DShape& sh, uint32_t bits) {
+  uint32_t word = sh.truth[0];
+  if (sh.n_prims > 5) word = sh.truth[bits >> 5];
+  return (word >> (bits & 31u)) & 1u;
+}
 
 /* max_k g_k over a convex primitive's constraints, g_k the signed distance
  * to constraint k (plane rows scaled by sdscale <= 1/|n|): <= 0 inside.
@@ -1221,16 +1266,11 @@ MD float prim_gmax_in(const DevScene& S, const MONSEL_CS DPrim& pr, float px, fl
   if (pr.kind == PRIM_PLANES) {
     float g = -kInf;
     bool all = true;
-    auto row = [&](const float4& pl) {
+    for_planes(S, pr, [&](const float4& pl, int) {
       const float v = pl.x * px + pl.y * py + pl.z * pz - pl.w;
       g = fmaxf(g, v);
       all = all & (v <= 0.f);
-    };
-    const int n = pr.n_planes;
-#pragma unroll
-    for (int k = 0; k < kInlinePlanes; ++k)
-      if (k < n) row(pr.pl[k]);
-    for (int k = kInlinePlanes; k < n; ++k) row(S.planes[pr.first_plane + k]);
+    });
     in = all;
     return g * pr.sdscale;
   }
@@ -1367,9 +1407,9 @@ MD int descend(const DevScene& S, int r, float px, float py, float pz) {
     by_value(open, r, [&](int r0) {
       const MONSEL_CS DRegion& rg = S.regions[r0];
       for (int c = 0; c < rg.n_children; ++c) {
-        const int ch = S.children[rg.first_child + c];
-        const bool in = shape_contains(S, S.regions[ch].sh, px, py, pz);
-        if (next < 0 && in) next = ch;
+        const MONSEL_CS DShape& ch = S.children[rg.first_child + c];
+        const bool in = shape_contains(S, ch, px, py, pz);
+        next = (next < 0) & in ? ch.region : next;
       }
     });
     open = open && next >= 0;
@@ -1485,7 +1525,7 @@ MD float region_safety(const DevScene& S, int r, float px, float py, float pz) {
   if (!inside) return 0.f;
   for (int c = 0; c < rg.n_children; ++c) {
     bool in_child;
-    d = fminf(d, shape_safety(S, S.regions[S.children[rg.first_child + c]].sh, px, py, pz, in_child));
+    d = fminf(d, shape_safety(S, S.children[rg.first_child + c], px, py, pz, in_child));
   }
   return d;
 }
@@ -1518,8 +1558,9 @@ MD StepEnd find_end_of_step(const DevScene& S, int r, float px, float py, float 
   /* c = -1: the region's own shape; c >= 0: its children, each limited to
    * the nearest crossing found so far */
   for (int c = -1; c < rg.n_children; ++c) {
-    const int reg = c < 0 ? r : S.children[rg.first_child + c];
-    ShapeHit h = shape_first(S, S.regions[reg].sh, px, py, pz, dx, dy, dz, c < 0 ? s : fminf(s, t), want_normal);
+    const MONSEL_CS DShape& sh = c < 0 ? rg.sh : S.children[rg.first_child + c];
+    const int reg = c < 0 ? r : sh.region;
+    ShapeHit h = shape_first(S, sh, px, py, pz, dx, dy, dz, c < 0 ? s : fminf(s, t), want_normal);
     if (c < 0) {
       se.ownNx = se.winNx = h.nx;
       se.ownNy = se.winNy = h.ny;
