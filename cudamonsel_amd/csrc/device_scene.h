@@ -168,12 +168,35 @@ struct DRegion {
   DShape sh;
 };
 
+/* One axis of a non-uniform table.  The search words (DevScene::nu_words) hold
+ * its abscissae (FP64), a guide -- for each bucket of the map below the
+ * interval bounds {lo, hi} a point of that bucket lies in -- and for each
+ * interval the first point of its cubic window; nu_recs holds a DNUWindow for
+ * each interval.  Interval i is between points i and i + 1, i = -1 .. n - 1. */
+struct DNUAxis {
+  double origin, scale; /* bucket = clamp((v - origin) * scale, 0, last) */
+  double last;
+  int log;              /* v: the high word of x instead of x */
+  int n;
+  int x, guide, first;  /* offsets in nu_words: point 0, bucket 0, interval 0 */
+  int rec;              /* offset in nu_recs of interval 0 */
+  int asc;              /* ascending: bit 0 in FP64, bit 1 rounded to FP32 */
+  int pad;
+};
+
+/* The x-independent part of the four Lagrange weights over a cubic window. */
+struct DNUWindow {
+  double x[4];
+  double den[4], rden[4]; /* products of differences in units of the span, and 1 / den */
+  double inv;             /* 1 / span */
+  double pad[3];
+};
+
 /* Non-uniform table (NUTableInterpolation) in the file's own units. */
 struct DNUTable {
+  DNUAxis axis[4];
   int dim;
-  int n[4];
-  int xoff[4];  /* offsets of the abscissae in nu_data */
-  int voff;     /* offset of the values */
+  int voff;     /* offset of the values, in nu_data (FP32) of a 1-D table, else in nu_data64 */
   int pad[2];
 };
 
@@ -195,7 +218,10 @@ struct DevScene {
   const MONSEL_CS float* mott_x1;    /* [n_mott][61*201] */
   const MONSEL_CS DNUTable* nu;
   const MONSEL_CS float* nu_data;
-  const MONSEL_CS double* nu_data64; /* the same values and abscissae in FP64 */
+  const MONSEL_CS double* nu_data64;
+  const MONSEL_CS unsigned long long* nu_words; /* see DNUAxis */
+  const MONSEL_CS DNUWindow* nu_recs;
+  int n_nu_words;
 };
 
 }  // namespace monsel_dev

@@ -815,9 +815,11 @@ __device__ __forceinline__ const MONSEL_CS TransportArgs* launch_args() {
  * here, so the SIMD's throughput comes from its waves.  Without the tabulated
  * mechanism 5 (96 registers, 56 B of spills): 64 x 64 hole image 106.7 ms, 4:
  * 117.0 ms, 256 x 256 image 816 and 897 ms; 6 (80 registers, more spills) is
- * no faster.  The tabulated mechanism's FP64 scatter keeps that kernel at 4. */
+ * no faster.  With it, whose FP64 scatter holds windows and rows, 3 (168
+ * registers): transport of 400000 primaries of 1 keV in Si 53 ms, 4: 69 ms,
+ * 2: 63 ms; of 40000 of 5 keV in Cu 14.7, 16.5 and 16.3 ms. */
 #ifndef MONSEL_TRANSPORT_WAVES_TAB
-#define MONSEL_TRANSPORT_WAVES_TAB 4
+#define MONSEL_TRANSPORT_WAVES_TAB 3
 #endif
 #ifndef MONSEL_TRANSPORT_WAVES_PER_EU
 #define MONSEL_TRANSPORT_WAVES_PER_EU 5
@@ -842,7 +844,7 @@ k_transport(TransportArgs args) {
   const int tail_lanes = args.G.tail_lanes, regroup = args.G.steps_per_launch;
   const JobRec* jobs = args.G.jobs;
   st.path = 0u;
-  stage_mott_sigma(S);
+  stage_tables<TAB>(S);
   PT_INIT();
   for (;;) {
     PT_BEGIN(t_cl);
@@ -1386,7 +1388,7 @@ __global__ void k_pixels_to_double(const unsigned long long* px, int np, double*
 /* ---- probe kernels ---------------------------------------------------- */
 
 __global__ void k_probe_rates(DevScene S, int msm, int n, const float* E, float* out) {
-  stage_mott_sigma(S);
+  stage_tables<true>(S);
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const MONSEL_CS DMSM& m = S.msms[msm];
@@ -1421,7 +1423,7 @@ __global__ void k_probe_elastic(DevScene S, int mech, int element, int n, const 
  * E, secondary dir (3), trapped flag, 0. */
 __global__ void k_probe_scatter(DevScene S, int mech, int n, const float* prevE, const float* E, const float* dir,
                                 const float* u, float* out) {
-  stage_mott_sigma(S);
+  stage_tables<true>(S);
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const MONSEL_CS DMech& m = S.mechs[mech];
@@ -1544,6 +1546,7 @@ __global__ void k_probe_primaries(DevScene S, const JobRec* J, int n, float* out
 }
 
 __global__ void k_probe_nu(DevScene S, int table, int order, int n, const float* x, float* out) {
+  stage_tables<true>(S);
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int dim = S.nu[table].dim;
@@ -1651,6 +1654,8 @@ struct HostScene {
   std::vector<DNUTable> nu;
   std::vector<float> nudata;
   std::vector<double> nudata64;
+  std::vector<unsigned long long> nuwords;
+  std::vector<DNUWindow> nurecs;
   uint32_t compat = 0;
   /* bound on tracked secondaries per eV of primary energy (queue reservation) */
   double secondaries_per_eV = 0.;
@@ -1808,6 +1813,106 @@ bool eval_tree(const monsel_scene_desc* d, int s, const std::vector<int>& leaves
   return (bits >> k) & 1u;
 }
 
+/* nu_locate's cubic window of the interval `lo` (NULagrangeInterpolation.cu:5-68) */
+int cubic_window(const double* xs, int n, int lo) {
+  const int order = 3, maxindex = n - 1;
+  if (n <= order || lo < 0) return 0;
+  if (lo + 1 > maxindex) return maxindex - order;
+  const bool asc = xs[maxindex] > xs[0];
+  int first = lo, last = lo + 1;
+  while (last - first < order && first > 0 && last < maxindex) {
+    if ((((xs[lo] - xs[first - 1]) + xs[lo + 1]) - xs[last + 1] >= 0.) == asc) ++last;
+    else --first;
+  }
+  if (last >= maxindex) return maxindex - order;
+  return first <= 0 ? 0 : first;
+}
+
+/* An axis's search words and windows.  The guide maps x linearly, or by the
+ * high word of its bits (about its logarithm) for a positive axis, whichever
+ * leaves the fewer points in the fullest bucket; a bucket's bounds hold for x
+ * compared with the points in FP64 and rounded to FP32.  An axis that is not
+ * ascending gets one bucket, from which the search bisects as the reference
+ * does. */
+DNUAxis compile_axis(HostScene& H, const double* xs, int n) {
+  DNUAxis a;
+  memset(&a, 0, sizeof(a));
+  auto f32 = [](double v) {
+    const float f = (float)v;
+    return fabsf(f) < 1.17549435e-38f ? 0.f : f;
+  };
+  a.n = n;
+  a.asc = (xs[n - 1] > xs[0] ? 1 : 0) | (f32(xs[n - 1]) > f32(xs[0]) ? 2 : 0);
+  bool sorted = true;
+  for (int i = 0; i < n; ++i) sorted = sorted && std::isfinite(xs[i]) && (i == 0 || xs[i] > xs[i - 1]);
+  std::vector<std::array<int, 2>> bounds(1, {-1, n});
+  if (sorted && std::isfinite(f32(xs[0])) && std::isfinite(f32(xs[n - 1]))) {
+    auto value = [](int log, double x) {
+      if (!log) return x;
+      uint64_t b;
+      memcpy(&b, &x, sizeof(b));
+      return (double)(int32_t)(uint32_t)(b >> 32);
+    };
+    const int last = 2 * n - 1;
+    int best = n + 1;
+    for (int log = 0; log < (xs[0] > 0. ? 2 : 1); ++log) {
+      const double origin = value(log, xs[0]), scale = last / (value(log, xs[n - 1]) - origin);
+      if (!std::isfinite(scale)) continue;
+      auto bucket = [&](double x) {
+        return (int)std::min(std::max((value(log, x) - origin) * scale, 0.), (double)last);
+      };
+      std::vector<std::array<int, 2>> b((size_t)last + 1, {-1, n});
+      for (int i = 0; i < n; ++i) {
+        const int h0 = bucket(xs[i]), h1 = bucket((double)f32(xs[i]));
+        /* point i is below every x of the buckets above, above every x of those below */
+        if (std::max(h0, h1) < last) b[std::max(h0, h1) + 1][0] = i;
+        if (std::min(h0, h1) > 0) b[std::min(h0, h1) - 1][1] = std::min(b[std::min(h0, h1) - 1][1], i);
+      }
+      int widest = 0;
+      for (int k = 1; k <= last; ++k) b[k][0] = std::max(b[k][0], b[k - 1][0]);
+      for (int k = last - 1; k >= 0; --k) b[k][1] = std::min(b[k][1], b[k + 1][1]);
+      for (auto& w : b) widest = std::max(widest, w[1] - w[0]);
+      if (widest < best) {
+        best = widest;
+        bounds.swap(b);
+        a.log = log;
+        a.origin = origin;
+        a.scale = scale;
+        a.last = last;
+      }
+    }
+  }
+  a.x = (int)H.nuwords.size();
+  for (int i = 0; i < n; ++i) {
+    unsigned long long w;
+    memcpy(&w, &xs[i], sizeof(w));
+    H.nuwords.push_back(w);
+  }
+  a.guide = (int)H.nuwords.size();
+  for (auto& w : bounds) H.nuwords.push_back((unsigned int)w[0] | (unsigned long long)(unsigned int)w[1] << 32);
+  a.first = (int)H.nuwords.size() + 1;
+  a.rec = (int)H.nurecs.size() + 1;
+  for (int lo = -1; lo < n; ++lo) {
+    const int f = cubic_window(xs, n, lo);
+    H.nuwords.push_back((unsigned long long)f);
+    if (n < 4) continue;
+    /* the arithmetic of nu_weights<double, 3> */
+    DNUWindow r;
+    memset(&r, 0, sizeof(r));
+    for (int i = 0; i < 4; ++i) r.x[i] = xs[f + i];
+    r.inv = 1. / (r.x[3] - r.x[0]);
+    for (int i = 0; i < 4; ++i) {
+      double den = 1.;
+      for (int j = 0; j < 4; ++j)
+        if (j != i) den *= (r.x[i] - r.x[j]) * r.inv;
+      r.den[i] = den;
+      r.rden[i] = 1. / den;
+    }
+    H.nurecs.push_back(r);
+  }
+  return a;
+}
+
 HostScene compile_scene(const monsel_scene_desc* d) {
   if (!d || d->abi_version != MONSEL_ABI_VERSION) throw MonselError(MONSEL_E_INVALID, "bad scene descriptor or ABI version");
   if (d->n_regions < 1 || !d->regions) throw MonselError(MONSEL_E_INVALID, "scene has no regions");
@@ -1834,20 +1939,16 @@ HostScene compile_scene(const monsel_scene_desc* d) {
     size_t tot = 1;
     for (int k = 0; k < t.dim; ++k) {
       if (t.n[k] < 2) throw MonselError(MONSEL_E_INVALID, "NU table axis too short");
-      dt.n[k] = t.n[k];
-      dt.xoff[k] = (int)H.nudata.size();
-      for (int j = 0; j < t.n[k]; ++j) {
-        H.nudata.push_back((float)t.x[k][j]);
-        H.nudata64.push_back(t.x[k][j]);
-      }
+      dt.axis[k] = compile_axis(H, t.x[k], t.n[k]);
       tot *= (size_t)t.n[k];
     }
-    dt.voff = (int)H.nudata.size();
+    /* looked up in FP32 in one dimension, in FP64 otherwise */
+    dt.voff = t.dim == 1 ? (int)H.nudata.size() : (int)H.nudata64.size();
     double r0 = INFINITY, r1 = -INFINITY;
     for (size_t j = 0; j < tot; ++j) {
       double v = t.values[j];
-      H.nudata.push_back((float)v);
-      H.nudata64.push_back(v);
+      if (t.dim == 1) H.nudata.push_back((float)v);
+      else H.nudata64.push_back(v);
       /* NUTableInterpolation.cu:169-172 */
       if (v < r0) r0 = v;
       else if (v > r1) r1 = v;
@@ -2166,6 +2267,8 @@ size_t host_scene_bytes(const HostScene& H) {
   add(H.nu.size() * sizeof(DNUTable));
   add(H.nudata.size() * sizeof(float));
   add(H.nudata64.size() * sizeof(double));
+  add(H.nuwords.size() * sizeof(unsigned long long));
+  add(H.nurecs.size() * sizeof(DNUWindow));
   return total;
 }
 
@@ -2175,7 +2278,7 @@ void upload_scene(const HostScene& H, SceneDev& sd) {
   size_t o_pr = append(blob, H.prims), o_pl = append(blob, H.planes), o_msm = append(blob, H.msms);
   size_t o_me = append(blob, H.mechs), o_el = append(blob, H.elems), o_sp = append(blob, H.spwem);
   size_t o_x1 = append(blob, H.x1), o_nu = append(blob, H.nu), o_nd = append(blob, H.nudata);
-  size_t o_nd64 = append(blob, H.nudata64);
+  size_t o_nd64 = append(blob, H.nudata64), o_nw = append(blob, H.nuwords), o_nr = append(blob, H.nurecs);
   sd.blob.ensure(blob.size() + 256);
   HIP_TRY(hipMemcpy(sd.blob.p, blob.data(), blob.size(), hipMemcpyHostToDevice));
   char* b = sd.blob.as<char>();
@@ -2208,6 +2311,9 @@ void upload_scene(const HostScene& H, SceneDev& sd) {
   S.nu = (decltype(S.nu))(b + o_nu);
   S.nu_data = (decltype(S.nu_data))(b + o_nd);
   S.nu_data64 = (decltype(S.nu_data64))(b + o_nd64);
+  S.nu_words = (decltype(S.nu_words))(b + o_nw);
+  S.nu_recs = (decltype(S.nu_recs))(b + o_nr);
+  S.n_nu_words = (int)H.nuwords.size();
   sd.bytes = blob.size();
   sd.step_cost = max_step_cost(H);
 }
@@ -2224,7 +2330,8 @@ HostScene merge_scenes(const std::vector<const HostScene*>& parts, std::vector<i
     const int o_reg = (int)M.regions.size(), o_ch = (int)M.children.size(), o_sh = (int)M.shapes.size();
     const int o_pr = (int)M.prims.size(), o_pl = (int)M.planes.size(), o_msm = (int)M.msms.size();
     const int o_me = (int)M.mechs.size(), o_el = (int)M.elems.size(), o_mott = (int)(M.spwem.size() / kMottNE);
-    const int o_nu = (int)M.nu.size(), o_nd = (int)M.nudata.size();
+    const int o_nu = (int)M.nu.size(), o_nd = (int)M.nudata.size(), o_nd64 = (int)M.nudata64.size();
+    const int o_nw = (int)M.nuwords.size(), o_nr = (int)M.nurecs.size();
     roots.push_back(o_reg);
     for (DRegion r : P->regions) {
       if (r.parent >= 0) r.parent += o_reg;
@@ -2268,12 +2375,19 @@ HostScene merge_scenes(const std::vector<const HostScene*>& parts, std::vector<i
     M.spwem.insert(M.spwem.end(), P->spwem.begin(), P->spwem.end());
     M.x1.insert(M.x1.end(), P->x1.begin(), P->x1.end());
     for (DNUTable t : P->nu) {
-      for (int k = 0; k < t.dim; ++k) t.xoff[k] += o_nd;
-      t.voff += o_nd;
+      for (int k = 0; k < t.dim; ++k) {
+        t.axis[k].x += o_nw;
+        t.axis[k].guide += o_nw;
+        t.axis[k].first += o_nw;
+        t.axis[k].rec += o_nr;
+      }
+      t.voff += t.dim == 1 ? o_nd : o_nd64;
       M.nu.push_back(t);
     }
     M.nudata.insert(M.nudata.end(), P->nudata.begin(), P->nudata.end());
     M.nudata64.insert(M.nudata64.end(), P->nudata64.begin(), P->nudata64.end());
+    M.nuwords.insert(M.nuwords.end(), P->nuwords.begin(), P->nuwords.end());
+    M.nurecs.insert(M.nurecs.end(), P->nurecs.begin(), P->nurecs.end());
     M.compat = P->compat;
     M.chamber_r = std::max(M.chamber_r, P->chamber_r);
   }
@@ -3706,7 +3820,7 @@ int monsel_probe_nu_table(monsel_ctx ctx, monsel_scene_id scene, int table, int 
     DNUTable t;
     HIP_TRY(hipMemcpy(&t, sd->dev.nu + table, sizeof(DNUTable), hipMemcpyDeviceToHost));
     for (int k = 0; k < t.dim; ++k)
-      if (t.n[k] < order + 1) throw MonselError(MONSEL_E_INVALID, "table axis shorter than order + 1");
+      if (t.axis[k].n < order + 1) throw MonselError(MONSEL_E_INVALID, "table axis shorter than order + 1");
     Scratch<float> dX((size_t)n * t.dim), dO(n);
     HIP_TRY(hipMemcpy(dX.d, x, 4 * (size_t)n * t.dim, hipMemcpyHostToDevice));
     hipLaunchKernelGGL(k_probe_nu, dim3(grid_for(n)), dim3(256), 0, 0, sd->dev, table, order, n, dX.d, dO.d);

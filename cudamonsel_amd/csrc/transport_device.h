@@ -261,7 +261,7 @@ MD float rutherford_cos(float rz23, float EeV, float r) {
 /* The hot tables: the cross-section nodes (Spwem, 61 floats) of the first
  * kLdsMott NIST Mott elements of a scene, which every step above 50 eV reads
  * for every element of its material, live in LDS; each kernel that evaluates
- * cross-sections copies them there at its start (stage_mott_sigma).  The
+ * cross-sections copies them there at its start (stage_tables).  The
  * angle tables (61 x 201 per element, read once per elastic event) stay in
  * device memory. */
 #ifndef MONSEL_LDS_MOTT_TABLES
@@ -272,11 +272,24 @@ MD float* lds_spwem() {
   __shared__ float l_spwem[(kLdsMott > 0 ? kLdsMott : 1) * kMottNE];
   return l_spwem;
 }
-/* every thread of the block calls it before any cross-section */
-MD void stage_mott_sigma(const DevScene& S) {
+/* The search words of the inelastic tables (abscissae, guides and windows;
+ * some 11 KB for a four-table set), in LDS as well where they fit. */
+constexpr int kLdsNuWords = 1792;
+MD unsigned long long* lds_nu_words() {
+  __shared__ unsigned long long l_nu_words[kLdsNuWords];
+  return l_nu_words;
+}
+/* every thread of the block calls it before any cross-section (TAB: or
+ * inelastic table) */
+template <bool TAB>
+MD void stage_tables(const DevScene& S) {
   const int n = min(S.n_mott, kLdsMott) * kMottNE;
   float* l = lds_spwem();
   for (int i = threadIdx.x; i < n; i += blockDim.x) l[i] = S.mott_spwem[i];
+  if constexpr (TAB) {
+    if (S.n_nu_words <= kLdsNuWords)
+      for (int i = threadIdx.x; i < S.n_nu_words; i += blockDim.x) lds_nu_words()[i] = S.nu_words[i];
+  }
   __syncthreads();
 }
 
@@ -536,23 +549,26 @@ MD const float* nu_base<float>(const DevScene& S) { return S.nu_data; }
 template <>
 MD const double* nu_base<double>(const DevScene& S) { return S.nu_data64; }
 
+MD const double* nu_axis(const DevScene& S, const MONSEL_CS DNUAxis& a) { return (const double*)(S.nu_words + a.x); }
+
 /* NULagrangeInterpolation::locate (NULagrangeInterpolation.cu:5-68) on an
  * ascending or descending grid: first index of the order+1 window. */
 template <typename T>
-MD int nu_locate(const T* xs, int n, int order, T x) {
+MD int nu_locate(const double* xs64, int n, int order, T x) {
+  const auto xs = [=](int i) { return (T)xs64[i]; };
   int lowlim = -1, uplim = n, maxindex = n - 1;
-  bool asc = xs[maxindex] > xs[0];
+  bool asc = xs(maxindex) > xs(0);
   while (uplim - lowlim > 1) {
     int mid = (uplim + lowlim) >> 1;
-    if ((x > xs[mid]) == asc) lowlim = mid;
+    if ((x > xs(mid)) == asc) lowlim = mid;
     else uplim = mid;
   }
   if (lowlim < 0) return 0;
   if (uplim > maxindex) return maxindex - order;
-  T xl = xs[lowlim], xu = xs[uplim];
+  T xl = xs(lowlim), xu = xs(uplim);
   int first = lowlim, last = uplim;
   while ((last - first) < order && first > 0 && last < maxindex) {
-    if ((((xl - xs[first - 1]) + xu) - xs[last + 1] >= (T)0) == asc) last += 1;
+    if ((((xl - xs(first - 1)) + xu) - xs(last + 1) >= (T)0) == asc) last += 1;
     else first -= 1;
   }
   if (last >= maxindex) return maxindex - order;
@@ -565,13 +581,13 @@ MD int nu_locate(const T* xs, int n, int order, T x) {
  * (NULagrangeInterpolation.cu:85-112) evaluates.  Weights are formed once
  * per axis and shared by every row of a multi-dimensional window. */
 template <typename T, int ORDER>
-MD void nu_weights(const T* xs, T x, T* w) {
+MD void nu_weights(const double* xs, T x, T* w) {
   /* differences are taken in units of the window's span, so that products
    * of ORDER of them stay far from underflow whatever the grid's units
    * (energies in J are ~1e-17) */
   T xv[ORDER + 1];
 #pragma unroll
-  for (int i = 0; i <= ORDER; ++i) xv[i] = xs[i];
+  for (int i = 0; i <= ORDER; ++i) xv[i] = (T)xs[i];
   const T inv = (T)1 / (xv[ORDER] - xv[0]);
 #pragma unroll
   for (int i = 0; i <= ORDER; ++i) {
@@ -595,7 +611,7 @@ MD T nu_dot(const T* w, const T* f) {
 }
 
 template <typename T, int ORDER>
-MD T nu_poly(const T* xs, const T* f, T x) {
+MD T nu_poly(const double* xs, const T* f, T x) {
   T w[ORDER + 1];
   nu_weights<T, ORDER>(xs, x, w);
   return nu_dot<T, ORDER>(w, f);
@@ -605,8 +621,8 @@ MD T nu_poly(const T* xs, const T* f, T x) {
 template <typename T, int ORDER>
 MD T nu_d1(const DevScene& S, const MONSEL_CS DNUTable& t, T x0) {
   const T* d = nu_base<T>(S);
-  const T* xa = d + t.xoff[0];
-  int i0 = nu_locate<T>(xa, t.n[0], ORDER, x0);
+  const double* xa = nu_axis(S, t.axis[0]);
+  int i0 = nu_locate<T>(xa, t.axis[0].n, ORDER, x0);
   return nu_poly<T, ORDER>(xa + i0, d + t.voff + i0, x0);
 }
 
@@ -614,11 +630,11 @@ MD T nu_d1(const DevScene& S, const MONSEL_CS DNUTable& t, T x0) {
 template <typename T, int ORDER>
 MD T nu_d2(const DevScene& S, const MONSEL_CS DNUTable& t, T x0, T x1) {
   const T* d = nu_base<T>(S);
-  const T* xa = d + t.xoff[0];
-  const T* xb = d + t.xoff[1];
+  const double* xa = nu_axis(S, t.axis[0]);
+  const double* xb = nu_axis(S, t.axis[1]);
   const T* f = d + t.voff;
-  const int nb = t.n[1];
-  int i0 = nu_locate<T>(xa, t.n[0], ORDER, x0);
+  const int nb = t.axis[1].n;
+  int i0 = nu_locate<T>(xa, t.axis[0].n, ORDER, x0);
   int j0 = nu_locate<T>(xb, nb, ORDER, x1);
   T wb[ORDER + 1], y[ORDER + 1];
   nu_weights<T, ORDER>(xb + j0, x1, wb);
@@ -633,12 +649,12 @@ MD T nu_d2(const DevScene& S, const MONSEL_CS DNUTable& t, T x0, T x1) {
 template <typename T, int ORDER>
 MD T nu_d3(const DevScene& S, const MONSEL_CS DNUTable& t, int ax, int voff, T x0, T x1, T x2, bool compat_d3) {
   const T* d = nu_base<T>(S);
-  const T* xa = d + t.xoff[ax];
-  const T* xb = d + t.xoff[ax + 1];
-  const T* xc = d + t.xoff[ax + 2];
+  const double* xa = nu_axis(S, t.axis[ax]);
+  const double* xb = nu_axis(S, t.axis[ax + 1]);
+  const double* xc = nu_axis(S, t.axis[ax + 2]);
   const T* v = d + voff;
-  const int nb = t.n[ax + 1], nc = t.n[ax + 2];
-  int i0 = nu_locate<T>(xa, t.n[ax], ORDER, x0);
+  const int nb = t.axis[ax + 1].n, nc = t.axis[ax + 2].n;
+  int i0 = nu_locate<T>(xa, t.axis[ax].n, ORDER, x0);
   int j0 = nu_locate<T>(xb, nb, ORDER, x1);
   int k0 = nu_locate<T>(xc, nc, ORDER, x2);
   T wb[ORDER + 1], wc[ORDER + 1], y[ORDER + 1];
@@ -666,12 +682,12 @@ MD T nu_d3(const DevScene& S, const MONSEL_CS DNUTable& t, int ax, int voff, T x
 /* NULagrangeInterpolation::d4 (:259-306). */
 template <typename T, int ORDER>
 MD T nu_d4(const DevScene& S, const MONSEL_CS DNUTable& t, const T* x, bool compat_d3) {
-  const T* xa = nu_base<T>(S) + t.xoff[0];
-  int i0 = nu_locate<T>(xa, t.n[0], ORDER, x[0]);
+  const double* xa = nu_axis(S, t.axis[0]);
+  int i0 = nu_locate<T>(xa, t.axis[0].n, ORDER, x[0]);
   T y[ORDER + 1];
 #pragma unroll
   for (int i = 0; i <= ORDER; ++i)
-    y[i] = nu_d3<T, ORDER>(S, t, 1, t.voff + (i0 + i) * t.n[1] * t.n[2] * t.n[3], x[1], x[2], x[3], compat_d3);
+    y[i] = nu_d3<T, ORDER>(S, t, 1, t.voff + (i0 + i) * t.axis[1].n * t.axis[2].n * t.axis[3].n, x[1], x[2], x[3], compat_d3);
   return nu_poly<T, ORDER>(xa + i0, y, x[0]);
 }
 
@@ -687,13 +703,156 @@ MD T nu_interp_o(const DevScene& S, int table, const T* x, bool compat_d3) {
   return 0;
 }
 
+/* The lookups of the transport step: FP64 cubic in two and three dimensions,
+ * FP32 linear in one, with the bits of nu_d2, nu_d3 and nu_d1 above.  Through
+ * those, an axis took a bisection of seven dependent reads of device memory
+ * and four more for the window, and a window nine double divisions; tabulated
+ * scatter was 55 to 65 % of a step with it, and a bulk run of few primaries is
+ * a chain of steps.  Here the axes of a lookup are searched together, in LDS,
+ * from the bounds their guides give (mostly one probe each), the window of an
+ * interval is a word beside them, and what the weights hold of the axis alone
+ * comes in a DNUWindow.  Transport of 3001 primaries of 5 keV in Cu: 8.7 ms to
+ * 5.9 ms; of 400000 of 1 keV in Si 53 ms. */
+template <typename T, int A, class P>
+MD void nu_search(P w, const MONSEL_CS DNUAxis* ax, const T* x, int* lo, int* first) {
+  int up[A];
+  bool more = false;
+#pragma unroll
+  for (int k = 0; k < A; ++k) {
+    const double xk = (double)x[k];
+    const double v = ax[k].log ? (double)__double2hiint(xk) : xk;
+    const double h = fmin(fmax((v - ax[k].origin) * ax[k].scale, 0.), ax[k].last);
+    const unsigned long long g = w[ax[k].guide + (xk == xk ? (int)h : 0)];
+    lo[k] = (int)(unsigned int)g;
+    up[k] = (int)(unsigned int)(g >> 32);
+    more |= up[k] - lo[k] > 1;
+  }
+  bool asc[A];
+#pragma unroll
+  for (int k = 0; k < A; ++k) asc[k] = (ax[k].asc & (sizeof(T) == 8 ? 1 : 2)) != 0;
+  while (more) {
+    more = false;
+#pragma unroll
+    for (int k = 0; k < A; ++k) {
+      const int mid = (up[k] + lo[k]) >> 1;
+      const T xm = (T)__longlong_as_double((long long)w[ax[k].x + max(mid, 0)]);
+      const bool above = (x[k] > xm) == asc[k], open = up[k] - lo[k] > 1;
+      lo[k] = (open & above) ? mid : lo[k];
+      up[k] = (open & !above) ? mid : up[k];
+      more |= up[k] - lo[k] > 1;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < A; ++k) first[k] = (int)w[ax[k].first + lo[k]];
+}
+
+template <int A>
+MD void nu_find(const DevScene& S, const MONSEL_CS DNUAxis* ax, const double* x, int* lo, int* first) {
+  if (S.n_nu_words <= kLdsNuWords)
+    nu_search<double, A>((const unsigned long long*)lds_nu_words(), ax, x, lo, first);
+  else
+    nu_search<double, A>(S.nu_words, ax, x, lo, first);
+}
+
+/* num / den, correctly rounded, from y = 1 / den correctly rounded (Markstein:
+ * a quotient within one unit and its exact remainder; the first correction
+ * brings the product within that unit, the second rounds it) */
+MD double nu_quotient(double num, double den, double y) {
+  double q = num * y;
+  q = __builtin_fma(__builtin_fma(-den, q, num), y, q);
+  q = __builtin_fma(__builtin_fma(-den, q, num), y, q);
+  return __builtin_amdgcn_div_fixup(q, den, num);
+}
+
+/* nu_weights<double, 3> over the window of a record */
+MD void nu_cubic_weights(const MONSEL_CS DNUWindow& r, double x, double* w) {
+  double d[4], den[4], rden[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    d[j] = (x - r.x[j]) * r.inv;
+    den[j] = r.den[j];
+    rden[j] = r.rden[j];
+  }
+  w[0] = nu_quotient((d[1] * d[2]) * d[3], den[0], rden[0]);
+  w[1] = nu_quotient((d[0] * d[2]) * d[3], den[1], rden[1]);
+  w[2] = nu_quotient((d[0] * d[1]) * d[3], den[2], rden[2]);
+  w[3] = nu_quotient((d[0] * d[1]) * d[2], den[3], rden[3]);
+}
+
+MD double nu_cubic2(const DevScene& S, const MONSEL_CS DNUTable& t, double x0, double x1) {
+  const MONSEL_CS DNUAxis* ax = t.axis;
+  const double x[2] = {x0, x1};
+  int lo[2], first[2];
+  nu_find<2>(S, ax, x, lo, first);
+  const int nb = ax[1].n;
+  const MONSEL_CS double* f = S.nu_data64 + t.voff + (size_t)first[0] * nb + first[1];
+  double v[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[i][j] = f[(size_t)i * nb + j];
+  double wa[4], wb[4], y[4];
+  nu_cubic_weights(S.nu_recs[ax[1].rec + lo[1]], x1, wb);
+  nu_cubic_weights(S.nu_recs[ax[0].rec + lo[0]], x0, wa);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y[i] = nu_dot<double, 3>(wb, v[i]);
+  return nu_dot<double, 3>(wa, y);
+}
+
+MD double nu_cubic3(const DevScene& S, const MONSEL_CS DNUTable& t, double x0, double x1, double x2, bool compat_d3) {
+  const MONSEL_CS DNUAxis* ax = t.axis;
+  const double x[3] = {x0, x1, x2};
+  int lo[3], first[3];
+  nu_find<3>(S, ax, x, lo, first);
+  const int nb = ax[1].n, nc = ax[2].n;
+  const MONSEL_CS double* f = S.nu_data64 + t.voff + ((size_t)first[0] * nb + first[1]) * nc + first[2];
+  double wa[4], wb[4], wc[4], y = 0.;
+  nu_cubic_weights(S.nu_recs[ax[2].rec + lo[2]], x2, wc);
+  nu_cubic_weights(S.nu_recs[ax[1].rec + lo[1]], x1, wb);
+  nu_cubic_weights(S.nu_recs[ax[0].rec + (compat_d3 ? -1 : lo[0])], x0, wa);
+  /* one outer point at a time: with the sixteen values of a point, or of two,
+   * loaded together and the windows beside them the registers spill, and
+   * 400000 primaries in Si take 58 ms where these take 53 */
+#pragma unroll 1
+  for (int i = 0; i < 4; ++i) {
+    double z[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      double v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = f[(size_t)j * nc + k];
+      z[j] = nu_dot<double, 3>(wc, v);
+    }
+    y = __builtin_fma(wa[0], nu_dot<double, 3>(wb, z), y);
+    wa[0] = wa[1];
+    wa[1] = wa[2];
+    wa[2] = wa[3];
+    f += (size_t)nb * nc;
+  }
+  return y;
+}
+
+MD float nu_linear1(const DevScene& S, const MONSEL_CS DNUTable& t, float x) {
+  const MONSEL_CS DNUAxis* ax = t.axis;
+  int lo, first;
+  if (S.n_nu_words <= kLdsNuWords)
+    nu_search<float, 1>((const unsigned long long*)lds_nu_words(), ax, &x, &lo, &first);
+  else
+    nu_search<float, 1>(S.nu_words, ax, &x, &lo, &first);
+  const int i0 = min(max(lo, 0), ax->n - 2);
+  return nu_poly<float, 1>(nu_axis(S, *ax) + i0, (const float*)(S.nu_data + t.voff + i0), x);
+}
+
 /* NUTableInterpolation::interpolate (NUTableInterpolation.cu:98-115) in
  * the arithmetic the transport uses for that table's dimension: FP32 for
  * 1-D (mean free path), FP64 otherwise. */
 MD double nu_interp(const DevScene& S, int table, int order, const double* x, bool compat_d3) {
-  if (S.nu[table].dim == 1) {
+  const MONSEL_CS DNUTable& t = S.nu[table];
+  if (order == 3 && t.dim == 2) return nu_cubic2(S, t, x[0], x[1]);
+  if (order == 3 && t.dim == 3) return nu_cubic3(S, t, x[0], x[1], x[2], compat_d3);
+  if (t.dim == 1) {
     const float xf = (float)x[0];
-    if (order == 1) return nu_interp_o<float, 1>(S, table, &xf, compat_d3);
+    if (order == 1) return nu_linear1(S, t, xf);
     if (order == 2) return nu_interp_o<float, 2>(S, table, &xf, compat_d3);
     return nu_interp_o<float, 3>(S, table, &xf, compat_d3);
   }
@@ -744,7 +903,7 @@ MD float mech_rate(const DevScene& S, const MONSEL_CS DMech& m, float EeV) {
     case MONSEL_MECH_TABULATED_INELASTIC: if constexpr (TAB) { /* TabulatedInelasticSM.cu:436-459 */
       float kE = (EeV + m.p[TP_OFFSET]) * kEcharge;
       if (kE < m.p[TP_IIMFPDOM0]) return 0.f;
-      return m.p[TP_RATEMULT] * nu_d1<float, 1>(S, S.nu[m.table[0]], kE) * 1.0e-9f;
+      return m.p[TP_RATEMULT] * nu_linear1(S, S.nu[m.table[0]], kE) * 1.0e-9f;
     }
   }
   return 0.f;
@@ -825,7 +984,7 @@ MD Spawn tabulated_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e,
   const double kE = kE0 + m.q[TP_OFFSET];
   if (kE < m.q[TP_EIDOM0]) return se;
   const double rnd0 = u[2], rnd1 = u[3], rnd2 = u[4], rnd3 = u[5];
-  double deltaE = kE * nu_d2<double, 3>(S, S.nu[m.table[1]], kE, rnd0);
+  double deltaE = kE * nu_cubic2(S, S.nu[m.table[1]], kE, rnd0);
   const double gap = m.q[TP_GAP], bandgap = m.q[TP_BANDGAP];
   if (deltaE < gap && deltaE > 0.95 * gap) deltaE = gap;
   const float d0x = e.dx, d0y = e.dy, d0z = e.dz;
@@ -835,7 +994,7 @@ MD Spawn tabulated_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e,
   if (deltaE >= bandgap) {
     double red = (deltaE - gap) / (kE - offsetFermi - 2. * gap);
     red = red > 1. ? 1. : (red < 0. ? 0. : red);
-    theta = nu_d3<double, 3>(S, S.nu[m.table[2]], 0, S.nu[m.table[2]].voff, kE, red, rnd1, cd3);
+    theta = nu_cubic3(S, S.nu[m.table[2]], kE, red, rnd1, cd3);
     __sincosf(kTwoPI * (float)rnd2, &sphi, &cphi);
     float st, ct;
     sincosf((float)theta, &st, &ct);
@@ -846,84 +1005,67 @@ MD Spawn tabulated_scatter(const DevScene& S, const MONSEL_CS DMech& m, Elec& e,
   const double Eq = (2. * kE) - deltaE - (2. * sqrt(kE * (kE - deltaE)) * (double)cosf((float)theta));
   const double cb = m.q[TP_CB], minEgen = m.q[TP_MINEGEN], bEref = m.q[TP_BEREF];
   const double offset = m.q[TP_OFFSET];
-  double energySE;
   const int method = m.method;
-  /* SE direction relative to the PE's original direction: thetaSE = pi/2 - theta,
-   * phiSE = phi + pi */
-  auto rel_dir = [&](float& sx, float& sy, float& sz) {
-    sx = d0x;
-    sy = d0y;
-    sz = d0z;
-    float st, ct;
-    sincosf((float)(0.5 * 3.14159265358979323846 - theta), &st, &ct);
-    rotate_dir(sx, sy, sz, ct, st, -cphi, -sphi);
-  };
-  auto se0 = [&](double dE) {
-    double e0 = nu_d2<double, 3>(S, S.nu[m.table[3]], dE, rnd3);
+  const double be = pick_be(m, Eq, deltaE);
+  const double root = 2. * sqrt(offsetFermi * (offsetFermi + deltaE));
+  const double sum = (2. * offsetFermi) + deltaE;
+  /* the source of the SE's energy: a bound level, the band (method 3 where the
+   * momentum transfer allows it) or the table; one lookup serves both methods */
+  const bool bound = method == 1 || be > 0.;
+  const bool band = !bound && method == 3 && (sum - root) <= Eq && Eq <= (sum + root);
+  double energySE = (deltaE + bEref) - be;
+  float thSE = 0.f;
+  if (band) {
+    /* simESEf (TabulatedInelasticSM.cu:87-101) */
+    const double q = sqrt(Eq);
+    const double kz = (deltaE - Eq) / 2. / q;
+    const double kzf = kz + q;
+    const double Ezq = kzf * kzf;
+    double minE = (offsetFermi + bandgap) - Ezq;
+    if (minE < 0.) minE = 0.;
+    const double maxE = offsetFermi - (kz * kz);
+    const double Exy = (minE * (1. - rnd3)) + (maxE * rnd3);
+    const double ESEf = Exy + Ezq;
+    thSE = acosf((float)(kzf / sqrt(ESEf)));
+    energySE = ESEf - offset;
+  } else if (!bound) {
+    double e0 = nu_cubic2(S, S.nu[m.table[3]], deltaE, rnd3);
     if (e0 < m.q[TP_SE0RANGE0]) e0 = m.q[TP_SE0RANGE0];
     else if (e0 > m.q[TP_SE0RANGE1]) e0 = m.q[TP_SE0RANGE1];
-    return e0;
-  };
-  if (method == 1) {
-    energySE = (deltaE + bEref) - pick_be(m, Eq, deltaE);
-    if (energySE + cb < minEgen) return se;
-    rel_dir(se.dx, se.dy, se.dz);
-  } else if (method == 2) {
-    const double be = pick_be(m, Eq, deltaE);
-    if (be > 0.) energySE = (deltaE + bEref) - be;
-    else energySE = (deltaE + se0(deltaE)) - offset;
-    if (energySE + cb < minEgen) return se;
-    rel_dir(se.dx, se.dy, se.dz);
+    energySE = (deltaE + e0) - offset;
+  }
+  if (energySE + cb < minEgen) return se;
+  if (method == 3 && !band) {
+    isotropic_dir(u[6], u[7], se.dx, se.dy, se.dz);
   } else {
-    const double be = pick_be(m, Eq, deltaE);
-    if (be > 0.) {
-      energySE = (deltaE + bEref) - be;
-      if (energySE + cb < minEgen) return se;
-      isotropic_dir(u[6], u[7], se.dx, se.dy, se.dz);
-    } else {
-      const double root = 2. * sqrt(offsetFermi * (offsetFermi + deltaE));
-      const double sum = (2. * offsetFermi) + deltaE;
-      if ((sum - root) <= Eq && Eq <= (sum + root)) {
-        /* simESEf (TabulatedInelasticSM.cu:87-101) */
-        const double q = sqrt(Eq);
-        const double kz = (deltaE - Eq) / 2. / q;
-        const double kzf = kz + q;
-        const double Ezq = kzf * kzf;
-        double minE = (offsetFermi + bandgap) - Ezq;
-        if (minE < 0.) minE = 0.;
-        const double maxE = offsetFermi - (kz * kz);
-        const double Exy = (minE * (1. - rnd3)) + (maxE * rnd3);
-        const double ESEf = Exy + Ezq;
-        const float thSE = acosf((float)(kzf / sqrt(ESEf)));
-        energySE = ESEf - offset;
-        if (energySE + cb < minEgen) return se;
-        /* TabulatedInelasticSM.cu:388-395: the q-vector direction (pi/2 - theta,
-         * phi + pi) is deflected by (thSE, 2 pi U) in the PE frame, and the SE
-         * is the PE's original direction rotated by the resulting angles. */
-        float st, ct;
-        sincosf((float)(0.5 * 3.14159265358979323846 - theta), &st, &ct);
-        float wx, wy, wz;
-        dir_from_angles(ct, st, -cphi, -sphi, wx, wy, wz);
-        float sp2, cp2, st2, ct2;
-        __sincosf(kTwoPI * u[6], &sp2, &cp2);
-        sincosf(thSE, &st2, &ct2);
-        rotate_dir(wx, wy, wz, ct2, st2, cp2, sp2);
-        float wst = fsqrt(fmaxf(0.f, wx * wx + wy * wy));
-        float wcp = 1.f, wsp = 0.f;
-        if (wst > 0.f) {
-          wcp = wx / wst;
-          wsp = wy / wst;
-        }
-        se.dx = d0x;
-        se.dy = d0y;
-        se.dz = d0z;
-        rotate_dir(se.dx, se.dy, se.dz, wz, wst, wcp, wsp);
-      } else {
-        energySE = (deltaE + se0(deltaE)) - offset;
-        if (energySE + cb < minEgen) return se;
-        isotropic_dir(u[6], u[7], se.dx, se.dy, se.dz);
+    /* SE direction relative to the PE's original direction: thetaSE = pi/2 -
+     * theta, phiSE = phi + pi */
+    float st, ct, sp = -sphi, cp = -cphi;
+    sincosf((float)(0.5 * 3.14159265358979323846 - theta), &st, &ct);
+    if (band) {
+      /* TabulatedInelasticSM.cu:388-395: the q-vector direction (pi/2 - theta,
+       * phi + pi) is deflected by (thSE, 2 pi U) in the PE frame, and the SE
+       * is the PE's original direction rotated by the resulting angles. */
+      float wx, wy, wz;
+      dir_from_angles(ct, st, cp, sp, wx, wy, wz);
+      float sp2, cp2, st2, ct2;
+      __sincosf(kTwoPI * u[6], &sp2, &cp2);
+      sincosf(thSE, &st2, &ct2);
+      rotate_dir(wx, wy, wz, ct2, st2, cp2, sp2);
+      const float wst = fsqrt(fmaxf(0.f, wx * wx + wy * wy));
+      cp = 1.f;
+      sp = 0.f;
+      if (wst > 0.f) {
+        cp = wx / wst;
+        sp = wy / wst;
       }
+      ct = wz;
+      st = wst;
     }
+    se.dx = d0x;
+    se.dy = d0y;
+    se.dz = d0z;
+    rotate_dir(se.dx, se.dy, se.dz, ct, st, cp, sp);
   }
   se.has = 1u;
   se.E = (float)(energySE / J);

@@ -200,6 +200,67 @@ def test_nu_tables(oracle, tmp_path, M, scale0):
             assert np.max(np.abs(g - o)) / scale < 1e-4
 
 
+@pytest.mark.parametrize("axes", ["log", "linear", "uneven", "descending", "shortest", "long"])
+def test_nu_lookups_on_any_axis(oracle, tmp_path, M, axes):
+    """The lookups of the transport step against the oracle's, on every kind
+    of axis their search distinguishes: mapped by the logarithm or linearly,
+    clustered so that buckets hold many points, descending (no map), of the
+    fewest points a cubic takes, and too long for on-chip memory; at the
+    points themselves, between them and a little outside.
+
+    Tolerances: the FP64 lookups are rounded to FP32 (2^-24 relative) after
+    FP64 rounding of sums whose weights stay below some tens here; the FP32 one
+    rounds the abscissae, 2^-24 of x against an interval, times a value step of
+    at most 1."""
+    from cudamonsel_amd import scenes, tables
+    from cudamonsel_amd.abi import probe_for
+    rng = np.random.default_rng(17)
+
+    def axis(n):
+        if axes == "log":
+            return np.geomspace(1.0, 2000.0, n)
+        if axes == "uneven":
+            return np.sort(np.concatenate([[1.0, 9.0], 2.0 + 0.2 * rng.uniform(0, 1, n - 2)]))
+        g = np.linspace(1.0, 9.0, n)
+        return g[::-1].copy() if axes == "descending" else g
+
+    sizes = dict(shortest=(4, 4, 4), long=(900, 5, 6)).get(axes, (37, 12, 9))
+    g = [axis(n).astype(np.float32).astype(np.float64) for n in sizes]
+    shapes = [(0,), (0, 1), (0, 1, 2), (0, 1)]
+    paths = []
+    for t, ks in enumerate(shapes):
+        paths.append(str(tmp_path / f"t{t}.csv"))
+        tables.write_nu_table(paths[-1], [g[k] for k in ks], rng.uniform(1.0, 2.0, [sizes[k] for k in ks]))
+    sc = scenes.Scene()
+    ch = scenes._chamber(sc)
+    msm = scenes.si_tabulated(sc, paths)
+    shp = scenes._half_space(0.0)
+    reg = M.Region(ch, msm, shp)
+    sc.hold(shp, reg)
+    scenes._finish(sc, 1000.0, 0.5, 0.0)
+    sc.monte.setRefCompat(M.MONSEL_COMPAT_FIXED)
+    pr, cs = probe_for(sc)
+    osc = oracle.OracleScene(cs)
+    cols = []
+    for k in range(3):
+        lo, hi = min(g[k]), max(g[k])
+        step = np.abs(np.diff(g[k]))
+        cols.append(np.concatenate([rng.choice(g[k], 300), rng.uniform(lo, hi, 300),
+                                    rng.choice(g[k][:-1], 300) + 0.5 * rng.choice(step, 300),
+                                    lo - 0.25 * step.min() * rng.uniform(0, 1, 50),
+                                    hi + 0.25 * step.min() * rng.uniform(0, 1, 50)]))
+        cols[-1] = np.clip(rng.permutation(cols[-1]), lo - 0.25 * step.min(), hi + 0.25 * step.min())
+    x = np.stack(cols, 1).astype(np.float32).astype(np.float64)
+    for table, order, dim in ((0, 1, 1), (1, 3, 2), (2, 3, 3)):
+        got = pr.nu_table(table, order, x[:, :dim], dim).astype(np.float64)
+        want = osc.nu_table(table, order, x[:, :dim], dim)
+        if dim == 1:
+            tol = 8 * 2.0 ** -24 * (1 + np.max(np.abs(x[:, 0])) / np.min(np.abs(np.diff(g[0]))))
+        else:
+            tol = 2.0 ** -23 * np.abs(want) + 1e-9
+        assert np.all(np.abs(got - want) <= tol), (table, np.max(np.abs(got - want)))
+
+
 def _unit(rng, n):
     d = rng.normal(size=(n, 3))
     d /= np.linalg.norm(d, axis=1)[:, None]
