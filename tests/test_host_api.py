@@ -148,3 +148,45 @@ def test_gaussian_beam_create_electron(M):
     sc = scenes.flat("Si")
     mc = M.MonteCarloSS(sc.gun, sc.chamber, g.createElectron())
     assert mc.getSeed() is not None
+
+
+@pytest.mark.parametrize("form", ["repr", "e24", "fixed", "signed", "midpoint", "tiny", "long"])
+def test_table_numbers_read_as_by_a_stream(tmp_path, M, form):
+    """A table of plain decimal numbers gives the scene that stream extraction
+    gives (a last number followed by a letter, where extraction stops, takes
+    that path), to the bit: the scene's hash covers every value."""
+    import numpy as np
+    from cudamonsel_amd import scenes, tables
+    rng = np.random.default_rng(23)
+    paths = tables.synthetic_inelastic_tables(str(tmp_path), name="t")
+    n = 41 * 64
+    v = rng.uniform(0.0, 1.0, n) * 10.0 ** rng.integers(-22, 3, n)
+    if form == "repr":
+        text = [repr(float(x)) for x in v]
+    elif form == "e24":
+        text = ["%.24e" % x for x in v]
+    elif form == "fixed":
+        text = ["%.12f" % x for x in v]
+    elif form == "signed":
+        text = [("+%.17g" if k % 2 else "-%.15E") % x for k, x in enumerate(v)]
+    elif form == "midpoint":
+        # halfway between two doubles, and a unit of the last digit to each side
+        m = rng.integers(2 ** 52, 2 ** 53, n) * 2 + 1
+        text = [str(int(x) + d) + e for x, d, e in zip(m, rng.integers(-1, 2, n), rng.choice(["", "e-30", "e5", ".0"], n))]
+    elif form == "tiny":
+        text = ["%.17ge%d" % (x, rng.integers(-290, -250)) if "e" not in "%.17g" % x else "0" for x in v]
+    else:
+        text = ["0" * int(rng.integers(0, 12)) + "%.30f" % x for x in v]
+    head = open(paths[1]).read().split("\n")[:5]
+
+    def scene_hash(last):
+        with open(paths[1], "w") as f:
+            f.write("\n".join(head) + "\n")
+            f.write("\t".join(text[:1000]) + "\r\n" + "  \n".join(text[1000:]) + last)
+        sc = scenes.Scene()
+        shp = scenes._half_space(0.0)
+        sc.hold(shp, M.Region(scenes._chamber(sc), scenes.si_tabulated(sc, paths), shp))
+        scenes._finish(sc, 1000.0, 0.5, 0.0)
+        return sc.monte.compileScene().hash
+
+    assert scene_hash("") == scene_hash("x")
