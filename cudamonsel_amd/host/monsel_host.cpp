@@ -144,7 +144,7 @@ MottData loadMottTable(int Z) {
 namespace {
 
 /* Reads plain decimal numbers separated by white space, each to the double
- * nearest it.  Stream extraction takes 0.1 us a number, and a run reads its
+ * nearest it.  Stream extraction takes 0.1 us a number and a run reads its
  * tables anew (a file may have changed): of a bulk Cu call of 17.4 ms, 10 ms
  * went into the 99 thousand numbers of its four tables; here 2.3 ms do (call
  * 7.7 ms), of which 0.6 ms read the files. */
