@@ -302,7 +302,9 @@ typedef struct monsel_tuning {
                                  * for the next launch */
   int32_t tail_requeue;         /* once a launch's own items are all claimed, a wave down to this many
                                  * live lanes queues them for the next launch and leaves
-                                 * (0 = default 32, -1 = never; launches of < 65536 items never do) */
+                                 * (0 = 32, or 48 in a launch of more items than the device has
+                                 * lanes without a regroup interval; -1 = never; launches of < 65536
+                                 * items never do) */
 } monsel_tuning;
 
 typedef struct monsel_ctx_s* monsel_ctx;
