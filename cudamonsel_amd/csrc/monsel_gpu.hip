@@ -820,9 +820,9 @@ __device__ __forceinline__ const MONSEL_CS TransportArgs* launch_args() {
 /* Waves per SIMD the register allocation of k_transport targets.  A wave
  * issues at most one vector instruction in 5 cycles and one scalar one in 8
  * here, so the SIMD's throughput comes from its waves.  Without the tabulated
- * mechanism 5 (96 registers, 56 B of spills): 64 x 64 hole image 106.7 ms, 4:
- * 117.0 ms, 256 x 256 image 816 and 897 ms; 6 (80 registers, more spills) is
- * no faster.  With it, whose FP64 scatter holds windows and rows, 3 (168
+ * mechanism 5 (96 registers, 36 B of spills): 64 x 64 hole image 86 ms, 256 x
+ * 256 image 702 ms, 512 yield jobs 538 ms; 4: 93, 770 and 561 ms; 6 (80
+ * registers, far more spills): 129, 929 and 767 ms.  With it, whose FP64 scatter holds windows and rows, 3 (168
  * registers): transport of 400000 primaries of 1 keV in Si 53 ms, 4: 69 ms,
  * 2: 63 ms; of 40000 of 5 keV in Cu 14.7, 16.5 and 16.3 ms. */
 #ifndef MONSEL_TRANSPORT_WAVES_TAB
@@ -1716,10 +1716,11 @@ int geometry_batch_for(int tuned, int stepCost, uint64_t items) {
  * ones: a wave's step costs it every path that some lane of it takes, so an
  * electron in a wave of its own steps two to three times as fast as among 63
  * others, and such a launch leaves most of the device idle anyway.  (One
- * pixel of 100 primaries 6.2 -> 2.9 ms, 20,000 primaries on tabulated Si 25.5
- * -> 19.9 ms; with the line at 16,384 items the latter stays at 26 ms, with
+ * pixel of 100 primaries 5.0 -> 2.0 ms, 20,000 primaries on tabulated Si 10.6
+ * -> 6.6 ms, 3,001 on tabulated Cu 15.7 -> 7.8 ms.  Before the kernel's later
+ * gains the line at 16,384 items left the second of these as it was, and with
  * launches of 65,536 to 262,144 items spread as well a line scan of 67,727
- * primaries takes 25.8 ms instead of 23.1.)  The share leaves the other lanes
+ * primaries took 25.8 ms instead of 23.1.)  The share leaves the other lanes
  * of the wave to the secondaries its electrons spawn. */
 void spread_launch(GenDev& G, const monsel_tuning& T, uint64_t items, uint64_t waves) {
   G.lane_cap = items < kSpreadItems ? (int)std::min<uint64_t>(64, std::max<uint64_t>(1, (items + waves - 1) / waves)) : 64;
