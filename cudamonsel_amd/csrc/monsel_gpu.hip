@@ -424,11 +424,15 @@ __device__ __forceinline__ float from_anchor(float x, float y, float z) {
 
 /* What the start of a step leaves for its end. */
 struct StepStart {
-  uint32_t path; /* the free path's bits; the sign bit: the step may reach a
-                  * boundary, findEndOfStep must run */
+  float freePath;
   float total;   /* summed mechanism rates (0 in a null material) */
-  float u1, u2, u3;
+  float u1, u2;
+  uint32_t u3;   /* a uniform's bits (it is positive); the sign bit: the step
+                  * may reach a boundary, findEndOfStep must run.  (The free
+                  * path's own sign is not free for it: a rate table can
+                  * extrapolate below zero.) */
 };
+__device__ __forceinline__ bool may_reach_boundary(const StepStart& st) { return (int)st.u3 < 0; }
 
 /* MonteCarloSS::takeStep (MonteCarloSS.cu:107-163), first half: the
  * mechanism rates and the free path (MONSEL_MaterialScatterModel::
@@ -485,14 +489,14 @@ __device__ __forceinline__ void begin_step_in(const DevScene& S, int region, Ele
       freePath = maxFreePath;
     }
   }
+  st.freePath = freePath;
   st.total = total;
   st.u1 = u[1];
   st.u2 = u[2];
-  st.u3 = u[3];
   const float margin = nudge_nm(e.px, e.py, e.pz);
   const float current = e.safe > 0.f ? e.safe - from_anchor(e.px, e.py, e.pz) : 0.f;  /* bound here */
   const bool near_surface = !(freePath + margin <= current);
-  st.path = (__float_as_uint(freePath) & 0x7FFFFFFFu) | (near_surface ? 0x80000000u : 0u);
+  st.u3 = __float_as_uint(u[3]) | (near_surface ? 0x80000000u : 0u);
   PT_END(PH_RATES, t_ra);
 }
 
@@ -536,8 +540,8 @@ __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* j
   pin(is_null, n_mech, mech0, elastic_k, minE);
   /* the reference's barrier ignores the surface normal in compat mode */
   const bool normals = (S.compat & MONSEL_COMPAT_BARRIER_NORMAL) == 0u;
-  const bool geo = (int)st.path < 0;
-  const float freePath = __uint_as_float(st.path & 0x7FFFFFFFu);
+  const bool geo = may_reach_boundary(st);
+  const float freePath = st.freePath;
   const float px = e.px, py = e.py, pz = e.pz;
   StepEnd se;
   se.t = freePath;
@@ -674,7 +678,7 @@ __device__ __forceinline__ int finish_step_in(const DevScene& S, const JobRec* j
     u[0] = 0.f;
     u[1] = st.u1;
     u[2] = st.u2;
-    u[3] = st.u3;
+    u[3] = __uint_as_float(st.u3 & 0x7FFFFFFFu);
     PT_END(PH_SELECT, t_se);
     /* the mechanisms in turn, each for the lanes that chose it: its record
      * is wave-uniform */
@@ -850,7 +854,7 @@ k_transport(TransportArgs args) {
   const int geo_batch = args.G.geo_batch, lane_cap = args.G.lane_cap, claim_min = args.G.claim_min;
   const int tail_lanes = args.G.tail_lanes, regroup = args.G.steps_per_launch;
   const JobRec* jobs = args.G.jobs;
-  st.path = 0u;
+  st.u3 = 0u;
   stage_tables<TAB>(S);
   PT_INIT();
   for (;;) {
@@ -950,7 +954,7 @@ k_transport(TransportArgs args) {
      * reach a boundary waits for the wave's next findEndOfStep pass, which
      * runs once geo_batch lanes wait or no lane could move without it */
     if (lane_in(alive & ~pending)) begin_step<TAB>(S, e, st);
-    const unsigned long long m_geo = wave_ballot((int)st.path < 0) & alive;
+    const unsigned long long m_geo = wave_ballot(may_reach_boundary(st)) & alive;
     const bool run_geo = m_geo == alive || __popcll(m_geo) >= geo_batch;
     const unsigned long long step = run_geo ? alive : alive & ~m_geo;
     pending = alive & ~step;

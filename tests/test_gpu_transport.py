@@ -254,3 +254,43 @@ def test_min_energy_for_tracking(oracle, M):
     free.monte.setSeed(11)
     f = free.monte.runPixels(centers, 1000, 50, 50.0)
     assert np.sum(r.se) < 0.9 * np.sum(f.se)
+
+
+def test_negative_rate_steps_backwards(M, tmp_path, monkeypatch, capfd):
+    """A free path is -ln(u) / rate whatever the rate's sign
+    (MONSEL_MaterialScatterModel.cu): a mean free path table that falls
+    steeply towards its end extrapolates below zero at higher energies, and
+    an electron there steps against its direction.  Two steps deep inside the
+    material, from the states of the electrons the step limit drops: the
+    first along the beam, the second along the recorded direction."""
+    from cudamonsel_amd import scenes, tables
+    from cudamonsel_amd.abi import Engine, probe_for
+    paths = tables.synthetic_inelastic_tables(str(tmp_path))
+    e = np.append(np.geomspace(16.0, 1150.0, 40), 1200.0)
+    rate = np.append(np.full(40, 1.0e9), 0.9e9)      # 1/m; -0.1e9 per 50 eV beyond
+    tables.write_nu_table(paths[0], [e * tables.EV], rate)
+    sc = scenes.Scene()
+    ch = scenes._chamber(sc)
+    msm = scenes.si_tabulated(sc, paths)
+    shp = scenes._half_space(-1.0e6)
+    reg = M.Region(ch, msm, shp)
+    sc.hold(shp, reg)
+    scenes._finish(sc, 2000.0, 0.0, 0.0)
+    pr, cs = probe_for(sc)
+    total = float(pr.rates(1, [2000.0], 3)[0, -1])
+    assert total < -0.2, total                       # 1/nm
+    monkeypatch.setenv("MONSEL_DEBUG_WATCHDOG", "1")
+    with Engine() as eng:
+        r = eng.result(eng.submit(eng.upload(cs), [[0.0, 0.0, sc.beam_z]], 16, 2000.0, 0.0, 5, max_steps=1))
+    assert r["stats"]["watchdog_drops"] == 16
+    lines = [l for l in capfd.readouterr().err.splitlines() if l.startswith("[monsel]   p=(")]
+    assert len(lines) == 16
+    fp = []
+    for line in lines:
+        p, d = (np.array([float(v) for v in line.split(k)[1].split(")")[0].split()]) for k in ("p=(", "d=("))
+        second = (p[0] * d[0] + p[1] * d[1]) / (d[0] ** 2 + d[1] ** 2)
+        fp += [p[2] - sc.beam_z * 1e9 - second * d[2], second]
+    # exponential with mean 1 / total: the mean of 32 within 5 of its deviations
+    # (positions are printed to six digits, 1e-4 nm here)
+    assert max(fp) < 1e-3, fp
+    assert abs(np.mean(fp) * total - 1.0) < 5.0 / np.sqrt(32.0), (np.mean(fp), 1.0 / total)
