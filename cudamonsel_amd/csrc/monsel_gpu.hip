@@ -174,8 +174,12 @@ struct GenDev {
 /* launches with fewer items than this run their tail out (compaction would
  * only pass a few electrons from launch to launch) */
 constexpr uint32_t kTailMinItems = 65536;
-/* launches with fewer items than this spread them over all waves (spread_launch) */
+/* launches with fewer items than this spread them over all waves; where
+ * electrons are followed below kFewStepsEV only with new primaries of no more
+ * than kSpreadEnergy eV in all (spread_launch) */
 constexpr uint32_t kSpreadItems = 65536;
+constexpr float kFewStepsEV = 8.f;
+constexpr double kSpreadEnergy = 40e6;
 /* items a wave claims at a time (kept in reserve for its idle lanes);
  * 4 to 24 measure alike on the line scan, 128 and more starve other waves;
  * with the claim threshold below, 32 and 64 are 4 % and 8 % slower */
@@ -1679,6 +1683,7 @@ struct SceneDev {
   DevScene dev{};
   size_t bytes = 0;
   int step_cost = 0; /* what one findEndOfStep call costs at most (max_step_cost) */
+  float tracked_eV = 0.f; /* the lowest energy electrons are followed to (min_tracked_eV) */
   HostScene host;     /* kept to assemble batch scenes */
 };
 
@@ -1715,19 +1720,38 @@ int geometry_batch_for(int tuned, int stepCost, uint64_t items) {
   return stepCost >= 6 ? 12 : (stepCost >= 3 ? 8 : 1);
 }
 
+/* The lowest energy to which the scene's scatter models follow electrons. */
+float min_tracked_eV(const HostScene& H) {
+  float e = INFINITY;
+  for (const DRegion& r : H.regions)
+    if (r.m.n_mech > 0) e = std::min(e, r.m.minE);
+  return e;
+}
+
 /* How a launch spreads its items over its waves.  A launch of fewer than
  * kSpreadItems gives every wave the same share instead of filling the first
  * ones: a wave's step costs it every path that some lane of it takes, so an
  * electron in a wave of its own steps two to three times as fast as among 63
- * others, and such a launch leaves most of the device idle anyway.  (One
- * pixel of 100 primaries 5.0 -> 2.0 ms, 20,000 primaries on tabulated Si 10.6
- * -> 6.6 ms, 3,001 on tabulated Cu 15.7 -> 7.8 ms.  Before the kernel's later
- * gains the line at 16,384 items left the second of these as it was, and with
- * launches of 65,536 to 262,144 items spread as well a line scan of 67,727
- * primaries took 25.8 ms instead of 23.1.)  The share leaves the other lanes
- * of the wave to the secondaries its electrons spawn. */
-void spread_launch(GenDev& G, const monsel_tuning& T, uint64_t items, uint64_t waves) {
-  G.lane_cap = items < kSpreadItems ? (int)std::min<uint64_t>(64, std::max<uint64_t>(1, (items + waves - 1) / waves)) : 64;
+ * others, and such a launch leaves most of the device idle anyway.  The share
+ * leaves the other lanes of the wave to the secondaries its electrons spawn.
+ * Not so where the launch has steps enough to keep all its waves busy: then
+ * half-empty waves cost throughput.  That shows where electrons are followed
+ * down to a few eV, 50 to 100 steps each (PMMA to 0.5 eV, Si to 3.8; in Cu 6
+ * down to 11.7), once the new primaries bring more than kSpreadEnergy; and
+ * where more primaries wait for the next launch, which a spread launch holds
+ * up until its longest cascade has ended.
+ * Milliseconds filled / spread: Si 1 keV, 20,000 primaries 2.4 / 1.9, 40,000
+ * 3.1 / 3.5, 65,000 3.9 / 5.6; PMMA 2 keV, 8,000 5.4 / 5.3, 20,000 6.4 / 7.7,
+ * 65,000 10.6 / 13.8; line scan 0.5 keV, 20,000 6.9 / 3.6, 65,000 8.2 / 8.1; Cu 5
+ * keV, 5,000 2.6 / 1.8, 65,000 7.7 / 2.5; with tables Si 5 keV 65,000 36 / 32,
+ * Cu 25 / 19.  In chains of ten launches: line scan, 3,000 primaries each 29 /
+ * 23, 10,000 17 / 29, 20,000 19 / 33; Cu 2 keV, 20,000 17 / 11. */
+void spread_launch(GenDev& G, const monsel_tuning& T, const SceneDev& sd, uint64_t items, uint64_t waves,
+                   double primaries_eV, bool primaries_wait) {
+  bool spread = items < kSpreadItems;
+  if (!sd.dev.has_tabulated && sd.tracked_eV < kFewStepsEV)
+    spread = spread && primaries_eV <= kSpreadEnergy && (items <= waves || !primaries_wait);
+  G.lane_cap = spread ? (int)std::min<uint64_t>(64, std::max<uint64_t>(1, (items + waves - 1) / waves)) : 64;
   G.claim_min = std::min(kClaimMin, G.lane_cap);
   G.claim_chunk = std::min((int)kClaimChunk, G.lane_cap);
   const int tail = T.tail_requeue != 0 ? std::max(T.tail_requeue, 0) : (items > 64 * waves && T.steps_per_launch == 0 ? kTailLanesFull : kTailLanes);
@@ -2329,6 +2353,7 @@ void upload_scene(const HostScene& H, SceneDev& sd) {
   S.n_nu_words = (int)H.nuwords.size();
   sd.bytes = blob.size();
   sd.step_cost = max_step_cost(H);
+  sd.tracked_eV = min_tracked_eV(H);
 }
 
 /* One device scene holding several scenes side by side: every index is
@@ -2578,6 +2603,7 @@ void rebuild_batch_scene(monsel_ctx_s* C) {
   C->batch.dev = fresh.dev;
   C->batch.bytes = fresh.bytes;
   C->batch.step_cost = fresh.step_cost;
+  C->batch.tracked_eV = fresh.tracked_eV;
 }
 
 void finish_job(monsel_ctx_s* C, const std::shared_ptr<Job>& job, int st, const std::string& msg) {
@@ -2825,6 +2851,8 @@ void run_generation(monsel_ctx_s* C) {
                      [](const Job* a, const Job* b) { return a->total - a->launched < b->total - b->launched; });
   int nseg = 0;
   uint64_t nprim = 0;
+  double primaries_eV = 0.;
+  bool primaries_wait = false;
   for (Job* jp : order) {
     Job& j = *jp;
     if (j.launched >= j.total || nseg >= kMaxJobs) continue;
@@ -2840,7 +2868,9 @@ void run_generation(monsel_ctx_s* C) {
     j.launched += n;
     j.reserved += n * j.K;
     reservedTotal += n * j.K;
+    primaries_eV += (double)n * C->jobrec[j.slot].E0eV;
   }
+  for (auto& jp : C->active) primaries_wait = primaries_wait || jp->launched < jp->total;
   for (auto& jp : C->active)
     if (jp->outstanding > 0 || jp->reserved > 0) inflight.push_back(jp.get());
   if (nprim == 0 && C->in_count == 0) {
@@ -2882,7 +2912,7 @@ void run_generation(monsel_ctx_s* C) {
   G.handoff = C->tuning.spawn_handoff >= 0 ? 1 : 0;
   const int block = C->tuning.block_size > 0 ? C->tuning.block_size : 256;
   const int grid = C->n_cu * C->blocks_per_cu[C->batch.dev.has_tabulated ? 1 : 0];
-  spread_launch(G, C->tuning, nprim + C->in_count, (uint64_t)grid * (block / 64));
+  spread_launch(G, C->tuning, C->batch, nprim + C->in_count, (uint64_t)grid * (block / 64), primaries_eV, primaries_wait);
   /* Event markers time the kernels; MONSEL_NO_EVENT_TIMING=1 leaves them out
    * (hardware-counter profiling sessions reject the marker packets). */
   const bool timing = !getenv("MONSEL_NO_EVENT_TIMING");
@@ -3587,7 +3617,7 @@ int monsel_run_static(monsel_ctx ctx, monsel_scene_id scene, const monsel_job_de
       G.steps_per_launch = T.steps_per_launch;
       G.geo_batch = geometry_batch_for(T.geometry_batch, sd->step_cost, n + in_count);
       G.handoff = T.spawn_handoff >= 0 ? 1 : 0;
-      spread_launch(G, T, n + in_count, (uint64_t)grid * (block / 64));
+      spread_launch(G, T, *sd, n + in_count, (uint64_t)grid * (block / 64), (double)n * E0eV, launched + n < total);
       g_hip_call = "launch k_transport";
       if (sd->dev.has_tabulated)
         hipLaunchKernelGGL(k_transport<true>, dim3(grid), dim3(block), 0, stream, TransportArgs{sd->dev, G});

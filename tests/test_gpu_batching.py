@@ -309,3 +309,30 @@ def test_jobs_of_both_reference_modes_in_one_context(M):
                  for sid, (_, _, c, per, seed) in zip(sids, specs)]
     for a, b in zip(alone, mixed):
         _same(a, b)
+
+
+def test_spread_launches_only_where_steps_are_few(M):
+    """A launch of few items gives each wave a small share and runs its
+    cascades to their end.  Where electrons are followed to low energies
+    (PMMA) it does so only up to 40 MeV of new primaries and only while none
+    wait for a later launch: in a chain of ten launches the secondaries of one
+    then run beside the next one's primaries, so the chain ends a few launches
+    later, where a spread chain (Cu) ends with its tenth; and a job just
+    beyond 40 MeV needs more launches than one just below it.  The results
+    are those of launches of any size."""
+    from cudamonsel_amd import scenes
+    from cudamonsel_amd.abi import Engine
+
+    def run(material, beam_eV, primaries, **tuning):
+        sc = scenes.flat(material, beam_eV=beam_eV)
+        cs = sc.monte.compileScene()
+        with Engine(**tuning) as eng:
+            return eng.result(eng.submit(eng.upload(cs), [[0.0, 0.0, sc.beam_z]], primaries, beam_eV, 0.5e-9, 31))
+
+    chain = {m: run(m, e, 100000, primaries_per_launch=10000) for m, e in (("PMMA", 500.0), ("Cu", 2000.0))}
+    assert chain["Cu"]["stats"]["transport_launches"] <= 11
+    assert chain["PMMA"]["stats"]["transport_launches"] >= 12
+    for m, e in (("PMMA", 500.0), ("Cu", 2000.0)):
+        _same(chain[m], run(m, e, 100000))
+    below, above = (run("PMMA", 2000.0, n)["stats"]["transport_launches"] for n in (20000, 20001))
+    assert above > below, (above, below)
