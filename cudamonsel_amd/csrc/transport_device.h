@@ -1455,10 +1455,13 @@ struct ShapeHit {
  * inside bits, until the truth table changes value.  Each pass over the
  * primitives forms their intervals and finds the next crossing after tcur;
  * a segment that ends before the first one, or crosses the boundary there,
- * takes one pass.  Forming the intervals again for a later crossing keeps
- * them out of LDS (20 KB per block of 256 lanes), which held the kernel to 4
- * waves per SIMD.  The normal is formed only when asked for.  Requires the
- * same shape on every active lane. */
+ * takes one pass.  A crossing that leaves the truth value takes another, of
+ * the primitives that have a crossing left on the segment of some lane still
+ * walking (all primitives again: a shape of 8 parts 5 to 30 % slower, 1.6 M
+ * primaries on random ones 20 to 37 ms instead of 16 to 30).  Forming the
+ * intervals again keeps them out of LDS (20 KB per block of 256 lanes), which
+ * held the kernel to 4 waves per SIMD.  The normal is formed only when asked
+ * for.  Requires the same shape on every active lane. */
 MD ShapeHit shape_first(const DevScene& S, const MONSEL_CS DShape& sh, float px, float py, float pz, float dx,
                         float dy, float dz, float tmax, bool want_normal) {
   ShapeHit h;
@@ -1468,20 +1471,23 @@ MD ShapeHit shape_first(const DevScene& S, const MONSEL_CS DShape& sh, float px,
   const MONSEL_CS DPrim* prims = S.prims + sh.first_prim;
   uint32_t bits = 0;
   float tcur = 0.f;
+  uint32_t live = (1u << n) - 1u;   /* primitives the next pass visits (wave-uniform) */
   bool inside = false, open = true;
   /* primitive and face of the lowest two indices crossing at the hit */
   int k1 = 0, f1 = 0, k2 = -1, f2 = 0;
   PT_BEGIN(t_iv);
   for (int it = 0; it < 2 * n; ++it) {
-    uint32_t mask = 0;
+    uint32_t mask = 0, within = 0;
     float tnext = kInf;
-    for (int k = 0; k < n; ++k) {
+    for (uint32_t todo = live; todo; todo &= todo - 1u) {
+      const int k = __ffs((int)todo) - 1;
       const Interval iv = prim_interval(S, prims[k], px, py, pz, dx, dy, dz);
       const bool empty = !(iv.tin < iv.tout);
       const float a = empty ? -kInf : iv.tin, b = empty ? -kInf : iv.tout;
       if (it == 0) bits |= (a <= 0.f) & (b > 0.f) ? 1u << k : 0u;
       const bool at_in = a > tcur;
       const float nk = at_in ? a : (b > tcur ? b : kInf);
+      within |= nk <= tmax ? 1u << k : 0u;
       const bool nearer = nk < tnext, same = nk == tnext;
       if (want_normal && open) {
         const int f = at_in ? iv.fin : iv.fout;
@@ -1494,13 +1500,18 @@ MD ShapeHit shape_first(const DevScene& S, const MONSEL_CS DShape& sh, float px,
       tnext = nearer ? nk : tnext;
     }
     if (it == 0) inside = truth(sh, bits);
-    open = open & (tnext <= tmax);
+    open = open & (within != 0u);
     bits ^= open ? mask : 0u;
     const bool hit = open & (truth(sh, bits) != inside);
     h.t = hit ? tnext : h.t;
     open = open & !hit;
     tcur = tnext;
     if (!wave_any(open)) break;
+    /* those with a crossing left on some open lane's segment */
+    for (uint32_t todo = live; todo; todo &= todo - 1u) {
+      const uint32_t bit = todo & (0u - todo);
+      if (!wave_any(open & ((within & bit) != 0u))) live &= ~bit;
+    }
   }
   PT_END(PH_GEOM_IV, t_iv);
   PT_BEGIN(t_wk);

@@ -208,3 +208,66 @@ def test_nested_csg_geometry_and_transport_against_oracle(oracle, M, seed):
     assert g.stats.queue_overflow == 0 and g.stats.watchdog_drops == 0 and o["stats"]["watchdog_drops"] == 0
     zs, zb = su.total_z(su.from_gpu(g), su.from_oracle(o))
     assert abs(zs) < 3 and abs(zb) < 3, (zs, zb)
+
+
+@pytest.mark.parametrize("n", [2, 3, 5, 8])
+def test_walk_through_a_row_of_overlapping_boxes(oracle, M, n):
+    """The union of n boxes 12 nm long, each overlapping the next by 2 nm, is
+    one box: a segment along it passes up to 2 n - 2 crossings inside the
+    shape, each a pass of the walk over the parts that are left on the
+    segment.  Against the oracle's findEndOfStep of that one box; segments in
+    every direction, a third of them along the row and some of those from
+    outside.  (FP32 distances of some tens of nm: 1e-3 nm; the faces' normals
+    are axis vectors, exact in FP32.)"""
+    from cudamonsel_amd import scenes
+    from cudamonsel_amd.abi import probe_for
+
+    def box(hold, x0, x1):
+        s = M.NormalMultiPlaneShape()
+        for nrm, p in (([1, 0, 0], [x1, 0, 0]), ([-1, 0, 0], [x0, 0, 0]), ([0, 1, 0], [0, 9, 0]),
+                       ([0, -1, 0], [0, -9, 0]), ([0, 0, 1], [0, 0, 7]), ([0, 0, -1], [0, 0, -7])):
+            s.addPlane([float(v) for v in nrm], [v * NM for v in p])
+        hold.append(s)
+        return s
+
+    def scene(parts):
+        sc = scenes.Scene()
+        ch = scenes._chamber(sc)
+        hold = []
+        shape = box(hold, *parts[0])
+        for p in parts[1:]:
+            shape = M.NormalUnionShape(shape, box(hold, *p))
+            hold.append(shape)
+        reg = M.Region(ch, scenes.MATERIALS["PMMA"](sc), shape)
+        sc.hold(*hold, reg)
+        scenes._finish(sc, 500.0, 0.5, 40.0)
+        sc.monte.setRefCompat(M.MONSEL_COMPAT_FIXED)
+        return sc
+
+    row = scene([(10.0 * k, 10.0 * k + 12.0) for k in range(n)])
+    pr, _ = probe_for(row)
+    whole = scene([(0.0, 10.0 * n + 2.0)])
+    osc = oracle.OracleScene(whole.monte.compileScene())
+    rng = np.random.default_rng(n)
+    m = 6000
+    L = rng.uniform(1.0, 12.0 * n, m)
+    d = rng.normal(size=(m, 3))
+    d[::3] = np.array([1.0, 0.0, 0.0]) + 0.05 * rng.normal(size=d[::3].shape)
+    d[::6] *= -1.0
+    d /= np.linalg.norm(d, axis=1)[:, None]
+    p0 = rng.uniform(0.0, 1.0, (m, 3)) * [10.0 * n, 16.0, 12.0] + [1.0, -8.0, -6.0]
+    p0[::4, 0] = -rng.uniform(1.0, 9.0, p0[::4].shape[0])
+    p1 = (p0 + d * L[:, None]).astype(np.float32).astype(np.float64)
+    p0 = p0.astype(np.float32).astype(np.float64)
+    for region, part in ((1, p0[:, 0] > 0), (0, p0[:, 0] < 0)):
+        ou, onx, on = osc.find_end_of_step(region, p0[part], p1[part])
+        gu, gnx, gn = pr.find_end_of_step(region, p0[part], p1[part])
+        hit = ou <= 1.0
+        assert hit.sum() > 100
+        ok = (onx == gnx) & (hit == (gu <= 1.0))
+        ok[hit] &= np.abs(ou[hit] - gu[hit]) * L[part][hit] < 1e-3
+        # the last crossing of a segment that ends on a face may round either way
+        assert np.sum(~ok) <= 3, (region, np.sum(~ok))
+        both = ok & hit
+        far = np.sort(np.abs(np.abs(on[both]) - 1.0), axis=1)[:, 0] < 1e-6   # not on an edge
+        assert np.array_equal(on[both][far], gn[both][far].astype(np.float64))
