@@ -336,3 +336,52 @@ def test_spread_launches_only_where_steps_are_few(M):
         _same(chain[m], run(m, e, 100000))
     below, above = (run("PMMA", 2000.0, n)["stats"]["transport_launches"] for n in (20000, 20001))
     assert above > below, (above, below)
+
+
+def test_tabulated_scenes_in_one_batch(M, tmp_path):
+    """Jobs on two scenes with table sets of their own and, before them in the
+    batch, one without tables: the merged scene's table offsets are beyond
+    zero, and its search words exceed the 1,792 kept on chip, so that every
+    lookup searches device memory.  Each job matches the same job alone, which
+    searches on chip."""
+    from cudamonsel_amd import scenes, tables
+    from cudamonsel_amd.abi import Engine
+    sets = [tables.synthetic_inelastic_tables(str(tmp_path / "a")),
+            tables.synthetic_inelastic_tables(str(tmp_path / "b"), e_fermi_eV=9.0, gap_eV=3.0)]
+
+    def words(paths):
+        total = 0
+        for p in paths:
+            f = open(p).read().split()
+            dim, at = int(f[0]), 1
+            for _ in range(dim):
+                n = int(f[at])
+                total += 4 * n + 1      # points, two buckets a point, intervals
+                at += 1 + n
+        return total
+
+    assert all(words(s) <= 1792 for s in sets) and sum(words(s) for s in sets) > 1792
+    jobs = [(scenes.line_on_substrate(), 600, 500.0, 21)]
+    for k, s in enumerate(sets):
+        sc = scenes.Scene()
+        shp = scenes._half_space(0.0)
+        sc.hold(shp, M.Region(scenes._chamber(sc), scenes.si_tabulated(sc, s), shp))
+        scenes._finish(sc, 1000.0, 0.5, 0.0)
+        sc.monte.setRefCompat(M.MONSEL_COMPAT_REFERENCE)
+        jobs.append((sc, 400, 1000.0 - 200.0 * k, 22 + k))
+    # several launches a job, so that those submitted last join the first
+    with Engine(primaries_per_launch=300) as eng:
+        up = [(eng.upload(sc.monte.compileScene()), [[0.0, 0.0, sc.beam_z]] * 4, per, e, seed)
+              for sc, per, e, seed in jobs]
+        alone = [eng.result(eng.submit(sid, cen, per, e, 0.5e-9, seed)) for sid, cen, per, e, seed in up]
+        before = eng.counters()[0]
+        ids = [eng.submit(sid, cen, per, e, 0.5e-9, seed) for sid, cen, per, e, seed in up]
+        mixed = [eng.result(i) for i in ids]
+        assert eng.counters()[0] - before < sum(r["stats"]["transport_launches"] for r in mixed)
+        # and in the opposite order
+        ids = [eng.submit(sid, cen, per, e, 0.5e-9, seed) for sid, cen, per, e, seed in up[::-1]]
+        back = [eng.result(i) for i in ids][::-1]
+    for a, b, c in zip(alone, mixed, back):
+        assert a["stats"]["steps"] > 0 and a["stats"]["queue_overflow"] == 0
+        _same(a, b)
+        _same(a, c)

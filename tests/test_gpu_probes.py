@@ -383,3 +383,48 @@ def test_elastic_factories(oracle, M, factory):
         ga = pr.elastic_angle(1, slot, E, u).astype(np.float64)
         oa = osc.elastic_angle(1, slot, E, u)
         assert np.max(np.abs(np.cos(ga) - np.cos(oa))) < 5e-5, (slot, np.max(np.abs(np.cos(ga) - np.cos(oa))))
+
+
+@pytest.mark.parametrize("axes", ["log", "linear", "uneven", "descending", "shortest", "long"])
+def test_linear_lookup_near_table_points(oracle, tmp_path, M, axes):
+    """The FP32 linear lookup takes the interval the oracle's takes: at and
+    closely around every point of the axis, and halfway between them.
+
+    The abscissae and arguments here are FP32 numbers, so their differences
+    carry one rounding.  A weight is formed with at most 8 roundings (span
+    reciprocal and division each within 2.5 units), is at most 1.25 in size and
+    multiplies a value of at most 2; two of them and the sum stay within 64 x
+    2^-24.  A neighbouring interval's line is off by 1e-3 of a slope change of
+    order 1 or more."""
+    from cudamonsel_amd import scenes, tables
+    from cudamonsel_amd.abi import probe_for
+    rng = np.random.default_rng(29)
+    n = dict(shortest=4, long=900).get(axes, 37)
+    if axes == "log":
+        g = np.geomspace(1.0, 2000.0, n)
+    elif axes == "uneven":
+        g = np.sort(np.concatenate([[1.0, 9.0], 2.0 + 0.2 * rng.uniform(0, 1, n - 2)]))
+    else:
+        g = np.linspace(1.0, 9.0, n)
+        if axes == "descending":
+            g = g[::-1].copy()
+    g = g.astype(np.float32).astype(np.float64)
+    # values that alternate, so that the slope changes at every point
+    v = np.where(np.arange(n) % 2, 1.0, 2.0) - 0.2 * rng.uniform(0, 1, n)
+    paths = tables.synthetic_inelastic_tables(str(tmp_path))
+    tables.write_nu_table(paths[0], [g], v)
+    sc = scenes.Scene()
+    shp = scenes._half_space(0.0)
+    sc.hold(shp, M.Region(scenes._chamber(sc), scenes.si_tabulated(sc, paths), shp))
+    scenes._finish(sc, 1000.0, 0.5, 0.0)
+    pr, cs = probe_for(sc)
+    osc = oracle.OracleScene(cs)
+    step = np.diff(g)
+    x = [g]
+    for f in (0.0, 0.001, 0.01, 0.1, 0.5):
+        x += [g[:-1] + f * step, g[1:] - f * step]
+    x += [g[:1] - 0.2 * step[:1], g[-1:] + 0.2 * step[-1:]]
+    x = np.concatenate(x).astype(np.float32).astype(np.float64)[:, None]
+    got = pr.nu_table(0, 1, x, 1).astype(np.float64)
+    want = osc.nu_table(0, 1, x, 1)
+    assert np.max(np.abs(got - want)) <= 64 * 2.0 ** -24, np.max(np.abs(got - want))
