@@ -542,13 +542,6 @@ MD float csd_compute_split(const MONSEL_CS DCSD& c, const CSDHead& h, float len,
  * mode extrapolates a cubic far outside its abscissae
  * (NULagrangeInterpolation.cu:236) with weights up to ~1e7, so that FP32
  * rounding of the table values would change the result. */
-template <typename T>
-MD const T* nu_base(const DevScene& S);
-template <>
-MD const float* nu_base<float>(const DevScene& S) { return S.nu_data; }
-template <>
-MD const double* nu_base<double>(const DevScene& S) { return S.nu_data64; }
-
 MD const double* nu_axis(const DevScene& S, const MONSEL_CS DNUAxis& a) { return (const double*)(S.nu_words + a.x); }
 
 /* NULagrangeInterpolation::locate (NULagrangeInterpolation.cu:5-68) on an
@@ -618,89 +611,81 @@ MD T nu_poly(const double* xs, const T* f, T x) {
 }
 
 /* NULagrangeInterpolation::d1 (:144-158). */
-template <typename T, int ORDER>
-MD T nu_d1(const DevScene& S, const MONSEL_CS DNUTable& t, T x0) {
-  const T* d = nu_base<T>(S);
+template <int ORDER>
+MD float nu_d1(const DevScene& S, const MONSEL_CS DNUTable& t, float x0) {
   const double* xa = nu_axis(S, t.axis[0]);
-  int i0 = nu_locate<T>(xa, t.axis[0].n, ORDER, x0);
-  return nu_poly<T, ORDER>(xa + i0, d + t.voff + i0, x0);
+  int i0 = nu_locate<float>(xa, t.axis[0].n, ORDER, x0);
+  return nu_poly<float, ORDER>(xa + i0, (const float*)(S.nu_data + t.voff + i0), x0);
 }
 
 /* NULagrangeInterpolation::d2 (:169-192); values are an [na][nb] block. */
-template <typename T, int ORDER>
-MD T nu_d2(const DevScene& S, const MONSEL_CS DNUTable& t, T x0, T x1) {
-  const T* d = nu_base<T>(S);
+template <int ORDER>
+MD double nu_d2(const DevScene& S, const MONSEL_CS DNUTable& t, double x0, double x1) {
   const double* xa = nu_axis(S, t.axis[0]);
   const double* xb = nu_axis(S, t.axis[1]);
-  const T* f = d + t.voff;
+  const double* f = (const double*)(S.nu_data64 + t.voff);
   const int nb = t.axis[1].n;
-  int i0 = nu_locate<T>(xa, t.axis[0].n, ORDER, x0);
-  int j0 = nu_locate<T>(xb, nb, ORDER, x1);
-  T wb[ORDER + 1], y[ORDER + 1];
-  nu_weights<T, ORDER>(xb + j0, x1, wb);
+  int i0 = nu_locate<double>(xa, t.axis[0].n, ORDER, x0);
+  int j0 = nu_locate<double>(xb, nb, ORDER, x1);
+  double wb[ORDER + 1], y[ORDER + 1];
+  nu_weights<double, ORDER>(xb + j0, x1, wb);
 #pragma unroll
-  for (int i = 0; i <= ORDER; ++i) y[i] = nu_dot<T, ORDER>(wb, f + (size_t)(i0 + i) * nb + j0);
-  return nu_poly<T, ORDER>(xa + i0, y, x0);
+  for (int i = 0; i <= ORDER; ++i) y[i] = nu_dot<double, ORDER>(wb, f + (size_t)(i0 + i) * nb + j0);
+  return nu_poly<double, ORDER>(xa + i0, y, x0);
 }
 
 /* NULagrangeInterpolation::d3 (:215-240); compat_d3 reproduces line 236
  * (outer abscissae taken from the start of the grid).  voff overrides the
  * value offset (the 4-D lookup walks 3-D slices). */
-template <typename T, int ORDER>
-MD T nu_d3(const DevScene& S, const MONSEL_CS DNUTable& t, int ax, int voff, T x0, T x1, T x2, bool compat_d3) {
-  const T* d = nu_base<T>(S);
+template <int ORDER>
+MD double nu_d3(const DevScene& S, const MONSEL_CS DNUTable& t, int ax, int voff, double x0, double x1, double x2, bool compat_d3) {
   const double* xa = nu_axis(S, t.axis[ax]);
   const double* xb = nu_axis(S, t.axis[ax + 1]);
   const double* xc = nu_axis(S, t.axis[ax + 2]);
-  const T* v = d + voff;
+  const double* v = (const double*)(S.nu_data64 + voff);
   const int nb = t.axis[ax + 1].n, nc = t.axis[ax + 2].n;
-  int i0 = nu_locate<T>(xa, t.axis[ax].n, ORDER, x0);
-  int j0 = nu_locate<T>(xb, nb, ORDER, x1);
-  int k0 = nu_locate<T>(xc, nc, ORDER, x2);
-  T wb[ORDER + 1], wc[ORDER + 1], y[ORDER + 1];
-  nu_weights<T, ORDER>(xb + j0, x1, wb);
-  nu_weights<T, ORDER>(xc + k0, x2, wc);
+  int i0 = nu_locate<double>(xa, t.axis[ax].n, ORDER, x0);
+  int j0 = nu_locate<double>(xb, nb, ORDER, x1);
+  int k0 = nu_locate<double>(xc, nc, ORDER, x2);
+  double wb[ORDER + 1], wc[ORDER + 1], y[ORDER + 1];
+  nu_weights<double, ORDER>(xb + j0, x1, wb);
+  nu_weights<double, ORDER>(xc + k0, x2, wc);
 #pragma unroll 1
   for (int i = 0; i <= ORDER; ++i) {
-    T z[ORDER + 1];
-    const T* blk = v + (size_t)(i0 + i) * nb * nc;
+    double z[ORDER + 1];
+    const double* blk = v + (size_t)(i0 + i) * nb * nc;
 #pragma unroll 1
     for (int j = 0; j <= ORDER; ++j) {
-      const T zj = nu_dot<T, ORDER>(wc, blk + (size_t)(j0 + j) * nc + k0);
+      const double zj = nu_dot<double, ORDER>(wc, blk + (size_t)(j0 + j) * nc + k0);
 #pragma unroll
       for (int q = 0; q <= ORDER; ++q)
         if (q == j) z[q] = zj;
     }
-    const T yi = nu_dot<T, ORDER>(wb, z);
+    const double yi = nu_dot<double, ORDER>(wb, z);
 #pragma unroll
     for (int q = 0; q <= ORDER; ++q)
       if (q == i) y[q] = yi;
   }
-  return nu_poly<T, ORDER>(compat_d3 ? xa : xa + i0, y, x0);
+  return nu_poly<double, ORDER>(compat_d3 ? xa : xa + i0, y, x0);
 }
 
 /* NULagrangeInterpolation::d4 (:259-306). */
-template <typename T, int ORDER>
-MD T nu_d4(const DevScene& S, const MONSEL_CS DNUTable& t, const T* x, bool compat_d3) {
+template <int ORDER>
+MD double nu_d4(const DevScene& S, const MONSEL_CS DNUTable& t, const double* x, bool compat_d3) {
   const double* xa = nu_axis(S, t.axis[0]);
-  int i0 = nu_locate<T>(xa, t.axis[0].n, ORDER, x[0]);
-  T y[ORDER + 1];
+  int i0 = nu_locate<double>(xa, t.axis[0].n, ORDER, x[0]);
+  double y[ORDER + 1];
 #pragma unroll
   for (int i = 0; i <= ORDER; ++i)
-    y[i] = nu_d3<T, ORDER>(S, t, 1, t.voff + (i0 + i) * t.axis[1].n * t.axis[2].n * t.axis[3].n, x[1], x[2], x[3], compat_d3);
-  return nu_poly<T, ORDER>(xa + i0, y, x[0]);
+    y[i] = nu_d3<ORDER>(S, t, 1, t.voff + (i0 + i) * t.axis[1].n * t.axis[2].n * t.axis[3].n, x[1], x[2], x[3], compat_d3);
+  return nu_poly<double, ORDER>(xa + i0, y, x[0]);
 }
 
-template <typename T, int ORDER>
-MD T nu_interp_o(const DevScene& S, int table, const T* x, bool compat_d3) {
-  const MONSEL_CS DNUTable& t = S.nu[table];
-  switch (t.dim) {
-    case 1: return nu_d1<T, ORDER>(S, t, x[0]);
-    case 2: return nu_d2<T, ORDER>(S, t, x[0], x[1]);
-    case 3: return nu_d3<T, ORDER>(S, t, 0, t.voff, x[0], x[1], x[2], compat_d3);
-    case 4: return nu_d4<T, ORDER>(S, t, x, compat_d3);
-  }
-  return 0;
+template <int ORDER>
+MD double nu_interp_o(const DevScene& S, const MONSEL_CS DNUTable& t, const double* x, bool compat_d3) {
+  if (t.dim == 2) return nu_d2<ORDER>(S, t, x[0], x[1]);
+  if (t.dim == 3) return nu_d3<ORDER>(S, t, 0, t.voff, x[0], x[1], x[2], compat_d3);
+  return nu_d4<ORDER>(S, t, x, compat_d3);
 }
 
 /* The lookups of the transport step: FP64 cubic in two and three dimensions,
@@ -848,17 +833,16 @@ MD float nu_linear1(const DevScene& S, const MONSEL_CS DNUTable& t, float x) {
  * 1-D (mean free path), FP64 otherwise. */
 MD double nu_interp(const DevScene& S, int table, int order, const double* x, bool compat_d3) {
   const MONSEL_CS DNUTable& t = S.nu[table];
-  if (order == 3 && t.dim == 2) return nu_cubic2(S, t, x[0], x[1]);
-  if (order == 3 && t.dim == 3) return nu_cubic3(S, t, x[0], x[1], x[2], compat_d3);
   if (t.dim == 1) {
     const float xf = (float)x[0];
     if (order == 1) return nu_linear1(S, t, xf);
-    if (order == 2) return nu_interp_o<float, 2>(S, table, &xf, compat_d3);
-    return nu_interp_o<float, 3>(S, table, &xf, compat_d3);
+    return order == 2 ? nu_d1<2>(S, t, xf) : nu_d1<3>(S, t, xf);
   }
-  if (order == 1) return nu_interp_o<double, 1>(S, table, x, compat_d3);
-  if (order == 2) return nu_interp_o<double, 2>(S, table, x, compat_d3);
-  return nu_interp_o<double, 3>(S, table, x, compat_d3);
+  if (order == 1) return nu_interp_o<1>(S, t, x, compat_d3);
+  if (order == 2) return nu_interp_o<2>(S, t, x, compat_d3);
+  if (t.dim == 2) return nu_cubic2(S, t, x[0], x[1]);
+  if (t.dim == 3) return nu_cubic3(S, t, x[0], x[1], x[2], compat_d3);
+  return nu_d4<3>(S, t, x, compat_d3);
 }
 
 /* ------------------------------------------------------ mechanisms ----- */
