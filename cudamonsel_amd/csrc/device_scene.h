@@ -159,12 +159,11 @@ struct DMSM {
 struct DRegion {
   DMSM m;
   int parent;
-  int shape;
   int msm;
   int first_child;
   int n_children;
   int depth;
-  int pad[2];
+  int pad[3];
   DShape sh;
 };
 
@@ -201,14 +200,13 @@ struct DNUTable {
 };
 
 struct DevScene {
-  int n_regions, n_shapes, n_prims, n_planes, n_msm, n_mech, n_elem, n_mott, n_nu;
+  int n_regions, n_prims, n_planes, n_msm, n_mech, n_elem, n_mott, n_nu;
   int has_tabulated;      /* some mechanism is TabulatedInelasticSM (selects the transport kernel) */
   uint32_t compat;
   float chamber_r;        /* nm */
   float chamber_c[3];     /* nm */
   const MONSEL_CS DRegion* regions;
   const MONSEL_CS DShape* children;   /* the shapes of each region's children, in a run */
-  const MONSEL_CS DShape* shapes;
   const MONSEL_CS DPrim* prims;
   const MONSEL_CS float4* planes;   /* (nx, ny, nz, b) */
   const MONSEL_CS DMSM* msms;

@@ -1659,7 +1659,7 @@ struct HBuf {
 struct HostScene {
   std::vector<DRegion> regions;
   std::vector<DShape> children;
-  std::vector<DShape> shapes;
+  std::vector<DShape> shapes;   /* a compiled scene's; regions and children hold their copies */
   std::vector<DPrim> prims;
   std::vector<float4> planes;
   std::vector<DMSM> msms;
@@ -1692,7 +1692,7 @@ struct SceneDev {
  * chamber's sphere aside (an electron meets it once, on its way out). */
 int max_step_cost(const HostScene& H) {
   auto cost = [&](int region) {
-    const DShape& sh = H.shapes[H.regions[region].shape];
+    const DShape& sh = H.regions[region].sh;
     int n = 0;
     for (int k = 0; k < sh.n_prims; ++k) n += H.prims[sh.first_prim + k].kind == PRIM_CYLINDER ? 2 : 1;
     return sh.is_sphere ? 0 : n;
@@ -2262,13 +2262,12 @@ HostScene compile_scene(const monsel_scene_desc* d) {
     DRegion dr;
     memset(&dr, 0, sizeof(dr));
     dr.parent = d->regions[r].parent;
-    dr.shape = shapeIdx[d->regions[r].shape];
     dr.msm = d->regions[r].msm;
     dr.first_child = (int)H.children.size();
     dr.n_children = (int)kids[r].size();
     dr.depth = dr.parent < 0 ? 0 : H.regions[dr.parent].depth + 1;
     dr.m = H.msms[dr.msm];
-    dr.sh = H.shapes[dr.shape];
+    dr.sh = H.shapes[shapeIdx[d->regions[r].shape]];
     for (int c : kids[r]) {
       H.children.push_back(H.shapes[shapeIdx[d->regions[c].shape]]);
       H.children.back().region = c;
@@ -2293,7 +2292,6 @@ size_t host_scene_bytes(const HostScene& H) {
   auto add = [&](size_t bytes) { total = ((total + 255) & ~(size_t)255) + bytes; };
   add(H.regions.size() * sizeof(DRegion));
   add(H.children.size() * sizeof(DShape));
-  add(H.shapes.size() * sizeof(DShape));
   add(H.prims.size() * sizeof(DPrim));
   add(H.planes.size() * sizeof(float4));
   add(H.msms.size() * sizeof(DMSM));
@@ -2311,7 +2309,7 @@ size_t host_scene_bytes(const HostScene& H) {
 
 void upload_scene(const HostScene& H, SceneDev& sd) {
   std::vector<char> blob;
-  size_t o_reg = append(blob, H.regions), o_ch = append(blob, H.children), o_sh = append(blob, H.shapes);
+  size_t o_reg = append(blob, H.regions), o_ch = append(blob, H.children);
   size_t o_pr = append(blob, H.prims), o_pl = append(blob, H.planes), o_msm = append(blob, H.msms);
   size_t o_me = append(blob, H.mechs), o_el = append(blob, H.elems), o_sp = append(blob, H.spwem);
   size_t o_x1 = append(blob, H.x1), o_nu = append(blob, H.nu), o_nd = append(blob, H.nudata);
@@ -2321,7 +2319,6 @@ void upload_scene(const HostScene& H, SceneDev& sd) {
   char* b = sd.blob.as<char>();
   DevScene& S = sd.dev;
   S.n_regions = (int)H.regions.size();
-  S.n_shapes = (int)H.shapes.size();
   S.n_prims = (int)H.prims.size();
   S.n_planes = (int)H.planes.size();
   S.n_msm = (int)H.msms.size();
@@ -2337,7 +2334,6 @@ void upload_scene(const HostScene& H, SceneDev& sd) {
   for (int k = 0; k < 3; ++k) S.chamber_c[k] = H.chamber_c[k];
   S.regions = (decltype(S.regions))(b + o_reg);
   S.children = (decltype(S.children))(b + o_ch);
-  S.shapes = (decltype(S.shapes))(b + o_sh);
   S.prims = (decltype(S.prims))(b + o_pr);
   S.planes = (decltype(S.planes))(b + o_pl);
   S.msms = (decltype(S.msms))(b + o_msm);
@@ -2365,7 +2361,7 @@ HostScene merge_scenes(const std::vector<const HostScene*>& parts, std::vector<i
   M.chamber_r = 0.f;
   roots.clear();
   for (const HostScene* P : parts) {
-    const int o_reg = (int)M.regions.size(), o_ch = (int)M.children.size(), o_sh = (int)M.shapes.size();
+    const int o_reg = (int)M.regions.size(), o_ch = (int)M.children.size();
     const int o_pr = (int)M.prims.size(), o_pl = (int)M.planes.size(), o_msm = (int)M.msms.size();
     const int o_me = (int)M.mechs.size(), o_el = (int)M.elems.size(), o_mott = (int)(M.spwem.size() / kMottNE);
     const int o_nu = (int)M.nu.size(), o_nd = (int)M.nudata.size(), o_nd64 = (int)M.nudata64.size();
@@ -2373,7 +2369,6 @@ HostScene merge_scenes(const std::vector<const HostScene*>& parts, std::vector<i
     roots.push_back(o_reg);
     for (DRegion r : P->regions) {
       if (r.parent >= 0) r.parent += o_reg;
-      r.shape += o_sh;
       r.sh.first_prim += o_pr;
       r.msm += o_msm;
       r.m.mech0 += o_me;
@@ -2384,10 +2379,6 @@ HostScene merge_scenes(const std::vector<const HostScene*>& parts, std::vector<i
       c.first_prim += o_pr;
       c.region += o_reg;
       M.children.push_back(c);
-    }
-    for (DShape sh : P->shapes) {
-      sh.first_prim += o_pr;
-      M.shapes.push_back(sh);
     }
     for (DPrim pr : P->prims) {
       if (pr.kind == PRIM_PLANES) pr.first_plane += o_pl;
