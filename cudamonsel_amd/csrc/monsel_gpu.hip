@@ -1402,11 +1402,17 @@ __global__ void k_pixels_to_double(const unsigned long long* px, int np, double*
 
 /* ---- probe kernels ---------------------------------------------------- */
 
-__global__ void k_probe_rates(DevScene S, int msm, int n, const float* E, float* out) {
+/* a scatter model's record as transport reads it: its region's copy (region
+ * -1: no region has the model) */
+__device__ __forceinline__ const MONSEL_CS DMSM& probe_msm(const DevScene& S, int msm, int region) {
+  return region >= 0 ? S.regions[region].m : S.msms[msm];
+}
+
+__global__ void k_probe_rates(DevScene S, int msm, int region, int n, const float* E, float* out) {
   stage_tables<true>(S);
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const MONSEL_CS DMSM& m = S.msms[msm];
+  const MONSEL_CS DMSM& m = probe_msm(S, msm, region);
   float tot = 0.f;
   for (int k = 0; k < m.n_mech; ++k) {
     float r = mech_rate(S, S.mechs[m.mech0 + k], E[i]);
@@ -1485,8 +1491,7 @@ __global__ void k_probe_barrier(DevScene S, int from, int to, int n, const float
   e.dz = dir[3 * i + 2];
   e.E = E[i];
   e.region = from;
-  int sign = barrier_core(S, S.msms[S.regions[from].msm], S.msms[S.regions[to].msm], e, to, nb[3 * i], nb[3 * i + 1],
-                          nb[3 * i + 2], u[i]);
+  int sign = barrier_core(S, S.regions[from].m, S.regions[to].m, e, to, nb[3 * i], nb[3 * i + 1], nb[3 * i + 2], u[i]);
   float* o = out + 6 * (size_t)i;
   o[0] = e.dx;
   o[1] = e.dy;
@@ -1496,10 +1501,10 @@ __global__ void k_probe_barrier(DevScene S, int from, int to, int n, const float
   o[5] = (float)sign;
 }
 
-__global__ void k_probe_csd(DevScene S, int msm, int n, const float* len, const float* E, float* out) {
+__global__ void k_probe_csd(DevScene S, int msm, int region, int n, const float* len, const float* E, float* out) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  out[i] = csd_compute(S.msms[msm].csd, len[i], E[i]);
+  out[i] = csd_compute(probe_msm(S, msm, region).csd, len[i], E[i]);
 }
 
 __global__ void k_probe_step_end(DevScene S, int region, int n, const float* p0, const float* p1, float* out_u,
@@ -3710,6 +3715,13 @@ int probe_prologue(monsel_ctx ctx, monsel_scene_id scene, std::shared_ptr<SceneD
 }
 
 inline unsigned grid_for(int n) { return (unsigned)((n + 255) / 256); }
+
+/* the first region with scatter model msm, -1 if none */
+int region_of(const SceneDev& sd, int msm) {
+  for (size_t r = 0; r < sd.host.regions.size(); ++r)
+    if (sd.host.regions[r].msm == msm) return (int)r;
+  return -1;
+}
 }  // namespace
 
 extern "C" {
@@ -3727,7 +3739,7 @@ int monsel_probe_rates(monsel_ctx ctx, monsel_scene_id scene, int msm, int n, co
     int w = m[0].n_mech + 1;
     Scratch<float> dE(n), dO((size_t)n * w);
     HIP_TRY(hipMemcpy(dE.d, energies_ev, 4 * (size_t)n, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_probe_rates, dim3(grid_for(n)), dim3(256), 0, 0, sd->dev, msm, n, dE.d, dO.d);
+    hipLaunchKernelGGL(k_probe_rates, dim3(grid_for(n)), dim3(256), 0, 0, sd->dev, msm, region_of(*sd, msm), n, dE.d, dO.d);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpy(out, dO.d, 4 * (size_t)n * w, hipMemcpyDeviceToHost));
     return MONSEL_OK;
@@ -3778,7 +3790,7 @@ int monsel_probe_csd(monsel_ctx ctx, monsel_scene_id scene, int msm, int n, cons
     Scratch<float> dL(n), dE(n), dO(n);
     HIP_TRY(hipMemcpy(dL.d, len_nm, 4 * (size_t)n, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(dE.d, energies_ev, 4 * (size_t)n, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_probe_csd, dim3(grid_for(n)), dim3(256), 0, 0, sd->dev, msm, n, dL.d, dE.d, dO.d);
+    hipLaunchKernelGGL(k_probe_csd, dim3(grid_for(n)), dim3(256), 0, 0, sd->dev, msm, region_of(*sd, msm), n, dL.d, dE.d, dO.d);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpy(out, dO.d, 4 * (size_t)n, hipMemcpyDeviceToHost));
     return MONSEL_OK;
