@@ -76,7 +76,7 @@ struct DCSD {
   float breakE;  /* eV */
   float gamma15; /* 1.5 gamma, 1/(nm eV^1.5) */
   float minE;    /* eV (barrier height) */
-  struct Term {  /* one element's; the first three end the record's first 16 words */
+  struct Term {  /* one element's; the first three end the record's first 14 words */
     float recipJ; /* 1/eV */
     float beta;
     float coef;   /* eV^2/nm */

@@ -199,10 +199,10 @@ constexpr int kClaimMin = MONSEL_CLAIM_MIN;
 /* Live lanes at which a wave with nothing left to claim passes its electrons
  * on, by default: 32, and 48 in a launch of more items than the device has
  * lanes, which the next launch packs with many others (256 x 256 line image
- * 700 ms with 32, 682 with 48, 746 with 16; six requests 280 and 275 ms; a
- * scan of 256,000 primaries, whose launches stay below, 11.9 and 12.3).  Where
+ * 688 ms with 32, 670 with 48, 731 with 16; six requests 278 and 274 ms; a
+ * scan of 256,000 primaries, whose launches stay below, 11.8 and 12.0).  Where
  * electrons return to the queue every steps_per_launch steps anyway 48 gains
- * nothing (512 yield jobs 539 and 542 ms). */
+ * nothing (512 yield jobs 542 and 543 ms). */
 constexpr int kTailLanes = 32, kTailLanesFull = 48;
 
 /* per-wave LDS table of the handoff: lane of the k-th spawning lane */
@@ -828,11 +828,13 @@ __device__ __forceinline__ const MONSEL_CS TransportArgs* launch_args() {
 /* Waves per SIMD the register allocation of k_transport targets.  A wave
  * issues at most one vector instruction in 5 cycles and one scalar one in 8
  * here, so the SIMD's throughput comes from its waves.  Without the tabulated
- * mechanism 5 (96 registers, 36 B of spills): 64 x 64 hole image 86 ms, 256 x
- * 256 image 702 ms, 512 yield jobs 538 ms; 4: 93, 770 and 561 ms; 6 (80
- * registers, far more spills): 129, 929 and 767 ms.  With it, whose FP64 scatter holds windows and rows, 3 (168
- * registers): transport of 400000 primaries of 1 keV in Si 53 ms, 4: 69 ms,
- * 2: 63 ms; of 40000 of 5 keV in Cu 14.7, 16.5 and 16.3 ms. */
+ * mechanism 5 (96 registers, 36 B of spills): 64 x 64 hole image 85 ms, 256 x
+ * 256 image 669 ms, 512 yield jobs 541 ms; 4: 92, 737 and 563 ms; 6 (80
+ * registers, far more spills): 102, 737 and 643 ms.  With it, whose FP64
+ * scatter holds windows and rows, 3 (168 registers): transport of 400,000
+ * primaries of 1 keV in Si 39 ms, of 40,000 of 5 keV in Cu 10.5; 4: 47 and
+ * 11.0 ms; 2: 36 and 10.7, but scenes without tables in the same batch run on
+ * it too. */
 #ifndef MONSEL_TRANSPORT_WAVES_TAB
 #define MONSEL_TRANSPORT_WAVES_TAB 3
 #endif
@@ -1713,10 +1715,10 @@ int max_step_cost(const HostScene& H) {
 
 /* Lanes a wave gathers for findEndOfStep when the tuning leaves it open (0):
  * gathering pays the more the call costs.  256 x 256 image of three lines
- * (cost above 6): 8 lanes 723 ms, 12: 701, 16: 692 (1: 20 % more than 8), six
- * requests of mixed sizes and scenes 278, 281 and 288 ms; contact hole image
- * (cost 3): 1: 92.5 ms, 8: 86.7, 16: 91.2; flat and step-edge yield jobs (cost
- * 1 and 2): 1: 539 ms, 4: 554.  A launch of few items (a small job
+ * (cost above 6): 1: 844 ms, 8 lanes 696, 12: 671, 16: 661, six requests of
+ * mixed sizes and scenes 298, 273, 275 and 281 ms; contact hole image (cost 3):
+ * 1: 91 ms, 8: 86, 16: 91; flat and step-edge yield jobs (cost 1 and 2): 1: 541
+ * ms, 4: 554.  A launch of few items (a small job
  * alone) leaves most of the device idle and lasts as long as its longest
  * cascade, which waiting only lengthens. */
 int geometry_batch_for(int tuned, int stepCost, uint64_t items) {

@@ -273,7 +273,9 @@ MD float* lds_spwem() {
   return l_spwem;
 }
 /* The search words of the inelastic tables (abscissae, guides and windows;
- * some 11 KB for a four-table set), in LDS as well where they fit. */
+ * 12.8 KB for the dielectric model's four tables), in LDS as well where those
+ * of all tables of the launch's scenes fit; else all are searched in device
+ * memory. */
 constexpr int kLdsNuWords = 1792;
 MD unsigned long long* lds_nu_words() {
   __shared__ unsigned long long l_nu_words[kLdsNuWords];
@@ -451,8 +453,8 @@ MD float nieminen_factor(float eps) {
   return eps < 1e-3f ? series : power;
 }
 
-/* A stopping-power record's head and its first three elements, in scalar
- * registers: one 16-word load. */
+/* A stopping-power record's head and its first three elements, 14 words read
+ * together into scalar registers. */
 struct CSDHead {
   int active, nce;
   float breakE, gamma15, minE;
@@ -696,8 +698,8 @@ MD double nu_interp_o(const DevScene& S, const MONSEL_CS DNUTable& t, const doub
  * a chain of steps.  Here the axes of a lookup are searched together, in LDS,
  * from the bounds their guides give (mostly one probe each), the window of an
  * interval is a word beside them, and what the weights hold of the axis alone
- * comes in a DNUWindow.  Transport of 3001 primaries of 5 keV in Cu: 8.7 ms to
- * 5.9 ms; of 400000 of 1 keV in Si 53 ms. */
+ * comes in a DNUWindow.  Transport of 3001 primaries of 5 keV in Cu, with the
+ * spread of small launches: 19.7 ms to 4.7; of 400,000 of 1 keV in Si 71 to 39. */
 template <typename T, int A, class P>
 MD void nu_search(P w, const MONSEL_CS DNUAxis* ax, const T* x, int* lo, int* first) {
   int up[A];
@@ -796,8 +798,8 @@ MD double nu_cubic3(const DevScene& S, const MONSEL_CS DNUTable& t, double x0, d
   nu_cubic_weights(S.nu_recs[ax[1].rec + lo[1]], x1, wb);
   nu_cubic_weights(S.nu_recs[ax[0].rec + (compat_d3 ? -1 : lo[0])], x0, wa);
   /* one outer point at a time: with the sixteen values of a point, or of two,
-   * loaded together and the windows beside them the registers spill, and
-   * 400000 primaries in Si take 58 ms where these take 53 */
+   * loaded together and the windows beside them the registers spill (9 % more
+   * time for 400,000 primaries in Si) */
 #pragma unroll 1
   for (int i = 0; i < 4; ++i) {
     double z[4];

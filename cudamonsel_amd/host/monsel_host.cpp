@@ -199,8 +199,10 @@ class NumberReader {
  private:
   static bool space(char c) { return c == ' ' || (c >= '\t' && c <= '\r'); }
 
-  /* eight at a time (the bytes of a little-endian word: pairs, then fours),
-   * then one by one */
+  /* eight at a time, then one by one.  The eight by the known SIMD-within-a-
+   * register method for decimal strings (as Lemire describes it, "Number
+   * parsing at a gigabyte per second"): the bytes of a little-endian word are
+   * combined to pairs, the pairs to fours, the fours to eight */
   void digits(uint64_t& m) {
     while (end_ - p_ >= 8) {
       uint64_t w;
