@@ -1752,7 +1752,11 @@ float min_tracked_eV(const HostScene& H) {
  * 65,000 10.6 / 13.8; line scan 0.5 keV, 20,000 6.9 / 3.6, 65,000 8.2 / 8.1; Cu 5
  * keV, 5,000 2.6 / 1.8, 65,000 7.7 / 2.5; with tables Si 5 keV 65,000 36 / 32,
  * Cu 25 / 19.  In chains of ten launches: line scan, 3,000 primaries each 29 /
- * 23, 10,000 17 / 29, 20,000 19 / 33; Cu 2 keV, 20,000 17 / 11. */
+ * 23, 10,000 17 / 29, 20,000 19 / 33; Cu 2 keV, 20,000 17 / 11.  From
+ * kSpreadItems on every launch is filled: 70,000 primaries Si 4.0 / 6.0, PMMA
+ * 5.7 / 8.1, line scan 6.5 / 11.9, 200,000 9.0 / 9.9, 10.4 / 10.9 and 10.1 /
+ * 12.2; with tables Si alike.  (Cu, 3 keV, would gain up to some 150,000: 5.9 /
+ * 2.0 at 70,000, 11.1 / 9.5 at 150,000, alike from 200,000.) */
 void spread_launch(GenDev& G, const monsel_tuning& T, const SceneDev& sd, uint64_t items, uint64_t waves,
                    double primaries_eV, bool primaries_wait) {
   bool spread = items < kSpreadItems;
