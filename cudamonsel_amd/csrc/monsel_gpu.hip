@@ -1743,7 +1743,7 @@ float min_tracked_eV(const HostScene& H) {
  * leaves the other lanes of the wave to the secondaries its electrons spawn.
  * Not so where the launch has steps enough to keep all its waves busy: then
  * half-empty waves cost throughput.  That shows where electrons are followed
- * down to a few eV, 50 to 100 steps each (PMMA to 0.5 eV, Si to 3.8; in Cu 6
+ * down to a few eV, 60 to 170 steps each (PMMA to 0.5 eV, Si to 3.8; in Cu 6
  * down to 11.7), once the new primaries bring more than kSpreadEnergy; and
  * where more primaries wait for the next launch, which a spread launch holds
  * up until its longest cascade has ended.
